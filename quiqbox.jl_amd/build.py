@@ -1,7 +1,7 @@
 """Build libqbx_hip.so for gfx950 in-tree.
 
 Steps: run csrc/gen_eri.py (one translation unit per ERI angular class into
-csrc/gen/), compile csrc/qbx.hip, csrc/qbx_mlp.hip, csrc/qbx_linalg.hip, csrc/qbx_boys_probe.hip, csrc/qbx_eri_generic.hip and every
+csrc/gen/), compile csrc/qbx.hip, csrc/qbx_mlp.hip, csrc/qbx_linalg.hip, csrc/qbx_boys_probe.hip, csrc/qbx_eri_generic.hip, csrc/qbx_one_e.hip and every
 csrc/gen/eri_*.hip to objects in
 parallel with hipcc, link quiqbox_amd/libqbx_hip.so.  Objects whose sources and
 headers are unchanged are reused.
@@ -90,10 +90,11 @@ def build(verbose=True, extra=(), jobs=None, force=False):
     t0 = time.time()
     generate()
     headers = sorted(glob.glob(os.path.join(CSRC, "*.h")) + [os.path.join(GEN, "eri_table.inc"),
+                                                              os.path.join(GEN, "one_e_classes.inc"),
                                                               os.path.join(INCLUDE, "qbx.h")])
     srcs = [os.path.join(CSRC, "qbx.hip"), os.path.join(CSRC, "qbx_mlp.hip"),
             os.path.join(CSRC, "qbx_linalg.hip"), os.path.join(CSRC, "qbx_boys_probe.hip"),
-            os.path.join(CSRC, "qbx_eri_generic.hip")] + sorted(glob.glob(os.path.join(GEN, "eri_*.hip")),
+            os.path.join(CSRC, "qbx_eri_generic.hip"), os.path.join(CSRC, "qbx_one_e.hip")] + sorted(glob.glob(os.path.join(GEN, "eri_*.hip")),
                                                      key=lambda p: -os.path.getsize(p))
     jobs = jobs or max(1, min(len(srcs), os.cpu_count() or 4))
     objs = {}

@@ -63,6 +63,11 @@ LMAX = 2
 PAIR_LMAX = 4
 # classes with an adjoint (gradient) kernel: every shell s or p
 GRAD_LMAX = 1
+# Gradient classes whose [e0|f0] seeds are split by bra component into groups,
+# one kernel each (the gradient is linear in the seeds, and so are the derivatives
+# with respect to A-B and C-D in the contracted [e0|f0]): the forward and adjoint
+# values of all 81 targets of (pp|pp) do not fit 512 registers.
+GRAD_GROUPS = {(1, 1, 1, 1): 3}
 # classes evaluated in groups of bra components through a workspace
 STAGED = {(2, 1, 1, 1), (2, 1, 2, 1), (2, 2, 1, 1), (2, 2, 2, 0), (2, 2, 2, 1), (2, 2, 2, 2)}
 STAGE_ACC = 32     # accumulators per group
@@ -464,16 +469,11 @@ def _adj(x):
     return "b" + x
 
 
-def gen_adjoint(la, lb, lc, ld):
-    """EriAdj<la, lb, lc, ld> (see the module docstring) and its flop counts."""
-    es = [e for L in range(la, la + lb + 1) for e in cart(L)]
-    fs = [f for L in range(lc, lc + ld + 1) for f in cart(L)]
-    eidx = {e: n for n, e in enumerate(es)}
-    fidx = {f: n for n, f in enumerate(fs)}
-    nF = len(fs)
-    targets = [(e, f) for e in es for f in fs]
-    nodes, out = vrr_dag(targets)
-    Lt = la + lb + lc + ld
+def adjoint_statements(sub, tidx):
+    """Forward recurrence of the targets `sub` ({target: index} tidx) and its
+    adjoint: (forward lines, adjoint lines, seeded-sum terms, {target: name},
+    operations of the adjoint)."""
+    nodes, out = vrr_dag(sub)
     fwd, rev = [], []
     flops = 0
     for name, terms in nodes:
@@ -486,13 +486,13 @@ def gen_adjoint(la, lb, lc, ld):
             else:
                 ex.append("%d.0 * inv2pq * %s" % (t[1], t[2]))
         fwd.append("const double %s = %s;" % (name, " + ".join(ex)))
-    decl = ["double %s = 0.0;" % _adj(n) for n, _ in nodes]
-    decl += ["double b_%s = 0.0;" % x for x in VRR_INPUTS]
-    seed = []
+    rev += ["double %s = 0.0;" % _adj(n) for n, _ in nodes]
+    rev += ["double b_%s = 0.0;" % x for x in VRR_INPUTS]
     lsum = []
-    for k, t in enumerate(targets):
-        seed.append("%s += g[%d];" % (_adj(out[t]), k))
-        lsum.append("g[%d] * %s" % (k, out[t]))
+    for t in sub:
+        rev.append("%s += g[%d];" % (_adj(out[t]), tidx[t]))
+        lsum.append("g[%d] * %s" % (tidx[t], out[t]))
+    nk = 0
     for name, terms in reversed(nodes):
         b = _adj(name)
         for t in terms:
@@ -501,16 +501,40 @@ def gen_adjoint(la, lb, lc, ld):
                 rev.append("b_%s += %s * %s;" % (t[1], t[2], b))
                 flops += 4
             elif t[0] == "ho":
+                # y = k inv (c - rho d): with kb = k b and x = inv kb, bc += x,
+                # bd -= rho x, b_inv += (c - rho d) kb, b_rho -= d x
                 k, inv, rho, c, d = t[1:]
-                rev.append("%s += %d.0 * %s * %s;" % (_adj(c), k, inv, b))
-                rev.append("%s -= %d.0 * %s * %s * %s;" % (_adj(d), k, inv, rho, b))
-                rev.append("b_%s += %d.0 * (%s - %s * %s) * %s;" % (inv, k, c, rho, d, b))
-                rev.append("b_%s -= %d.0 * %s * %s * %s;" % (rho, k, inv, d, b))
-                flops += 14
+                nk += 1
+                rev.append("const double kb%d = %d.0 * %s;" % (nk, k, b))
+                rev.append("const double xb%d = %s * kb%d;" % (nk, inv, nk))
+                rev.append("%s += xb%d;" % (_adj(c), nk))
+                rev.append("%s -= %s * xb%d;" % (_adj(d), rho, nk))
+                rev.append("b_%s += (%s - %s * %s) * kb%d;" % (inv, c, rho, d, nk))
+                rev.append("b_%s -= %s * xb%d;" % (rho, d, nk))
+                flops += 11
             else:
-                rev.append("%s += %d.0 * inv2pq * %s;" % (_adj(t[2]), t[1], b))
-                rev.append("b_inv2pq += %d.0 * %s * %s;" % (t[1], t[2], b))
-                flops += 6
+                nk += 1
+                rev.append("const double kb%d = %d.0 * %s;" % (nk, t[1], b))
+                rev.append("%s += inv2pq * kb%d;" % (_adj(t[2]), nk))
+                rev.append("b_inv2pq += %s * kb%d;" % (t[2], nk))
+                flops += 5
+    rev.append(" ".join("bin[%d] = b_%s;" % (k, x) for k, x in enumerate(VRR_INPUTS)))
+    return fwd, rev, lsum, out, flops
+
+
+def gen_adjoint(la, lb, lc, ld, groups=None):
+    """EriAdj<la, lb, lc, ld> (see the module docstring) and its flop counts.
+    groups=None: vrr_adj over all targets; an integer: vrr_adj_grp<0 ..
+    groups - 1>, each over its share of the bra components e, which also adds
+    the forward values to acc."""
+    es = [e for L in range(la, la + lb + 1) for e in cart(L)]
+    fs = [f for L in range(lc, lc + ld + 1) for f in cart(L)]
+    eidx = {e: n for n, e in enumerate(es)}
+    fidx = {f: n for n, f in enumerate(fs)}
+    nF = len(fs)
+    targets = [(e, f) for e in es for f in fs]
+    tidx = {t: k for k, t in enumerate(targets)}
+    Lt = la + lb + lc + ld
     code = []
     code.append("template <> struct EriAdj<%d, %d, %d, %d> {" % (la, lb, lc, ld))
     code.append("    static constexpr int NACC = %d;" % len(targets))
@@ -518,19 +542,37 @@ def gen_adjoint(la, lb, lc, ld):
     code.append("    // g[NACC] on [e0|f0]: Fb[m] = d/dF_m, bin[] = d/d(%s)," % ", ".join(VRR_INPUTS[:4]) + " ...")
     code.append("    // in the order PA, WP, QC, WQ (x, y, z each), inv2p, inv2q, inv2pq, rho_p, rho_q;")
     code.append("    // returns sum_k g[k] [e0|f0]_k")
-    code.append("    static __device__ __forceinline__ double vrr_adj(const double* __restrict__ F, "
-                "const double* __restrict__ g,")
-    code.append("        double PAx, double PAy, double PAz, double WPx, double WPy, double WPz,")
-    code.append("        double QCx, double QCy, double QCz, double WQx, double WQy, double WQz,")
-    code.append("        double inv2p, double inv2q, double inv2pq, double rho_p, double rho_q,")
-    code.append("        double* __restrict__ Fb, double* __restrict__ bin) {")
-    code += ["        " + l for l in fwd]
-    code.append("#pragma unroll")
-    code.append("        for (int m = 0; m <= %d; ++m) Fb[m] = 0.0;" % Lt)
-    code += ["        " + l for l in decl + seed + rev]
-    code.append("        " + " ".join("bin[%d] = b_%s;" % (k, x) for k, x in enumerate(VRR_INPUTS)))
-    code.append("        return %s;" % " + ".join(lsum))
-    code.append("    }")
+    geo = ["        double PAx, double PAy, double PAz, double WPx, double WPy, double WPz,",
+           "        double QCx, double QCy, double QCz, double WQx, double WQy, double WQz,",
+           "        double inv2p, double inv2q, double inv2pq, double rho_p, double rho_q,",
+           "        double* __restrict__ Fb, double* __restrict__ bin) {",
+           "#pragma unroll",
+           "        for (int m = 0; m <= %d; ++m) Fb[m] = 0.0;" % Lt]
+    if groups is None:
+        fwd, rev, lsum, _, flops = adjoint_statements(targets, tidx)
+        code.append("    static __device__ __forceinline__ double vrr_adj(const double* __restrict__ F, "
+                    "const double* __restrict__ g,")
+        code += geo + ["        " + l for l in fwd + rev]
+        code.append("        return %s;" % " + ".join(lsum))
+        code.append("    }")
+    else:
+        flops = 0
+        bounds = [k * len(es) // groups for k in range(groups + 1)]
+        code.append("    // Group GR takes its share of the bra components e; acc[k] += [e0|f0]_k of the group.")
+        code.append("    static constexpr int NGRP = %d;" % groups)
+        code.append("    template <int GR> static __device__ __forceinline__ double vrr_adj_grp(const double* __restrict__ F,")
+        code.append("        const double* __restrict__ g, double* __restrict__ acc,")
+        code += geo
+        for gr in range(groups):
+            sub = [(e, f) for e in es[bounds[gr]:bounds[gr + 1]] for f in fs]
+            fwd, rev, lsum, out, fl = adjoint_statements(sub, tidx)
+            flops += fl
+            fwd += ["acc[%d] += %s;" % (tidx[t], out[t]) for t in sub]
+            code.append("        %sif constexpr (GR == %d) {" % ("" if gr == 0 else "else ", gr))
+            code += ["            " + l for l in fwd + rev]
+            code.append("            return %s;" % " + ".join(lsum))
+            code.append("        }")
+        code.append("    }")
 
     # full horizontal recurrence (ket, then bra) as a graph of n = x + coef * y
     C_, D_, A_, B_ = cart(lc), cart(ld), cart(la), cart(lb)
@@ -593,8 +635,9 @@ def gen_adjoint(la, lb, lc, ld):
         hflops += 5
     code.append("    static constexpr int NINT = %d;" % len(outs))
     code.append("    // adjoint of the horizontal recurrence: seeds G[NINT] on the contracted (ab|cd)")
-    code.append("    // (index ((ia * NB + ib) * NC + ic) * ND + id) -> accb[NACC] on the contracted [e0|f0],")
-    code.append("    // bAB[3], bCD[3] = derivatives with respect to A-B and C-D; returns sum_k G[k] (ab|cd)_k")
+    code.append("    // (index ((ia * NB + ib) * NC + ic) * ND + id) -> accb[NACC] on the contracted [e0|f0]")
+    code.append("    // (independent of acc), bAB[3], bCD[3] = derivatives with respect to A-B and C-D (linear in")
+    code.append("    // acc); returns sum_k G[k] (ab|cd)_k")
     code.append("    static __device__ __forceinline__ double hrr_adj(const double* __restrict__ acc, "
                 "const double* __restrict__ G,")
     code.append("        double* __restrict__ accb, double* __restrict__ bAB, double* __restrict__ bCD,")
@@ -609,6 +652,151 @@ def gen_adjoint(la, lb, lc, ld):
     code.append("    }")
     code.append("};")
     return "\n".join(code), flops, hflops
+
+
+# ---------------------------------------------------------------------------
+# one-electron recurrences: nuclear attraction of every pair class, and the
+# one-electron energy gradient of the s and p pair classes
+# ---------------------------------------------------------------------------
+def nuclear_vrr(targets):
+    """Statements of the one-body vertical recurrence
+    [e+1_i]^(m) = PA_i [e]^(m) - PC_i [e]^(m+1) + e_i/2p ([e-1_i]^(m) - [e-1_i]^(m+1))
+    and {e: name} of the m = 0 targets."""
+    em = Emitter()
+    memo = {}
+
+    def V(e, m):
+        if (e, m) in memo:
+            return memo[e, m]
+        if sum(e) == 0:
+            memo[e, m] = "F[%d]" % m
+            return memo[e, m]
+        i = pick_axis(e)
+        e1 = sub1(e, i)
+        expr = "PA%s * %s - PC%s * %s" % (AX[i], V(e1, m), AX[i], V(e1, m + 1))
+        if e1[i] > 0:
+            e2 = sub1(e1, i)
+            expr += " + %d.0 * inv2p * (%s - %s)" % (e1[i], V(e2, m), V(e2, m + 1))
+        name = em.fresh("v")
+        em.lines.append("const double %s = %s;" % (name, expr))
+        memo[e, m] = name
+        return name
+
+    out = {e: V(e, 0) for e in targets}
+    return em.lines, out
+
+
+def bra_transfer(em, leaf):
+    """(a, b) -> name with (a, b+1_i) = (a+1_i, b) + AB_i (a, b); leaf(e) names
+    the one-index values."""
+    memo = {}
+
+    def H(a, b):
+        if (a, b) in memo:
+            return memo[a, b]
+        if sum(b) == 0:
+            memo[a, b] = leaf(a)
+            return memo[a, b]
+        i = pick_axis(b)
+        b1 = sub1(b, i)
+        x, y = H(add1(a, i), b1), H(a, b1)
+        name = em.fresh("h")
+        em.lines.append("const double %s = %s + AB%s * %s;" % (name, x, AX[i], y))
+        memo[a, b] = name
+        return name
+
+    return H
+
+
+def gen_nuclear(la, lb):
+    """OneE<la, lb>: recurrences of the nuclear-attraction kernel."""
+    es = [e for L in range(la, la + lb + 1) for e in cart(L)]
+    eidx = {e: n for n, e in enumerate(es)}
+    lines, out = nuclear_vrr(es)
+    hm = Emitter()
+    H = bra_transfer(hm, lambda e: "acc[%d]" % eidx[e])
+    outs = ["out[%d] = %s;" % (ia * ncart(lb) + ib, H(a, b))
+            for ia, a in enumerate(cart(la)) for ib, b in enumerate(cart(lb))]
+    code = ["template <> struct OneE<%d, %d> {" % (la, lb),
+            "    static constexpr int NACC = %d;" % len(es),
+            "    // acc[e] += [e] of one primitive pair and nucleus, F scaled by the prefactor",
+            "    static __device__ __forceinline__ void vrr(const double* __restrict__ F, double* __restrict__ acc,",
+            "        double PAx, double PAy, double PAz, double PCx, double PCy, double PCz, double inv2p) {"]
+    code += ["        " + l for l in lines]
+    code += ["        acc[%d] += %s;" % (eidx[e], out[e]) for e in es]
+    code += ["    }",
+             "    // out[ia * NB + ib] = (a b) from the contracted [e]",
+             "    static __device__ __forceinline__ void hrr(const double* __restrict__ acc, double* __restrict__ out,",
+             "        double ABx, double ABy, double ABz) {"]
+    code += ["        " + l for l in hm.lines + outs]
+    code += ["    }", "};"]
+    return "\n".join(code)
+
+
+def gen_one_e_grad(la, lb):
+    """OneGrad<la, lb>: the one-electron energy gradient of one primitive pair.
+    acc[e], |e| <= la + lb + 2, hold the attraction values of the raised
+    functions on A summed over the nuclei; the derivatives of
+    sum_ab wd_ab (T + V)_ab - ww_ab S_ab are combinations of integrals with one
+    centre raised by one or two or lowered by one:
+        d/dA_i = 2 alpha (a+1_i, b) - a_i (a-1_i, b),  d/dalpha = -sum_i (a+2_i, b)
+    and likewise for B."""
+    es = [e for L in range(0, la + lb + 3) for e in cart(L)]
+    eidx = {e: n for n, e in enumerate(es)}
+    lines, out = nuclear_vrr(es)
+    hm = Emitter()
+    H = bra_transfer(hm, lambda e: "acc[%d]" % eidx[e])
+    names = {}
+    body = []
+
+    def I(a, b):
+        """(T + V, S) names of one integral"""
+        if (a, b) not in names:
+            v = H(a, b)
+            k = len(names)
+            sx = ["s[%d][%d][%d]" % (t, a[t], b[t]) for t in range(3)]
+            kx = ["k[%d][%d][%d]" % (t, a[t], b[t]) for t in range(3)]
+            hm.lines.append("const double S%d = pre * (%s * %s * %s);" % (k, sx[0], sx[1], sx[2]))
+            hm.lines.append("const double I%d = %s - 0.5 * pre * (%s * %s * %s + %s * %s * %s + %s * %s * %s);" % (
+                k, v, kx[0], sx[1], sx[2], sx[0], kx[1], sx[2], sx[0], sx[1], kx[2]))
+            names[a, b] = k
+        return names[a, b]
+
+    for ia, a in enumerate(cart(la)):
+        for ib, b in enumerate(cart(lb)):
+            n = ia * ncart(lb) + ib
+
+            def term(*cs):
+                x = " + ".join("%s * I%d" % c if c[0] != "1" else "I%d" % c[1] for c in cs)
+                y = " + ".join("%s * S%d" % c if c[0] != "1" else "S%d" % c[1] for c in cs)
+                return "wd[%d] * (%s) - ww[%d] * (%s)" % (n, x, n, y)
+
+            body.append("gl += %s;" % term(("1", I(a, b))))
+            for who, x, y, g in (("alpha", a, b, "gA"), ("beta", b, a, "gB")):
+                J = (lambda p, q: I(p, q)) if who == "alpha" else (lambda p, q: I(q, p))
+                up2 = [("1", J(add1(add1(x, i), i), y)) for i in range(3)]
+                body.append("%s -= %s;" % ("gxa" if who == "alpha" else "gxb", term(*up2)))
+                for i in range(3):
+                    cs = [("(2.0 * %s)" % who, J(add1(x, i), y))]
+                    if x[i] > 0:
+                        cs.append(("-%d.0" % x[i], J(sub1(x, i), y)))
+                    body.append("%s[%d] += %s;" % (g, i, term(*cs)))
+    code = ["template <> struct OneGrad<%d, %d> {" % (la, lb),
+            "    static constexpr int NACC = %d;" % len(es),
+            "    static __device__ __forceinline__ void vrr(const double* __restrict__ F, double* __restrict__ acc,",
+            "        double PAx, double PAy, double PAz, double PCx, double PCy, double PCz, double inv2p) {"]
+    code += ["        " + l for l in lines]
+    code += ["        acc[%d] += %s;" % (eidx[e], out[e]) for e in es]
+    code += ["    }",
+             "    // s, k: the overlap and second-derivative factors per axis, [a power][b power]",
+             "    static __device__ __forceinline__ void derivatives(const double* __restrict__ acc,",
+             "        const double (&s)[3][%d][%d], const double (&k)[3][%d][%d], double pre," % (
+                 la + 3, lb + 5, la + 3, lb + 3),
+             "        const double* __restrict__ wd, const double* __restrict__ ww, double alpha, double beta,",
+             "        double ABx, double ABy, double ABz, double& gl, double& gxa, double& gxb, double* gA, double* gB) {"]
+    code += ["        " + l for l in hm.lines + body]
+    code += ["    }", "};"]
+    return "\n".join(code)
 
 
 def stage_ws(la, lb, lc, ld):
@@ -780,14 +968,14 @@ def main(outdir):
         if (la, lb) == (lc, ld):
             variants.append(("double", "MODE_SCHWARZ", "schwarz"))
         if max(la, lb, lc, ld) <= GRAD_LMAX:
-            acode, af, ah = gen_adjoint(la, lb, lc, ld)
+            acode, af, ah = gen_adjoint(la, lb, lc, ld, GRAD_GROUPS.get((la, lb, lc, ld), 1))
             flops[tag]["adjoint_vrr_per_prim_quartet"] = af
             flops[tag]["adjoint_hrr_per_quartet"] = ah
             tu = ["// Generated by gen_eri.py -- do not edit.",
                   "// ERI class (%d %d | %d %d): adjoint recurrences and gradient kernel instantiation."
                   % (la, lb, lc, ld),
                   '#include "qbx_grad.h"', "", code, "", acode, "", "namespace qbx {",
-                  "template void launch_eri_grad<%d, %d, %d, %d>(const EriArgs&, hipStream_t);" % (la, lb, lc, ld),
+                  "template void launch_eri_grad<%d, %d, %d, %d>(const EriArgs&, hipStream_t*, int);" % (la, lb, lc, ld),
                   "}  // namespace qbx"]
             with open(os.path.join(outdir, "eri_%s_grad.hip" % tag), "w") as f:
                 f.write("\n".join(tu) + "\n")
@@ -801,6 +989,14 @@ def main(outdir):
                   "}  // namespace qbx"]
             with open(os.path.join(outdir, "eri_%s_%s.hip" % (tag, vtag)), "w") as f:
                 f.write("\n".join(tu) + "\n")
+    tu = ["// Generated by gen_eri.py -- do not edit.",
+          "// One-electron recurrences of the pair classes (nuclear attraction, energy gradient).", "#pragma once",
+          "namespace qbx {", "template <int LA, int LB> struct OneE;", "template <int LA, int LB> struct OneGrad;"]
+    tu += [gen_nuclear(a, b) for a in range(PAIR_LMAX + 1) for b in range(a + 1)]
+    tu += [gen_one_e_grad(a, b) for a in range(GRAD_LMAX + 1) for b in range(a + 1)]
+    tu.append("}  // namespace qbx")
+    with open(os.path.join(outdir, "one_e_classes.inc"), "w") as f:
+        f.write("\n".join(tu) + "\n")
     # class table for the host dispatcher
     lines = ["// Generated by gen_eri.py -- do not edit.", "#pragma once",
              "#define QBX_GEN_LMAX %d" % LMAX,

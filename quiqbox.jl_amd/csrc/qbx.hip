@@ -37,6 +37,7 @@
 #include "qbx_common.h"
 #include "qbx_eri_api.h"
 #include "qbx_linalg.h"
+#include "qbx_one_e.h"
 #include "gen/eri_table.inc"
 
 using namespace qbx;
@@ -480,135 +481,6 @@ __global__ __launch_bounds__(256) void prim_one_e_kernel(PrimOneArgs g)
     g.out[i] = val;
 }
 
-// ---------------------------------------------------------------------------
-// kernel: one-electron part of the RHF energy gradient
-// ---------------------------------------------------------------------------
-struct OneGradArgs {
-    const DevShell* sh;
-    const PrimPair* pp;
-    const int* ppk;
-    const int* pA;
-    const int* pB;
-    const int* po;
-    const int* pn;
-    int npair;
-    int N;
-    const double* boys;
-    const double* bexp;
-    int nnuc;
-    const double* Z;
-    const double* R;
-    const double* Dt;      // total density
-    const double* W;       // energy-weighted density
-    const int* poff;
-    double* g_xpn;
-    double* g_lin;
-    double* g_cen;
-};
-
-constexpr int kGradPairPrims = QBX_GRAD_MAXP * QBX_GRAD_MAXP;   // primitive pairs per shell pair in the 1e gradient grid
-
-// D (T + V) - W S for one primitive pair and Cartesian components la, lb of
-// the two primitives (any angular momentum up to 2 above the shells').
-__device__ double one_e_energy(const int* la, const int* lb, const PrimPair& P, const double* AB,
-                               const OneGradArgs& a, double wd, double ww)
-{
-    const double PA[3] = {P.PAx, P.PAy, P.PAz};
-    const double PB[3] = {P.PAx + AB[0], P.PAy + AB[1], P.PAz + AB[2]};
-    double S[3][QBX_OV_MAX][QBX_OV_MAX];
-    for (int t = 0; t < 3; ++t) qbx_ov1d(PA[t], PB[t], P.inv2p, la[t], lb[t] + 2, S[t]);
-    const double sx = S[0][la[0]][lb[0]], sy = S[1][la[1]][lb[1]], sz = S[2][la[2]][lb[2]];
-    const double b = P.pad;
-    double d2[3];
-    for (int t = 0; t < 3; ++t) {
-        const int j = lb[t];
-        double r = -2.0 * b * (2 * j + 1) * S[t][la[t]][j] + 4.0 * b * b * S[t][la[t]][j + 2];
-        if (j > 1) r += (double)(j * (j - 1)) * S[t][la[t]][j - 2];
-        d2[t] = r;
-    }
-    const double pre = 5.568327996831707845 * P.Kp * rsqrt(P.p);
-    const double ovl = pre * sx * sy * sz;
-    const double kin = pre * -0.5 * (d2[0] * sy * sz + sx * d2[1] * sz + sx * sy * d2[2]);
-    double nuc = 0.0;
-    if (wd != 0.0) {
-        const int Lt = la[0] + la[1] + la[2] + lb[0] + lb[1] + lb[2];
-        for (int n = 0; n < a.nnuc; ++n) {
-            const double PC[3] = {P.Px - a.R[3 * n], P.Py - a.R[3 * n + 1], P.Pz - a.R[3 * n + 2]};
-            const double T = P.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
-            double F[9];   // s and p shells (the gradient rejects higher L), raised by up to two orders
-            qbx_boys_rt(Lt, T, F, a.boys, a.bexp);
-            nuc += a.Z[n] * coulomb1_comp_t<8>(la, lb, PA, PC, AB, P.inv2p, F, Lt);
-        }
-        nuc *= -2.0 * kPi * P.Kp;
-    }
-    return wd * (kin + nuc) - ww * ovl;
-}
-
-// One thread per (shell pair, primitive pair).  With I(a, b) an integral over
-// the primitives' Cartesian components a, b (weights included):
-//   dI/dA_i = 2 alpha I(a + 1_i, b) - a_i I(a - 1_i, b),
-//   dI/dalpha = -sum_i I(a + 2_i, b)   (d/dalpha exp(-alpha r_A^2) = -r_A^2 exp(...)),
-// likewise for B, beta; and c dI/dc = I for either primitive.
-__global__ __launch_bounds__(256) void one_e_grad_kernel(OneGradArgs a)
-{
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int pair = gid / kGradPairPrims, u = gid % kGradPairPrims;
-    if (pair >= a.npair || u >= a.pn[pair]) return;
-    const int sA = a.pA[pair], sB = a.pB[pair];
-    const DevShell A = a.sh[sA];
-    const DevShell B = a.sh[sB];
-    const PrimPair P = a.pp[a.po[pair] + u];
-    const int kab = a.ppk[a.po[pair] + u];
-    const int ka = kab & 0xffff, kb = kab >> 16;
-    const double alpha = P.p - P.pad, beta = P.pad;
-    const double AB[3] = {A.x - B.x, A.y - B.y, A.z - B.z};
-    const double fac = sA == sB ? 1.0 : 2.0;
-    const size_t N = (size_t)a.N;
-    double gxa = 0.0, gxb = 0.0, gl = 0.0, gAc[3] = {0.0, 0.0, 0.0}, gBc[3] = {0.0, 0.0, 0.0};
-    for (int ca = 0; ca < qbx_ncart(A.L); ++ca)
-        for (int cb = 0; cb < qbx_ncart(B.L); ++cb) {
-            const int ia = A.bf[ca], ib = B.bf[cb];
-            if (ia < 0 || ib < 0) continue;
-            int la[3], lb[3];
-            qbx_cart(A.L, ca, la);
-            qbx_cart(B.L, cb, lb);
-            const double sc = fac * A.sc[ca] * B.sc[cb];
-            const double wd = sc * a.Dt[ia * N + ib], ww = sc * a.W[ia * N + ib];
-            gl += one_e_energy(la, lb, P, AB, a, wd, ww);
-            for (int i = 0; i < 3; ++i) {
-                int l2[3] = {la[0], la[1], la[2]};
-                l2[i] += 2;
-                gxa -= one_e_energy(l2, lb, P, AB, a, wd, ww);
-                l2[i] -= 1;
-                double g = 2.0 * alpha * one_e_energy(l2, lb, P, AB, a, wd, ww);
-                if (la[i] > 0) {
-                    l2[i] -= 2;
-                    g -= la[i] * one_e_energy(l2, lb, P, AB, a, wd, ww);
-                }
-                gAc[i] += g;
-                int m2[3] = {lb[0], lb[1], lb[2]};
-                m2[i] += 2;
-                gxb -= one_e_energy(la, m2, P, AB, a, wd, ww);
-                m2[i] -= 1;
-                g = 2.0 * beta * one_e_energy(la, m2, P, AB, a, wd, ww);
-                if (lb[i] > 0) {
-                    m2[i] -= 2;
-                    g -= lb[i] * one_e_energy(la, m2, P, AB, a, wd, ww);
-                }
-                gBc[i] += g;
-            }
-        }
-    const int pA = a.poff[sA], pB = a.poff[sB];
-    atomicAdd(a.g_xpn + pA + ka, gxa);
-    atomicAdd(a.g_xpn + pB + kb, gxb);
-    atomicAdd(a.g_lin + pA + ka, gl);
-    atomicAdd(a.g_lin + pB + kb, gl);
-    for (int i = 0; i < 3; ++i) {
-        atomicAdd(a.g_cen + 3 * sA + i, gAc[i]);
-        atomicAdd(a.g_cen + 3 * sB + i, gBc[i]);
-    }
-}
-
 // One thread per (shell pair, component pair); a.mc components per shell
 // (those of the basis's highest L).  NM: twice the highest L (the nuclear
 // attraction's recurrence size).
@@ -648,18 +520,6 @@ __global__ __launch_bounds__(256) void one_e_kernel(OneArgs a)
                 if (side) accB += v;
                 else acc += v;
             }
-        } else if (KIND == ONE_NUCLEAR) {
-            const int Lt = A.L + B.L;
-            const double Pc[3] = {P.Px, P.Py, P.Pz};
-            double v = 0.0;
-            for (int n = 0; n < a.nnuc; ++n) {
-                const double PC[3] = {Pc[0] - a.R[3 * n], Pc[1] - a.R[3 * n + 1], Pc[2] - a.R[3 * n + 2]};
-                const double T = P.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
-                double F[NM + 1];
-                qbx_boys_rt(Lt, T, F, a.boys, a.bexp);
-                v += a.Z[n] * coulomb1_comp_t<NM>(la, lb, PA, PC, AB, P.inv2p, F, Lt);
-            }
-            acc += -2.0 * kPi * P.Kp * v;
         } else {
             double S[3][QBX_OV_MAX][QBX_OV_MAX];
             const int extra = KIND == ONE_KINETIC ? 2 : (KIND == ONE_MULTIPOLE ? 0 : 0);
@@ -803,7 +663,7 @@ const EriLaunch k_jk64[QBX_N_CLASSES] = {QBX_FOR_EACH_CLASS(QBX_E64JK)};
 const EriLaunch k_jk32[QBX_N_CLASSES] = {QBX_FOR_EACH_CLASS(QBX_E32JK)};
 const EriLaunch k_dense[QBX_N_CLASSES] = {QBX_FOR_EACH_CLASS(QBX_EDENSE)};
 
-EriLaunch grad_launcher(int cls)
+EriGradLaunch grad_launcher(int cls)
 {
     const int* L = qbx_class_l[cls];
 #define QBX_GR(a, b, c, d) \
@@ -1413,6 +1273,25 @@ void check_ctx_basis(qbx_ctx* ctx, const qbx_basis* b)
     if (b->ctx != ctx) throw QbxError(QBX_EINVAL, "basis belongs to another context");
 }
 
+// Boys rows of one order
+const double* boys_order(const qbx_ctx* ctx, int L)
+{
+    return ctx->boysl.p + (size_t)L * QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE;
+}
+
+NucArgs nuc_base(const qbx_basis* b, int nnuc, const double* dZ, const double* dR)
+{
+    NucArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.pp = b->d_pp.p;
+    g.sh = b->d_sh.p;
+    g.N = b->nbf;
+    g.nnuc = nnuc;
+    g.Z = dZ;
+    g.R = dR;
+    return g;
+}
+
 void run_one_e(qbx_ctx* ctx, const qbx_basis* b, int kind, int nnuc, const double* Z, const double* R,
                const double* M, const int32_t* deg, double* out)
 {
@@ -1468,7 +1347,16 @@ void run_one_e(qbx_ctx* ctx, const qbx_basis* b, int kind, int nnuc, const doubl
     }
     a.mc = qbx_ncart(b->maxL);
     const int64_t threads = (int64_t)a.npair * a.mc * a.mc;
-    if (threads > 0) {
+    if (kind == ONE_NUCLEAR) {
+        NucArgs g = nuc_base(b, nnuc, dZ.p, dR.p);
+        g.out = dout.p;
+        for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
+            const int la = qbx_pair_class_l[c][0], lb = qbx_pair_class_l[c][1];
+            g.pairs = pcdev(b->pc[c]);
+            g.boysl = boys_order(ctx, la + lb);
+            launch_nuclear(la, lb, g, st);
+        }
+    } else if (threads > 0) {
         if ((threads + 255) / 256 > 0x7fffffffLL) throw QbxError(QBX_EUNSUP, "basis too large for one grid");
         const int blocks = (int)((threads + 255) / 256);
         auto go = [&](auto nm) {
@@ -1479,9 +1367,6 @@ void run_one_e(qbx_ctx* ctx, const qbx_basis* b, int kind, int nnuc, const doubl
                 break;
             case ONE_KINETIC:
                 hipLaunchKernelGGL((one_e_kernel<ONE_KINETIC, NM>), dim3(blocks), dim3(256), 0, st, a);
-                break;
-            case ONE_NUCLEAR:
-                hipLaunchKernelGGL((one_e_kernel<ONE_NUCLEAR, NM>), dim3(blocks), dim3(256), 0, st, a);
                 break;
             case ONE_NUCLEAR_OWN:
                 hipLaunchKernelGGL((one_e_kernel<ONE_NUCLEAR_OWN, NM>), dim3(blocks), dim3(256), 0, st, a);
@@ -2743,43 +2628,31 @@ void hf_gradient(qbx_ctx* ctx, qbx_basis* b, const double* Dt, const double* Da,
         zero_async(gx.p, nr, st);
         zero_async(gl.p, nr, st);
         zero_async(gc.p, 3 * (size_t)ns, st);
-        // one-electron part
-        OneGradArgs o;
-        std::memset(&o, 0, sizeof(o));
-        o.sh = b->d_sh.p;
-        o.pp = b->d_pp.p;
-        o.ppk = b->d_ppk.p;
-        o.pA = b->d_p1A.p;
-        o.pB = b->d_p1B.p;
-        o.po = b->d_p1o.p;
-        o.pn = b->d_p1n.p;
-        o.npair = (int)b->p1.size();
-        o.N = b->nbf;
-        o.boys = ctx->boys.p;
-        o.bexp = ctx->bexp.p;
-        o.nnuc = n_nuc;
-        o.Z = dZ.p;
-        o.R = dR.p;
+        NucArgs o = nuc_base(b, n_nuc, dZ.p, dR.p);
         o.Dt = dD.p;
         o.W = dW.p;
+        o.ppk = b->d_ppk.p;
         o.poff = b->d_poff.p;
         o.g_xpn = gx.p;
         o.g_lin = gl.p;
         o.g_cen = gc.p;
-        const int64_t threads = (int64_t)o.npair * kGradPairPrims;
-        if (threads > 0) {
-            hipLaunchKernelGGL(one_e_grad_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, o);
-            QBX_HIP(hipGetLastError());
-        }
-        // two-electron part
-        for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
+        // the kernels only meet in the atomics of the three outputs: all classes
+        // run concurrently on the auxiliary streams, the largest work first
+        QBX_HIP(hipEventRecord(ctx->ev_fork, st));
+        for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
+        std::vector<int> order(QBX_N_CLASSES);
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(),
+                         [&](int x, int y) { return b->class_cost[x] > b->class_cost[y]; });
+        int launched = 0;
+        for (int cls : order) {
             const TaskSet& t64 = b->t64[cls];
             if (t64.nwave <= 0) continue;
-            EriLaunch f = grad_launcher(cls);
+            EriGradLaunch f = grad_launcher(cls);
             if (!f) throw QbxError(QBX_EINTERNAL, "no gradient kernel for an occupied class");
             EriArgs a = base_args(b, cls);
             const int lt = qbx_class_l[cls][0] + qbx_class_l[cls][1] + qbx_class_l[cls][2] + qbx_class_l[cls][3];
-            a.boysl = ctx->boysl.p + (size_t)(lt + 1) * QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE;
+            a.boysl = boys_order(ctx, lt + 1);
             a.D = dD.p;
             a.nset = uhf ? 2 : 1;
             a.prefix = t64.prefix.p;
@@ -2788,12 +2661,30 @@ void hf_gradient(qbx_ctx* ctx, qbx_basis* b, const double* Dt, const double* Da,
             a.total = t64.total;
             a.nwave = t64.nwave;
             a.nbra = t64.nbra;
+            a.lds_max = ctx->lds_max;
+            a.nshell = ns;
             a.ppk = b->d_ppk.p;
             a.shell_poff = b->d_poff.p;
+            a.n_radial = nr;
             a.g_xpn = gx.p;
             a.g_lin = gl.p;
             a.g_cen = gc.p;
-            f(a, st);
+            // rotated, so that each class starts on another stream
+            hipStream_t lanes[kStreams];
+            for (int k = 0; k < kStreams; ++k) lanes[k] = ctx->aux[(launched + k) % kStreams];
+            f(a, lanes, kStreams);
+            ++launched;
+        }
+        for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
+            const int la = qbx_pair_class_l[c][0], lb = qbx_pair_class_l[c][1];
+            if (b->pc[c].n() == 0) continue;
+            o.pairs = pcdev(b->pc[c]);
+            o.boysl = boys_order(ctx, la + lb + 2);
+            launch_one_e_grad(la, lb, o, ctx->aux[launched++ % kStreams]);
+        }
+        for (int k = 0; k < kStreams; ++k) {
+            QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
+            QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
         }
         QBX_HIP(hipMemcpyAsync(g_xpn, gx.p, nr * sizeof(double), hipMemcpyDeviceToHost, st));
         QBX_HIP(hipMemcpyAsync(g_lin, gl.p, nr * sizeof(double), hipMemcpyDeviceToHost, st));

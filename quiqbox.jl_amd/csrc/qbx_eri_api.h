@@ -95,6 +95,8 @@ struct EriArgs {
     // primitive dE/d(exponent) and c dE/dc, per shell dE/d(centre)
     const int* ppk;
     const int* shell_poff;
+    int n_radial;             // radial primitives (length of g_xpn and g_lin)
+    int grad_lds;             // doubles of a block's LDS copy of the three outputs (0: none)
     double* g_xpn;
     double* g_lin;
     double* g_cen;
@@ -105,9 +107,11 @@ struct EriArgs {
 template <int LA, int LB, int LC, int LD, typename R, int MODE>
 void launch_eri(const EriArgs& a, hipStream_t s);
 
-// Gradient kernels (classes whose shells are all s or p), generated units eri_<class>_grad.hip.
+// Gradient kernels (classes whose shells are all s or p), generated units
+// eri_<class>_grad.hip: group g of a class goes to stream s[g % ns].
 template <int LA, int LB, int LC, int LD>
-void launch_eri_grad(const EriArgs& a, hipStream_t s);
+void launch_eri_grad(const EriArgs& a, hipStream_t* s, int ns);
+typedef void (*EriGradLaunch)(const EriArgs&, hipStream_t*, int);
 
 typedef void (*EriLaunch)(const EriArgs&, hipStream_t);
 
