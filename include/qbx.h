@@ -304,17 +304,30 @@ int  qbx_gemm_f64(int32_t trans_a, int32_t trans_b, int32_t M, int32_t N, int32_
 int  qbx_gemm_bf16(int32_t trans_a, int32_t trans_b, int32_t M, int32_t N, int32_t K, float alpha,
                    const void* A, int32_t lda, const void* B, int32_t ldb, float beta, float* C, int32_t ldc,
                    int32_t epilogue, const float* bias, void* Cb, void* stream);
+/* One backward step through a ReLU layer: C (FP32) and Cb (BF16) = A B^T where
+   the layer's BF16 activations H are positive, else 0 (A: M x K, B: N x K; H,
+   C and Cb: M x N, row stride ldc). */
+int  qbx_gemm_bf16_relu_back(int32_t M, int32_t N, int32_t K, const void* A, int32_t lda, const void* B,
+                             int32_t ldb, const void* H, float* C, void* Cb, int32_t ldc, void* stream);
 /* op 0: out0 (BF16) = x (FP32) converted; op 1: ReLU backward, out1 (FP32) and
    out0 (BF16) = x (FP32 dH) where y (BF16 H) > 0, else 0. */
 int  qbx_mlp_elementwise(int32_t op, int64_t n, const void* x, const void* y, void* out0, void* out1, void* stream);
 /* weighted squared error: loss += sum w_r m_c (Y - T)^2 scale, dY = 2 w_r m_c (Y - T) scale (FP32 and BF16) */
 int  qbx_mlp_mse(int32_t rows, int32_t cols, const float* Y, const float* T, const float* row_w,
                  const float* col_mask, float scale, float* dY, void* dYb, float* loss, void* stream);
+/* the same with scale = 1 / max(sum_r w_r, 1), summed on the device */
+int  qbx_mlp_mse_mean(int32_t rows, int32_t cols, const float* Y, const float* T, const float* row_w,
+                      const float* col_mask, float* dY, void* dYb, float* loss, void* stream);
 /* out[c] = sum_r X[r][c] */
 int  qbx_mlp_colsum(int32_t rows, int32_t cols, const float* X, float* out, void* stream);
 /* Adam step `step` (1-based) on FP32 weights w with moments m, v and gradient g; BF16 copy to wb if non-NULL */
 int  qbx_mlp_adam(int64_t n, float* w, float* m, float* v, const float* g, void* wb, float lr, float b1, float b2,
                   float eps, int32_t step, void* stream);
+/* The same step on `count` (1..16) tensors in one launch; the arrays (host memory)
+   hold each tensor's length and device pointers, wb[t] may be NULL. */
+int  qbx_mlp_adam_multi(int32_t count, const int64_t* n, float* const* w, float* const* m, float* const* v,
+                        const float* const* g, void* const* wb, float lr, float b1, float b2, float eps,
+                        int32_t step, void* stream);
 
 /* Last error message of the calling thread; returns its full length. */
 int  qbx_last_error(char* buf, size_t len);

@@ -70,6 +70,11 @@ SIGNATURES = {
     "qbx_mlp_colsum": (_i32, [_i32, _i32, _vp, _vp, _vp]),
     "qbx_mlp_adam": (_i32, [_i64, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                             ctypes.c_float, _i32, _vp]),
+    "qbx_gemm_bf16_relu_back": (_i32, [_i32, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i32, _vp]),
+    "qbx_mlp_mse_mean": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "qbx_mlp_adam_multi": (_i32, [_i32, _pl, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp),
+                                  ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.c_float, ctypes.c_float,
+                                  ctypes.c_float, ctypes.c_float, _i32, _vp]),
     "qbx_last_error": (_i32, [ctypes.c_char_p, ctypes.c_size_t]),
 }
 

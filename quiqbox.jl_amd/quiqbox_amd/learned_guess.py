@@ -247,23 +247,23 @@ class LearnedGuess:
         L = _lib.load()
         d = self.dev
         y, acts_b = self._forward(xb, n, keep=True)
-        nreal = float(rw.sum().item())
         dY = torch.empty_like(y)
         dYb = torch.empty((n, self.layout.n_out), dtype=torch.bfloat16, device="cuda")
         loss = torch.zeros(1, dtype=torch.float32, device="cuda")
         cmask = getattr(self, "_cmask", None)
         if cmask is None:
             cmask = self._cmask = torch.ones(self.layout.n_out, dtype=torch.float32, device="cuda")
-        _lib.check(L.qbx_mlp_mse(n, self.layout.n_out, _p(y), _p(yt), _p(rw), _p(cmask), 1.0 / max(nreal, 1.0), _p(dY), _p(dYb),
-                                 _p(loss), None))
+        _lib.check(L.qbx_mlp_mse_mean(n, self.layout.n_out, _p(y), _p(yt), _p(rw), _p(cmask), _p(dY), _p(dYb),
+                                      _p(loss), None))
         grads = self.backward(acts_b, dY, dYb, n)
         self.step += 1
-        for li in range(len(self.sizes)):
-            gW, gb = grads[li]
-            _lib.check(L.qbx_mlp_adam(d.W[li].numel(), _p(d.W[li]), _p(d.mW[li]), _p(d.vW[li]), _p(gW), _p(d.Wb[li]),
-                                      lr, 0.9, 0.999, 1e-8, self.step, None))
-            _lib.check(L.qbx_mlp_adam(d.b[li].numel(), _p(d.b[li]), _p(d.mb[li]), _p(d.vb[li]), _p(gb), None,
-                                      lr, 0.9, 0.999, 1e-8, self.step, None))
+        tensors = [(d.W[l], d.mW[l], d.vW[l], grads[l][0], d.Wb[l]) for l in range(len(self.sizes))]
+        tensors += [(d.b[l], d.mb[l], d.vb[l], grads[l][1], None) for l in range(len(self.sizes))]
+        k = len(tensors)
+        ptrs = [(ctypes.c_void_p * k)(*[None if t[c] is None else t[c].data_ptr() for t in tensors])
+                for c in range(5)]
+        _lib.check(L.qbx_mlp_adam_multi(k, (ctypes.c_int64 * k)(*[t[0].numel() for t in tensors]), *ptrs,
+                                        lr, 0.9, 0.999, 1e-8, self.step, None))
         return loss
 
     def backward(self, acts_b, dY, dYb, n):
@@ -285,13 +285,11 @@ class LearnedGuess:
             _lib.check(L.qbx_mlp_colsum(n, fo, _p(g_f), _p(gbias), None))
             grads[li] = (gW, gbias)
             if li > 0:
-                # dh = g W^T, then through the ReLU of the layer below
-                dh = torch.empty((n, fi), dtype=torch.float32, device="cuda")
-                _lib.check(L.qbx_gemm_bf16(0, 1, n, fi, fo, 1.0, _p(g_b), fo, _p(d.Wb[li]), fo, 0.0, _p(dh), fi, 0,
-                                           None, None, None))
-                nf = torch.empty_like(dh)
+                # dh = g W^T through the ReLU of the layer below
+                nf = torch.empty((n, fi), dtype=torch.float32, device="cuda")
                 nb = torch.empty((n, fi), dtype=torch.bfloat16, device="cuda")
-                _lib.check(L.qbx_mlp_elementwise(1, n * fi, _p(dh), _p(acts_b[li]), _p(nb), _p(nf), None))
+                _lib.check(L.qbx_gemm_bf16_relu_back(n, fi, fo, _p(g_b), fo, _p(d.Wb[li]), fo, _p(acts_b[li]),
+                                                     _p(nf), _p(nb), fi, None))
                 g_f, g_b = nf, nb
         return grads
 
