@@ -105,12 +105,15 @@ constexpr double QBX_PRIM_PAIR_CUT = 1e-20;
 // lanes busy 36% -> 78% of the primitive loop, 3.5% more waves.
 constexpr int kKetBuckets = 5;
 
-// Fixed device work array of qbx_density_purify_noalloc: P, Q, T (n x n) and
-// 2n + 4 auxiliary values for n up to QBX_PURIFY_NOALLOC_MAX_N, 25 MB per
-// GPU for the life of the process.  Host code never uses the symbol itself as
+// Fixed device work array of qbx_density_purify_noalloc: P, Q, T (n x n, padded to
+// a multiple of 32) and the auxiliary values (row intervals, state, shares of 32 x
+// 32 tiles) for n up to QBX_PURIFY_NOALLOC_MAX_N, 25 MB per GPU for the life of
+// the process.  Host code never uses the symbol itself as
 // an address: qbx_init takes each device's address with hipGetSymbolAddress.
 constexpr size_t kPurifyScratch = 3 * (size_t)QBX_PURIFY_NOALLOC_MAX_N * QBX_PURIFY_NOALLOC_MAX_N +
-                                  2 * (size_t)QBX_PURIFY_NOALLOC_MAX_N + 4;
+                                  2 * (size_t)QBX_PURIFY_NOALLOC_MAX_N + 16 +
+                                  2 * (size_t)(QBX_PURIFY_NOALLOC_MAX_N / 32) * (QBX_PURIFY_NOALLOC_MAX_N / 32 + 1);
+static_assert(QBX_PURIFY_NOALLOC_MAX_N % 32 == 0, "the padded size of the largest matrix");
 static __device__ __align__(256) double scratch[kPurifyScratch];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -1565,10 +1568,20 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
     }
 }
 
-// Work matrices of the purification: P, Q, T (n x n each) and aux (2n + 4).
+// Work matrices of the purification: P, Q, T (sp2_padded(n)^2 each) and aux
+// (purify_aux(n)).
 struct PurifyWork {
     double *P, *Q, *T, *aux;
 };
+
+// row intervals, spectral interval, status, state, shares
+constexpr size_t kPurifyHead = 2 + sizeof(Sp2Status) / sizeof(double) + 2 * sizeof(Sp2State) / sizeof(double);
+size_t purify_aux(int n) { return 2 * (size_t)n + kPurifyHead + 4 * (size_t)sp2_blocks(n); }
+
+// Products queued between two looks at the state: the kernels decide on the device
+// and do nothing once the projector has settled, so a batch costs one
+// synchronization and at most its empty launches (4.5 us each).
+constexpr int kPurifyBatch = 12;
 
 // D = C[:, :nocc] C[:, :nocc]^T of eigen(X' F X) by trace-correcting
 // purification (device X and F, n x n row-major) on stream st, using only the
@@ -1577,55 +1590,42 @@ struct PurifyWork {
 const double* purify_density(int n, int nocc, const double* dX, const double* dF, const PurifyWork& w, int max_iter,
                              int32_t* iterations, double* idempotency, hipStream_t st)
 {
-    double* dP = w.P;
-    double* dQ = w.Q;
-    double* dT = w.T;
-    // Fock matrix in the orthonormal basis: Fo = X' F X (into dQ)
-    gemm_f64(false, false, n, n, n, 1.0, dF, n, dX, n, 0.0, nullptr, 0, dT, n, st);
-    gemm_f64(true, false, n, n, n, 1.0, dX, n, dT, n, 0.0, nullptr, 0, dQ, n, st);
-    // spectral interval from Gershgorin discs
-    double lohi[2];
-    gershgorin(dQ, n, w.aux, st);
-    spectral_interval(w.aux, n, w.aux + 2 * (size_t)n, st);
-    QBX_HIP(hipMemcpyAsync(lohi, w.aux + 2 * (size_t)n, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-    QBX_HIP(hipStreamSynchronize(st));
-    double lo = lohi[0], hi = lohi[1];
-    if (!(hi > lo)) hi = lo + 1.0;
-    sp2_start(dQ, n, lo, hi, dP, st);
+    static_assert(sizeof(Sp2Status) % sizeof(double) == 0 && sizeof(Sp2State) % sizeof(double) == 0, "aux layout");
+    double* rows = w.aux;
+    double* lohi = rows + 2 * (size_t)n;
+    Sp2Status* status = (Sp2Status*)(lohi + 2);
+    Sp2State* state = (Sp2State*)(status + 1);
+    double* shares = (double*)(state + 2);
+    // Fock matrix in the orthonormal basis: Fo = X' F X (into Q), its spectral
+    // interval from Gershgorin discs, P = (hi - Fo) / (hi - lo)
+    gemm_f64(false, false, n, n, n, 1.0, dF, n, dX, n, 0.0, nullptr, 0, w.T, n, st);
+    gemm_f64(true, false, n, n, n, 1.0, dX, n, w.T, n, 0.0, nullptr, 0, w.Q, n, st);
+    gershgorin(w.Q, n, rows, st);
+    spectral_interval(rows, n, lohi, st);
+    sp2_start(w.Q, n, lohi, w.P, shares, state, st);
     // trace-correcting purification (SP2): P <- P^2 or 2P - P^2, whichever
     // moves trace(P) toward nocc; quadratic convergence to the projector
     // on the nocc lowest eigenvectors once the trace is right
-    double tf[2];
-    double* dtf = w.aux + 2 * (size_t)n + 2;
-    auto measure = [&] {
-        trace_and_frobenius(dP, n, dtf, st);
-        QBX_HIP(hipMemcpyAsync(tf, dtf, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
+    double* buf[2] = {w.P, w.Q};
+    Sp2Status h;
+    int k = 0;
+    do {
+        for (int e = std::min(max_iter, k + kPurifyBatch); k < e; ++k)
+            sp2_product(buf[k & 1], buf[(k + 1) & 1], n, nocc, k, shares, state, st);
+        sp2_status(shares, n, k, state, status, st);
+        QBX_HIP(hipMemcpyAsync(&h, status, sizeof(h), hipMemcpyDeviceToHost, st));
         QBX_HIP(hipStreamSynchronize(st));
-    };
-    measure();
-    int it = 0, tail = -1;
-    const double N = (double)nocc;
-    for (; it < max_iter; ++it) {
-        const double tr = tf[0], fr = tf[1];
-        const double err = std::fabs(tr - fr);
-        if (tail < 0 && err < 1e-8 * std::max(1.0, N) && std::fabs(tr - N) < 1e-6) tail = 2;
-        if (tail == 0) break;
-        if (tail > 0) --tail;
-        if (std::fabs(fr - N) <= std::fabs(2.0 * tr - fr - N))
-            gemm_f64(false, false, n, n, n, 1.0, dP, n, dP, n, 0.0, nullptr, 0, dQ, n, st);
-        else
-            gemm_f64(false, false, n, n, n, -1.0, dP, n, dP, n, 2.0, dP, n, dQ, n, st);
-        std::swap(dP, dQ);
-        measure();
-    }
-    if (iterations) *iterations = it;
-    if (idempotency) *idempotency = std::fabs(tf[0] - tf[1]);
-    if (tail != 0 || !(std::fabs(tf[0] - N) < 1e-6))
+    } while (!h.s.stop && k < max_iter);
+    if (iterations) *iterations = h.s.it;
+    if (idempotency) *idempotency = std::fabs(h.tr - h.fr);
+    if (h.s.tail != 0 || !(std::fabs(h.tr - (double)nocc) < 1e-6))
         throw QbxError(QBX_ENOCONV, "purification did not converge (no gap at the Fermi level, or max_iter too small)");
     // D = X P X'
-    gemm_f64(false, false, n, n, n, 1.0, dX, n, dP, n, 0.0, nullptr, 0, dT, n, st);
-    gemm_f64(false, true, n, n, n, 1.0, dT, n, dX, n, 0.0, nullptr, 0, dQ, n, st);
-    return dQ;
+    const double* P = buf[h.s.it & 1];
+    double* D = buf[(h.s.it + 1) & 1];
+    gemm_f64(false, false, n, n, n, 1.0, dX, n, P, sp2_padded(n), 0.0, nullptr, 0, w.T, n, st);
+    gemm_f64(false, true, n, n, n, 1.0, w.T, n, dX, n, 0.0, nullptr, 0, D, n, st);
+    return D;
 }
 
 }  // namespace
@@ -2123,10 +2123,11 @@ int qbx_density_purify(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, c
         const size_t nn = (size_t)n * n;
         ctx->la_X.ensure(nn);
         ctx->la_F.ensure(nn);
-        ctx->la_P.ensure(nn);
-        ctx->la_Q.ensure(nn);
-        ctx->la_T.ensure(nn);
-        ctx->la_aux.ensure(2 * (size_t)n + 4);
+        const size_t pp = (size_t)sp2_padded(n) * sp2_padded(n);
+        ctx->la_P.ensure(pp);
+        ctx->la_Q.ensure(pp);
+        ctx->la_T.ensure(pp);
+        ctx->la_aux.ensure(purify_aux(n));
         QBX_HIP(hipMemcpyAsync(ctx->la_X.p, X, nn * sizeof(double), hipMemcpyHostToDevice, st));
         QBX_HIP(hipMemcpyAsync(ctx->la_F.p, F, nn * sizeof(double), hipMemcpyHostToDevice, st));
         const PurifyWork w{ctx->la_P.p, ctx->la_Q.p, ctx->la_T.p, ctx->la_aux.p};
@@ -2154,9 +2155,10 @@ int qbx_density_purify_noalloc(qbx_ctx* ctx, int32_t n, int32_t nocc, const doub
         hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
         // the work matrices in the library's fixed device array (its address on
         // this device, taken at qbx_init); every entry is written before it is read
-        const size_t nn = (size_t)n * n;
+        const size_t nn = (size_t)n * n, pp = (size_t)sp2_padded(n) * sp2_padded(n);
+        if (3 * pp + purify_aux(n) > kPurifyScratch) throw QbxError(QBX_EINTERNAL, "the fixed work array is too small");
         double* base = ctx->scratch;
-        const PurifyWork w{base, base + nn, base + 2 * nn, base + 3 * nn};
+        const PurifyWork w{base, base + pp, base + 2 * pp, base + 3 * pp};
         const double* dOut = purify_density(n, nocc, dX, dF, w, max_iter, iterations, idempotency, st);
         QBX_HIP(hipMemcpyAsync(dD, dOut, nn * sizeof(double), hipMemcpyDeviceToDevice, st));
         QBX_HIP(hipStreamSynchronize(st));

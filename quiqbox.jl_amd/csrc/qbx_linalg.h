@@ -28,11 +28,32 @@ void fix_column_signs(double* C, int n, double* sgn, hipStream_t s);
 // out[0] = min of lohi[2i], out[1] = max of lohi[2i+1] over the n rows
 void spectral_interval(const double* lohi, int n, double* out, hipStream_t s);
 
-// P = (hi I - F) / (hi - lo)
-void sp2_start(const double* F, int n, double lo, double hi, double* P, hipStream_t s);
+// Trace-correcting purification on the device.  Matrices are symmetric,
+// sp2_padded(n) square with zero rows and columns beyond n; `shares` holds 2 x 2 x
+// sp2_blocks(n) doubles, `state` two entries.
+struct Sp2State {
+    int tail;   // products still to make once the projector has settled, -1: not settled
+    int stop;   // no product any more
+    int it;     // products made
+    int pad;
+};
+struct Sp2Status {
+    Sp2State s;
+    double tr, fr;   // tr P and |P|_F^2 of the latest matrix
+};
+int sp2_padded(int n);
+int sp2_blocks(int n);
 
-// out[0] = trace(P), out[1] = sum_ij P_ij^2 (= trace(P^2) for symmetric P);
-// one block, fixed summation order
-void trace_and_frobenius(const double* P, int n, double* out, hipStream_t s);
+// P = (hi I - F) / (hi - lo), F's symmetric part (n x n, row stride n), [lo, hi] =
+// lohi (hi = lo + 1 where the interval is empty); state[0] and shares of P
+void sp2_start(const double* F, int n, const double* lohi, double* P, double* shares, Sp2State* state, hipStream_t s);
+
+// Product k (0, 1, ...): Q = P^2 or 2P - P^2, whichever moves tr P toward nocc, or
+// nothing after the projector has settled.  Matrix k is in the first buffer for
+// even k, in the second for odd k.
+void sp2_product(const double* P, double* Q, int n, int nocc, int k, double* shares, Sp2State* state, hipStream_t s);
+
+// state and measures after k launches of sp2_product
+void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2Status* out, hipStream_t s);
 
 }  // namespace qbx
