@@ -249,15 +249,14 @@ struct qbx_basis {
     // shell quartets with a shell above the generated classes (f, g): the
     // generic kernel's bra and ket lists at the threshold `thr`
     bool has_high = false;
-    int nm = 0;                     // its recurrence size, 4 x the highest L
-    DevBuf<double> d_pexp;
+    struct HighSet {                // one pair of pair classes
+        int X, Y;
+        int64_t first, total;       // its prefix within `prefix`, its quartets
+    };
     struct HighLists {
         bool valid = false;
         double thr = -1.0;
-        int nbra = 0;
-        int64_t total = 0;
-        DevBuf<int> hA, hB, ho, hn, lA, lB, lo, ln, nlow;
-        DevBuf<double> hQ, lQ;
+        std::vector<HighSet> sets;  // largest estimated work first
         DevBuf<int64_t> prefix;
     } hl;
     ~qbx_basis()
@@ -768,15 +767,26 @@ void find_twins(qbx_basis* b)
 
 bool high_class(int c) { return qbx_pair_class_l[c][0] > QBX_GEN_LMAX; }
 
-GenArgs gen_base(const qbx_basis* b)
+// The pairs of a class in plain Schwarz order.
+const PairClass& plain_class(const qbx_basis* b, int c) { return b->pc[c].plain ? *b->pc[c].plain : b->pc[c]; }
+
+GenArgs gen_base(const qbx_basis* b, int X, int Y)
 {
     GenArgs g;
     std::memset(&g, 0, sizeof(g));
+    const PairClass& PX = plain_class(b, X);
+    g.bra = pcdev(PX);
+    g.ket = pcdev(plain_class(b, Y));
+    for (int t = 0; t < 2; ++t) {
+        g.l[t] = qbx_pair_class_l[X][t];
+        g.l[2 + t] = qbx_pair_class_l[Y][t];
+    }
+    for (int n : PX.ppn) g.bn_max = std::max(g.bn_max, n);
+    for (int n : plain_class(b, Y).ppn) g.kn_max = std::max(g.kn_max, n);
+    g.same = X == Y;
+    g.nbra = PX.n();
     g.sh = b->d_sh.p;
     g.pp = b->d_pp.p;
-    g.ppk = b->d_ppk.p;
-    g.poff = b->d_poff.p;
-    g.pexp = b->d_pexp.p;
     g.boys = b->ctx->boys.p;
     g.bexp = b->ctx->bexp.p;
     g.N = b->nbf;
@@ -785,38 +795,20 @@ GenArgs gen_base(const qbx_basis* b)
 
 // Schwarz bounds of the pairs of a pair class above the generated classes:
 // max |(ab|ab)| over the pair's components from the generic kernel, in the
-// class's current order.
-std::vector<double> high_class_schwarz(qbx_basis* b, int c, hipStream_t st)
+// class's current order (q: one value per pair, 0 where no primitive pair is left).
+void high_class_schwarz(qbx_basis* b, int c, DevBuf<double>& q, DevBuf<int64_t>& pre, hipStream_t st)
 {
-    PairClass& P = b->pc[c];
-    const int n = P.n();
-    DevBuf<int64_t> pre;
-    DevBuf<unsigned long long> bits;
+    const int n = b->pc[c].n();
     std::vector<int64_t> h(n + 1);
     std::iota(h.begin(), h.end(), (int64_t)0);
     pre.upload(h, st);
-    bits.ensure(n);
-    QBX_HIP(hipMemsetAsync(bits.p, 0, n * sizeof(unsigned long long), st));
-    GenArgs g = gen_base(b);
-    g.nbra = n;
+    q.ensure(n);
+    zero_async(q.p, n, st);
+    GenArgs g = gen_base(b, c, c);
     g.total = n;
     g.prefix = pre.p;
-    g.hA = P.d_shA.p;
-    g.hB = P.d_shB.p;
-    g.ho = P.d_ppo.p;
-    g.hn = P.d_ppn.p;
-    g.qbits = bits.p;
-    launch_eri_generic(g, 2 * (qbx_pair_class_l[c][0] + qbx_pair_class_l[c][1]), MODE_SCHWARZ, st);
-    std::vector<unsigned long long> hb(n);
-    QBX_HIP(hipMemcpyAsync(hb.data(), bits.p, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    QBX_HIP(hipStreamSynchronize(st));
-    std::vector<double> Q(n);
-    for (int i = 0; i < n; ++i) {
-        double v;
-        std::memcpy(&v, &hb[i], sizeof(double));
-        Q[i] = std::sqrt(v);
-    }
-    return Q;
+    g.qout = q.p;
+    launch_eri_generic(g, MODE_SCHWARZ, st);
 }
 
 void ensure_schwarz(qbx_basis* b)
@@ -824,12 +816,12 @@ void ensure_schwarz(qbx_basis* b)
     if (b->schwarz) return;
     hipStream_t st = b->ctx->stream;
     std::vector<DevBuf<double>> q(QBX_N_PAIR_CLASSES);
-    std::vector<std::vector<double>> qhigh(QBX_N_PAIR_CLASSES);
+    std::vector<DevBuf<int64_t>> qpre(QBX_N_PAIR_CLASSES);
     for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
         PairClass& P = b->pc[c];
         if (P.n() == 0) continue;
         if (high_class(c)) {
-            qhigh[c] = high_class_schwarz(b, c, st);
+            high_class_schwarz(b, c, q[c], qpre[c], st);
             continue;
         }
         q[c].ensure(P.n());
@@ -861,12 +853,8 @@ void ensure_schwarz(qbx_basis* b)
             continue;
         }
         std::vector<double> Q(n);
-        if (high_class(c)) {
-            Q = qhigh[c];
-        } else {
-            QBX_HIP(hipMemcpyAsync(Q.data(), q[c].p, n * sizeof(double), hipMemcpyDeviceToHost, st));
-            QBX_HIP(hipStreamSynchronize(st));
-        }
+        QBX_HIP(hipMemcpyAsync(Q.data(), q[c].p, n * sizeof(double), hipMemcpyDeviceToHost, st));
+        QBX_HIP(hipStreamSynchronize(st));
         std::vector<int> perm(n);
         std::iota(perm.begin(), perm.end(), 0);
         std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return Q[x] > Q[y]; });
@@ -1170,95 +1158,69 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
     b->task_cut = cut;
 }
 
-// Quartet lists of the generic kernel at threshold thr: bras are the pairs of
-// the classes above the generated ones in descending Schwarz order; bra i
-// takes every lower pair with Q_i Q_j >= thr, then the higher pairs j <= i
-// with Q_i Q_j >= thr (each higher-higher quartet once).
+// Quartet lists of the generic kernel at threshold thr: for every pair class X
+// above the generated ones and every class Y up to it, bra i of X takes the kets j
+// of Y with Q_i Q_j >= thr (j up to i within one class, so that each quartet
+// appears once).
 void ensure_hl_tasks(qbx_basis* b, double thr)
 {
     if (!b->has_high) return;
     auto& H = b->hl;
     if (H.valid && H.thr == thr) return;
     if (b->built) QBX_HIP(hipEventSynchronize(b->ev_done));
-    struct Pr {
-        int A, B, o, n;
-        double Q;
-    };
-    std::vector<Pr> hi, lo;
-    for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
-        const PairClass& P = b->pc[c];
-        auto& dst = high_class(c) ? hi : lo;
-        for (int i = 0; i < P.n(); ++i) dst.push_back({P.shA[i], P.shB[i], P.ppo[i], P.ppn[i], P.Q[i]});
-    }
-    auto byQ = [](const Pr& x, const Pr& y) { return x.Q > y.Q; };
-    std::stable_sort(hi.begin(), hi.end(), byQ);
-    std::stable_sort(lo.begin(), lo.end(), byQ);
-    std::vector<double> hq(hi.size()), lq(lo.size());
-    for (size_t i = 0; i < hi.size(); ++i) hq[i] = hi[i].Q;
-    for (size_t i = 0; i < lo.size(); ++i) lq[i] = lo[i].Q;
-    const int nb = (int)hi.size();
-    std::vector<int64_t> pre(nb + 1, 0);
-    std::vector<int> nlow(nb);
-    for (int i = 0; i < nb; ++i) {
-        int nl, nh;
-        if (thr <= 0.0) {
-            nl = (int)lo.size();
-            nh = i + 1;
-        } else if (hq[i] > 0.0) {
-            nl = count_ge(lq, thr / hq[i]);
-            nh = std::min(i + 1, count_ge(hq, thr / hq[i]));
-        } else {
-            nl = nh = 0;
+    H.valid = false;
+    H.sets.clear();
+    std::vector<int64_t> pre;
+    std::vector<double> cost;
+    for (int X = 0; X < QBX_N_PAIR_CLASSES; ++X) {
+        if (!high_class(X)) continue;
+        for (int Y = 0; Y <= X; ++Y) {
+            const PairClass& PX = plain_class(b, X);
+            const PairClass& PY = plain_class(b, Y);
+            if (PX.n() == 0 || PY.n() == 0) continue;
+            qbx_basis::HighSet S{X, Y, (int64_t)pre.size(), 0};
+            pre.push_back(0);
+            for (int i = 0; i < PX.n(); ++i) {
+                int nk = thr <= 0.0 ? PY.n() : PX.Q[i] > 0.0 ? count_ge(PY.Q, thr / PX.Q[i]) : 0;
+                if (X == Y) nk = std::min(nk, i + 1);
+                S.total += nk;
+                pre.push_back(S.total);
+            }
+            if (S.total > 0) H.sets.push_back(S);
+            else pre.resize(S.first);
         }
-        nlow[i] = nl;
-        pre[i + 1] = pre[i] + nl + nh;
     }
-    hipStream_t st = b->ctx->stream;
-    auto up = [&](const std::vector<Pr>& v, DevBuf<int>& A, DevBuf<int>& B, DevBuf<int>& o, DevBuf<int>& n,
-                  DevBuf<double>& Q, const std::vector<double>& q) {
-        std::vector<int> a(v.size()), bb(v.size()), oo(v.size()), nn(v.size());
-        for (size_t i = 0; i < v.size(); ++i) {
-            a[i] = v[i].A;
-            bb[i] = v[i].B;
-            oo[i] = v[i].o;
-            nn[i] = v[i].n;
-        }
-        A.upload(a, st);
-        B.upload(bb, st);
-        o.upload(oo, st);
-        n.upload(nn, st);
-        Q.upload(q, st);
-    };
-    up(hi, H.hA, H.hB, H.ho, H.hn, H.hQ, hq);
-    up(lo, H.lA, H.lB, H.lo, H.ln, H.lQ, lq);
-    H.nlow.upload(nlow, st);
-    H.prefix.upload(pre, st);
-    QBX_HIP(hipStreamSynchronize(st));
-    H.nbra = nb;
-    H.total = pre[nb];
+    // the launches share the device: largest first, by quartets and Cartesian components
+    std::stable_sort(H.sets.begin(), H.sets.end(), [&](const qbx_basis::HighSet& x, const qbx_basis::HighSet& y) {
+        auto w = [&](const qbx_basis::HighSet& s) {
+            double v = (double)s.total;
+            for (int c : {s.X, s.Y})
+                for (int t = 0; t < 2; ++t) v *= qbx_ncart(qbx_pair_class_l[c][t]);
+            return v;
+        };
+        return w(x) > w(y);
+    });
+    if (!H.sets.empty()) {
+        hipStream_t st = b->ctx->stream;
+        H.prefix.upload(pre, st);
+        QBX_HIP(hipStreamSynchronize(st));
+    }
     H.thr = thr;
     H.valid = true;
 }
 
-GenArgs gen_lists(const qbx_basis* b)
+// The generic kernel over the lists, one launch per pair of pair classes, spread
+// over the `ns` streams; `fill` sets the mode's arguments.
+template <class Fill> void launch_high(const qbx_basis* b, int mode, hipStream_t* s, int ns, Fill fill)
 {
-    GenArgs g = gen_base(b);
-    const auto& H = b->hl;
-    g.nbra = H.nbra;
-    g.total = H.total;
-    g.prefix = H.prefix.p;
-    g.nlow = H.nlow.p;
-    g.hA = H.hA.p;
-    g.hB = H.hB.p;
-    g.ho = H.ho.p;
-    g.hn = H.hn.p;
-    g.hQ = H.hQ.p;
-    g.lA = H.lA.p;
-    g.lB = H.lB.p;
-    g.lo = H.lo.p;
-    g.ln = H.ln.p;
-    g.lQ = H.lQ.p;
-    return g;
+    int k = 0;
+    for (const qbx_basis::HighSet& S : b->hl.sets) {
+        GenArgs g = gen_base(b, S.X, S.Y);
+        g.prefix = b->hl.prefix.p + S.first;
+        g.total = S.total;
+        fill(g);
+        launch_eri_generic(g, mode, s[k++ % ns]);
+    }
 }
 
 // Before a Fock build on stream st touches the basis's work buffers: a
@@ -1512,21 +1474,19 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
         QBX_HIP(hipEventRecord(ctx->ev_fork, st));
         for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
     }
-    // quartets with an f or g shell: the generic kernel (FP64 in every mode),
-    // first on the last auxiliary stream
-    if (b->has_high && b->hl.total > 0) {
-        GenArgs g = gen_lists(b);
-        g.D = dD;
-        g.J = b->d_J.p;
-        g.K = b->d_K.p;
-        g.xcd_local = ctx->xcd_local ? 1 : 0;
-        g.jk_stride = NN * nset;
-        g.nset = nset;
-        g.pdmax = pdmax;
-        g.nshell = ns;
-        g.dthr = ctx->density_thr;
-        launch_eri_generic(g, b->nm, MODE_JK, fork ? ctx->aux[kStreams - 1] : st);
-    }
+    // quartets with an f or g shell: the generic kernel (FP64 in every mode), first
+    if (b->has_high)
+        launch_high(b, MODE_JK, fork ? ctx->aux : &st, fork ? kStreams : 1, [&](GenArgs& g) {
+            g.D = dD;
+            g.J = b->d_J.p;
+            g.K = b->d_K.p;
+            g.xcd_local = ctx->xcd_local ? 1 : 0;
+            g.jk_stride = NN * nset;
+            g.nset = nset;
+            g.pdmax = pdmax;
+            g.nshell = ns;
+            g.dthr = ctx->density_thr;
+        });
     std::vector<int> order(QBX_N_CLASSES);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
@@ -1915,9 +1875,7 @@ int qbx_basis_create(qbx_ctx* ctx, int32_t n_prim, const double* prim_cen, const
             }
         }
         b->d_sh.upload(ds, st);
-        b->d_pexp.upload(b->pexp, st);
         b->has_high = b->maxL > QBX_GEN_LMAX;
-        b->nm = 4 * b->maxL;
         b->d_pp.upload(b->pp, st);
         b->d_ppk.upload(b->ppk, st);
         std::vector<int> poff(ns);
@@ -2026,13 +1984,17 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
         d.ensure(N4);
         zero_async(d.p, N4, st);
         // each class's task lists (host and device) stay alive until the one
-        // synchronization below, so the classes' kernels queue back to back
+        // synchronization below; the classes write disjoint elements and run
+        // concurrently on the auxiliary streams
         struct DenseTasks {
             TaskCounts tc;
             DevBuf<int64_t> pre;
             DevBuf<int> ko, cw;
         };
         std::vector<std::unique_ptr<DenseTasks>> lists;
+        std::vector<EriArgs> args(QBX_N_CLASSES);
+        std::vector<int> order;
+        double cost[QBX_N_CLASSES] = {};
         for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
             auto L = std::make_unique<DenseTasks>();
             TaskCounts& tc = L->tc;
@@ -2042,23 +2004,29 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
             L->pre.upload(tc.p64, st);
             L->ko.upload(tc.k64, st);
             L->cw.upload(tc.w64, st);
-            EriArgs a = base_args(b, cls);
+            EriArgs& a = args[cls] = base_args(b, cls);
             a.prefix = L->pre.p;
             a.koff = L->ko.p;
             a.cpre = L->cw.p;
             a.total = tc.p64[nt];
             a.nwave = tc.w64[nt];
             a.nbra = nt;
+            a.scratch_stream = (void*)st;
             attach_workspace(b, cls, a.nwave, a);
             a.eri = d.p;
-            k_dense[cls](a, st);
+            cost[cls] = class_cost(b, cls, tc);
+            order.push_back(cls);
             lists.push_back(std::move(L));
         }
-        if (b->has_high) {
-            ensure_hl_tasks(b, 0.0);
-            GenArgs g = gen_lists(b);
-            g.eri = d.p;
-            launch_eri_generic(g, b->nm, MODE_DENSE, st);
+        ensure_hl_tasks(b, 0.0);
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+        QBX_HIP(hipEventRecord(ctx->ev_fork, st));
+        for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
+        for (size_t k = 0; k < order.size(); ++k) k_dense[order[k]](args[order[k]], ctx->aux[k % kStreams]);
+        if (b->has_high) launch_high(b, MODE_DENSE, ctx->aux, kStreams, [&](GenArgs& g) { g.eri = d.p; });
+        for (int k = 0; k < kStreams; ++k) {
+            QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
+            QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
         }
         QBX_HIP(hipMemcpyAsync(eri, d.p, N4 * sizeof(double), hipMemcpyDeviceToHost, st));
         QBX_HIP(hipStreamSynchronize(st));

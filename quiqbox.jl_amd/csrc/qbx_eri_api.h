@@ -116,27 +116,23 @@ typedef void (*EriGradLaunch)(const EriArgs&, hipStream_t*, int);
 typedef void (*EriLaunch)(const EriArgs&, hipStream_t);
 
 // Shell quartets with a shell above the generated classes (f and g): the
-// generic kernel of qbx_eri_generic.hip.  Bras are the pairs of the higher
-// pair classes in descending Schwarz order; the kets of bra i are the first
-// nlow[i] of the lower pairs (descending Schwarz order) followed by the first
-// prefix[i+1] - prefix[i] - nlow[i] higher pairs (those up to bra i itself).
-// One wave per quartet, lanes over its Cartesian component quartets.
+// generic kernel of qbx_eri_generic.hip, one launch per pair of pair classes
+// (bra (l0 l1), ket (l2 l3)).  Both classes are in descending Schwarz order; the
+// kets of bra i are the first prefix[i + 1] - prefix[i] of the ket class.  One
+// block per shell quartet.
 struct GenArgs {
+    PairClassDev bra, ket;
     const DevShell* sh;
     const PrimPair* pp;
-    const int* ppk;           // radial indices (k_a | k_b << 16) of every primitive pair
-    const int* poff;          // first radial primitive of every shell
-    const double* pexp;       // radial exponents
     const double* boys;       // one-electron Boys table (F_0..F_32 on the 0.1 grid)
     const double* bexp;
+    int l[4];
+    int bn_max, kn_max;       // largest primitive-pair counts of the two classes
+    int ub, cdc;              // bra primitive pairs and ket components held at a time (set by the launcher)
     int nbra;
-    int64_t total;            // quartets (waves)
+    int same;                 // bra and ket are one class
+    int64_t total;            // quartets (blocks)
     const int64_t* prefix;    // [nbra + 1]
-    const int* nlow;          // [nbra]
-    const int *hA, *hB, *ho, *hn;  // higher pairs: shells, primitive-pair offset and count
-    const double* hQ;
-    const int *lA, *lB, *lo, *ln;  // lower pairs
-    const double* lQ;
     int N;
     // J/K mode (as EriArgs)
     const double* D;
@@ -150,14 +146,12 @@ struct GenArgs {
     double dthr;
     // dense mode
     double* eri;
-    // Schwarz mode: every bra with itself, max |(ab|ab)| as the bits of a
-    // non-negative double
-    unsigned long long* qbits;
+    // Schwarz mode: every bra with itself, sqrt(max |(ab|ab)|)
+    double* qout;
 };
 
-// nm: the per-axis recurrence size (4 x the highest shell angular momentum
-// of the quartets, 12 or 16); mode: MODE_JK, MODE_DENSE or MODE_SCHWARZ
-void launch_eri_generic(const GenArgs& a, int nm, int mode, hipStream_t s);
+// mode: MODE_JK, MODE_DENSE or MODE_SCHWARZ
+void launch_eri_generic(const GenArgs& a, int mode, hipStream_t s);
 
 // Primitive-quartet ERIs with unit coefficients (qbx_eri_generic.hip), one
 // thread each: cen [n][4][3], xpn [n][4], ang [n][4][3] (order a, b, c, d of
