@@ -281,7 +281,7 @@ long double boys_seq_ld(long double T, int mtop, long double* F)
     for (int k = 1; k < 20000; ++k) {
         term *= 2.0L * T / (2 * mtop + 2 * k + 1);
         sum += term;
-        if (term < sum * 1e-21L) break;
+        if (fabsl(term) < fabsl(sum) * 1e-21L) break;
     }
     F[mtop] = e * sum;
     for (int m = mtop - 1; m >= 0; --m) F[m] = (2.0L * T * F[m + 1] + e) / (2 * m + 1);
@@ -290,7 +290,7 @@ long double boys_seq_ld(long double T, int mtop, long double* F)
 
 void build_boys_table(std::vector<double>& tab, std::vector<double>& et, std::vector<double>& rows)
 {
-    static_assert(QBX_BOYSL_LMAX + QBX_BOYSL_TAYLOR <= 24, "Boys row orders too high");
+    static_assert(QBX_BOYSL_LMAX < 23, "Boys row orders too high");
     static_assert((QBX_BOYSL_ROWS - 2) * QBX_BOYSL_DT >= QBX_BOYS_TMAX, "Boys rows do not cover the table range");
     tab.assign((size_t)QBX_BOYS_ROWS * QBX_BOYS_NCOL, 0.0);
     et.assign(QBX_BOYS_ROWS, 0.0);
@@ -303,17 +303,39 @@ void build_boys_table(std::vector<double>& tab, std::vector<double>& et, std::ve
         for (int m = 0; m < QBX_BOYS_NCOL; ++m) tab[(size_t)i * QBX_BOYS_NCOL + m] = (double)F[m];
         et[i] = (double)e;
     }
-    // ERI kernels: per-order Taylor rows on the 0.25 grid
+    // ERI kernels: per-order interpolation rows on the 0.25 grid.  f(y) = F_L(T_i - y)
+    // at the Chebyshev nodes x_j = cos((j + 1/2) pi / n) of y = x/8 gives f = sum_k
+    // a_k T_k(x), a_k = (2 - [k = 0])/n sum_j f_j cos(k (j + 1/2) pi / n); the T_k in
+    // monomials (T_k = 2x T_{k-1} - T_{k-2}) and x = 8y give the row.
+    constexpr int n = QBX_BOYSL_NCOEF;
+    const long double pi = acosl(-1.0L), half = QBX_BOYSL_DT / 2;
+    long double mono[n][n] = {};   // T_k in powers of x
+    mono[0][0] = 1.0L;
+    mono[1][1] = 1.0L;
+    for (int k = 2; k < n; ++k)
+        for (int m = 0; m < n; ++m) mono[k][m] = (m > 0 ? 2.0L * mono[k - 1][m - 1] : 0.0L) - mono[k - 2][m];
     for (int i = 0; i < QBX_BOYSL_ROWS; ++i) {
-        const long double e = boys_seq_ld((long double)i * QBX_BOYSL_DT, 23, F);
+        const long double Ti = (long double)i * QBX_BOYSL_DT;
+        long double f[n][QBX_BOYSL_LMAX + 1];
+        for (int j = 0; j < n; ++j) {
+            boys_seq_ld(Ti - half * cosl((j + 0.5L) * pi / n), 23, F);
+            for (int L = 0; L <= QBX_BOYSL_LMAX; ++L) f[j][L] = F[L];
+        }
         for (int L = 0; L <= QBX_BOYSL_LMAX; ++L) {
             double* r = &rows[((size_t)L * QBX_BOYSL_ROWS + i) * QBX_BOYSL_STRIDE];
-            long double fact = 1.0L;
-            for (int k = 0; k < QBX_BOYSL_TAYLOR; ++k) {
-                if (k > 0) fact *= k;
-                r[k] = (double)(F[L + k] / fact);
+            long double c[n] = {};
+            for (int k = 0; k < n; ++k) {
+                long double a = 0.0L;
+                for (int j = 0; j < n; ++j) a += f[j][L] * cosl(k * (j + 0.5L) * pi / n);
+                a *= (k == 0 ? 1.0L : 2.0L) / n;
+                for (int m = 0; m < n; ++m) c[m] += a * mono[k][m];
             }
-            r[QBX_BOYSL_TAYLOR] = (double)e;
+            long double scale = 1.0L;
+            for (int m = 0; m < n; ++m) {
+                r[m] = (double)(c[m] * scale);
+                scale /= half;
+            }
+            r[n] = (double)expl(-Ti);
         }
     }
 }

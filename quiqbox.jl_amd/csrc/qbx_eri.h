@@ -74,61 +74,75 @@ constexpr int boys_rows(int L) { return (int)(kBoysTmax[L] * QBX_BOYSL_INVDT) + 
 static_assert(kBoysTmax[QBX_BOYSL_LMAX] <= QBX_BOYS_TMAX && boys_rows(QBX_BOYSL_LMAX) <= QBX_BOYSL_ROWS,
               "the per-order extent must stay inside the table");
 
-// LDS copy of the Boys table: BOYS_HEAD doubles of constants (1/k! for
-// k = 11..0, the Taylor coefficients of e^x), then the rows; kernels hold
-// sb = table + BOYS_HEAD.  The constants come from LDS rather than from the
-// code: as literals the compiler kept them in VGPRs and copied one into the
-// accumulator before each Horner step of e^x (v_mov_b64 + v_fmac_f64, 22
-// VALU instructions per primitive quartet instead of 11), while a loaded value
-// is consumed in place.
-constexpr int BOYS_HEAD = 12;
-constexpr int BOYS_HEAD2 = BOYS_HEAD / 2;    // the head in double2
+// 1/sqrt(x) for finite x > 0 (p + q of a primitive quartet, Boys arguments above the
+// table): the hardware
+// estimate r refined by the second-order term of the binomial series,
+// 1/sqrt(x) = r (1 - e)^(-1/2) = r (1 + e/2 + 3e^2/8 + ...) with e = 1 - x r^2.
+// The library rsqrt() applies the same correction and then re-checks the
+// estimate for zero, infinite and NaN inputs, which cannot occur here.
+__device__ __forceinline__ double rsqrt_pos(double x)
+{
+    const double r = __builtin_amdgcn_rsq(x);
+    const double e = fma(r * -x, r, 1.0);
+    return fma(r * e, fma(e, 0.375, 0.5), r);
+}
 
-// Boys F_0..F_L from the LDS rows of order L (see qbx_device.h for the table):
-// an 11-term Taylor expansion of F_L about the nearest grid point, e^{-T} from
-// e^{-T_i} times the Taylor series of e^{T_i - T} (|T_i - T| <= 1/8, terms to
-// 11th order), the downward recurrence for the lower orders, and the
-// asymptotic form above the table.
+// LDS copy of the Boys table: BOYS_HEAD doubles of constants (the coefficients of
+// y^9..y^2 of e^y, |y| <= 1/8, interpolated like the rows; those of y and 1 are 1),
+// then the rows; kernels hold sb = table + BOYS_HEAD.  The constants come from LDS
+// rather than from the code: as literals the compiler kept them in VGPRs and copied
+// one into the accumulator before each Horner step of e^y (v_mov_b64 + v_fmac_f64),
+// while a loaded value is consumed in place.
+constexpr int BOYS_HEAD = 8;
+constexpr int BOYS_HEAD2 = BOYS_HEAD / 2;    // the head in double2
+__device__ const double kBoysExp[BOYS_HEAD] = {
+    2.74954363703727739109e-06, 2.48130760155618204318e-05, 1.98412913960055448115e-04, 1.38888871715607824416e-03,
+    8.33333333116712503263e-03, 4.16666666677564037635e-02, 1.66666666666672708130e-01, 4.99999999999997390976e-01};
+
+// Boys F_0..F_L from the LDS rows of order L (see qbx_device.h for the table): F_L by
+// its row about the nearest grid point, e^{-T} from e^{-T_i} times e^y, y = T_i - T,
+// the downward recurrence for the lower orders, and the asymptotic form above the
+// table.  The row index comes from adding 1.5 x 2^52 (the sum's low word is the
+// rounded 4T) and a 24-bit multiplication: rounding, two conversions and a 32-bit
+// multiplication took half again as long as the whole of F_0's Horner steps.
 template <int L>
 __device__ __forceinline__ void boys_lds(double T, double* __restrict__ F, const double* __restrict__ sb)
 {
     if (T < boys_tmax(L)) {
-        const int i = __double2int_rn(T * QBX_BOYSL_INVDT);
-        const double md = (double)i * QBX_BOYSL_DT - T;
-        const double2* row = (const double2*)(sb + i * QBX_BOYSL_STRIDE);
-        const double2 c01 = row[0], c23 = row[1], c45 = row[2], c67 = row[3], c89 = row[4], c10e = row[5];
-        double acc = fma(md, c10e.x, c89.y);
-        acc = fma(md, acc, c89.x);
-        acc = fma(md, acc, c67.y);
-        acc = fma(md, acc, c67.x);
-        acc = fma(md, acc, c45.y);
-        acc = fma(md, acc, c45.x);
-        acc = fma(md, acc, c23.y);
-        acc = fma(md, acc, c23.x);
-        acc = fma(md, acc, c01.y);
-        acc = fma(md, acc, c01.x);
+        constexpr double kRound = 6755399441055744.0;
+        const double ti = fma(T, QBX_BOYSL_INVDT, kRound);
+        const double y = fma(ti - kRound, QBX_BOYSL_DT, -T);
+        const double2* row =
+            (const double2*)((const char*)sb + __mul24(__double2loint(ti), QBX_BOYSL_STRIDE * (int)sizeof(double)));
+        const double2 c01 = row[0], c23 = row[1], c45 = row[2], c67 = row[3], c8e = row[4];
+        double acc = fma(y, c8e.x, c67.y);
+        acc = fma(y, acc, c67.x);
+        acc = fma(y, acc, c45.y);
+        acc = fma(y, acc, c45.x);
+        acc = fma(y, acc, c23.y);
+        acc = fma(y, acc, c23.x);
+        acc = fma(y, acc, c01.y);
+        acc = fma(y, acc, c01.x);
         F[L] = acc;
         if (L > 0) {
             const double2* kh = (const double2*)(sb - BOYS_HEAD);
-            const double2 k01 = kh[0], k23 = kh[1], k45 = kh[2], k67 = kh[3], k89 = kh[4], kab = kh[5];
-            double ex = fma(md, k01.x, k01.y);
-            ex = fma(md, ex, k23.x);
-            ex = fma(md, ex, k23.y);
-            ex = fma(md, ex, k45.x);
-            ex = fma(md, ex, k45.y);
-            ex = fma(md, ex, k67.x);
-            ex = fma(md, ex, k67.y);
-            ex = fma(md, ex, k89.x);
-            ex = fma(md, ex, k89.y);
-            ex = fma(md, ex, kab.x);
-            ex = fma(md, ex, kab.y);
-            const double e = c10e.y * ex;
+            const double2 k98 = kh[0], k76 = kh[1], k54 = kh[2], k32 = kh[3];
+            double ex = fma(y, k98.x, k98.y);
+            ex = fma(y, ex, k76.x);
+            ex = fma(y, ex, k76.y);
+            ex = fma(y, ex, k54.x);
+            ex = fma(y, ex, k54.y);
+            ex = fma(y, ex, k32.x);
+            ex = fma(y, ex, k32.y);
+            ex = fma(y, ex, 1.0);
+            ex = fma(y, ex, 1.0);
+            const double e = c8e.y * ex;
             const double t2 = 2.0 * T;
 #pragma unroll
             for (int m = L - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0 / (2 * m + 1));
         }
     } else {
-        const double rt = rsqrt(T);
+        const double rt = rsqrt_pos(T);
         F[0] = 0.88622692545275801365 * rt;
         const double h = 0.5 * rt * rt;
 #pragma unroll
@@ -141,30 +155,13 @@ __device__ __forceinline__ void boys_lds(double T, double* __restrict__ F, const
 template <int TPB, int ROWS = QBX_BOYSL_ROWS>
 __device__ __forceinline__ void stage_boys(double2* __restrict__ dst, const double* __restrict__ src)
 {
-    if (threadIdx.x < BOYS_HEAD2) {
-        // 1/k! for k = 11 - 2t and 10 - 2t
-        const int k = 11 - 2 * (int)threadIdx.x;
-        double f = 1.0;
-        for (int j = 2; j < k; ++j) f *= j;
-        dst[threadIdx.x] = make_double2(1.0 / (f * k), 1.0 / f);
-    }
+    if (threadIdx.x < BOYS_HEAD) ((double*)dst)[threadIdx.x] = kBoysExp[threadIdx.x];
     const double2* s = (const double2*)src;
     for (int i = threadIdx.x; i < ROWS * QBX_BOYSL_STRIDE / 2; i += TPB) dst[BOYS_HEAD2 + i] = s[i];
 }
 
-// 1/sqrt(x) for finite x > 0 (p + q of a primitive quartet): the hardware
-// estimate r refined by the second-order term of the binomial series,
-// 1/sqrt(x) = r (1 - e)^(-1/2) = r (1 + e/2 + 3e^2/8 + ...) with e = 1 - x r^2.
-// The library rsqrt() applies the same correction and then re-checks the
-// estimate for zero, infinite and NaN inputs, which cannot occur here.
-__device__ __forceinline__ double rsqrt_pos(double x)
-{
-    const double r = __builtin_amdgcn_rsq(x);
-    const double e = fma(r * -x, r, 1.0);
-    return fma(r * e, fma(e, 0.375, 0.5), r);
-}
-
-// The ket-pair quantities one primitive quartet reads.
+// The ket-pair quantities one primitive quartet reads; Kq carries the quartet's
+// constant 2 pi^{5/2}.
 struct KetPrim {
     double q, inv2q, Qx, Qy, Qz, QCx, QCy, QCz, Kq;
 };
@@ -180,8 +177,18 @@ __device__ __forceinline__ KetPrim load_ket(const PrimPair* __restrict__ p)
     k.QCx = p->PAx;
     k.QCy = p->PAy;
     k.QCz = p->PAz;
-    k.Kq = p->Kp;
+    k.Kq = 34.986836655249725693 * p->Kp;
     return k;
+}
+
+// The bra-pair quantities one primitive quartet reads.
+struct BraPrim {
+    double p, inv2p, Px, Py, Pz, PAx, PAy, PAz, Kp;
+};
+
+template <typename BraPtr> __device__ __forceinline__ BraPrim load_bra(BraPtr p)
+{
+    return BraPrim{p->p, p->inv2p, p->Px, p->Py, p->Pz, p->PAx, p->PAy, p->PAz, p->Kp};
 }
 
 // Sum over the primitive quartets of one contracted shell quartet: bra pairs
@@ -193,6 +200,7 @@ __device__ __forceinline__ void prim_loop(R* __restrict__ acc, BraPtr BP, int bn
                                           const PrimPair* __restrict__ KP, int kn,
                                           const double* __restrict__ sb)
 {
+    if (bn <= 0) return;    // every primitive pair of the bra was dropped
     KetPrim nxt;
     if (PREFETCH && kn > 0) nxt = load_ket(KP);
     for (int v = 0; v < kn; ++v) {
@@ -203,9 +211,13 @@ __device__ __forceinline__ void prim_loop(R* __restrict__ acc, BraPtr BP, int bn
         } else {
             Q = load_ket(KP + v);
         }
+        BraPrim bnext = load_bra(BP);
         for (int u = 0; u < bn; ++u) {
-            const double p = BP[u].p, inv2p = BP[u].inv2p, Px = BP[u].Px, Py = BP[u].Py, Pz = BP[u].Pz;
-            const double PAx = BP[u].PAx, PAy = BP[u].PAy, PAz = BP[u].PAz, Kp = BP[u].Kp;
+            // the next pair's loads are in flight while this one is evaluated
+            const BraPrim B = bnext;
+            bnext = load_bra(BP + (u + 1 < bn ? u + 1 : u));
+            const double p = B.p, inv2p = B.inv2p, Px = B.Px, Py = B.Py, Pz = B.Pz;
+            const double PAx = B.PAx, PAy = B.PAy, PAz = B.PAz, Kp = B.Kp;
             const double pq = p + Q.q;
             const double s = rsqrt_pos(pq);
             const double inv = s * s;
@@ -213,7 +225,7 @@ __device__ __forceinline__ void prim_loop(R* __restrict__ acc, BraPtr BP, int bn
             const double rho = p * Q.q * inv;
             const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);
             // 2 pi^{5/2} (c c K / p)_{ab} (c c K / q)_{cd} / sqrt(p+q)
-            const double pref = 34.986836655249725693 * Kp * Q.Kq * s;
+            const double pref = Kp * Q.Kq * s;
             double Fd[LT + 1];
             boys_lds<LT>(T, Fd, sb);
             R F[LT + 1];
@@ -824,7 +836,7 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
                 const double inv = s * s;
                 const double rho = p * Q.q * inv;
                 const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);
-                const double pref0 = 34.986836655249725693 * Q.Kq * s;
+                const double pref0 = Q.Kq * s;
                 double Fd[LT + 1];
                 boys_lds<LT>(T, Fd, sb);
                 const double rho_p = Q.q * inv, rho_q = p * inv;

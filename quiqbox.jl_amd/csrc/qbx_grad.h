@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void eri_grad_kernel(EriArgs a)
         const int pC = a.shell_poff[sC], pD = a.shell_poff[sD];
         double gA[3] = {0.0, 0.0, 0.0}, gB[3] = {0.0, 0.0, 0.0}, gC[3] = {0.0, 0.0, 0.0}, gD[3] = {0.0, 0.0, 0.0};
         for (int u = 0; u < bn; ++u) {
-            const double p = BP[u].p, inv2p = BP[u].inv2p, bx = BP[u].pad, KpC = 34.986836655249725693 * BP[u].Kp;
+            const double p = BP[u].p, inv2p = BP[u].inv2p, bx = BP[u].pad, Kp = BP[u].Kp;
             const double Px = BP[u].Px, Py = BP[u].Py, Pz = BP[u].Pz;
             const double PA[3] = {BP[u].PAx, BP[u].PAy, BP[u].PAz};
             double sa = 0.0, sbx = 0.0, sl = 0.0;
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void eri_grad_kernel(EriArgs a)
                 const double PQ[3] = {Px - Q.Qx, Py - Q.Qy, Pz - Q.Qz};
                 const double s = rsqrt_pos(p + Q.q), inv = s * s;
                 const double T = p * Q.q * inv * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
-                const double pref = KpC * Q.Kq * s;
+                const double pref = Kp * Q.Kq * s;
                 double Bm[LT + 2];
                 boys_lds<LT + 1>(T, Bm, sb);
                 double F[LT + 1];
