@@ -100,10 +100,14 @@ constexpr double QBX_PRIM_PAIR_CUT = 1e-20;
 // runs as long as its lane with the most primitive pairs; in Schwarz order,
 // contracted core pairs (81 primitive pairs in cc-pVDZ oxygen) sit among
 // single-primitive ones.  Each pair class is therefore ordered by bucket of
-// primitive-pair count, Schwarz order within a bucket, and every bra gets one
-// ket range per bucket.  Estimated on the (ss|ss) kets of 24 H2O in cc-pVDZ:
-// lanes busy 36% -> 78% of the primitive loop, 3.5% more waves.
-constexpr int kKetBuckets = 5;
+// primitive-pair count (most first), Schwarz order within a bucket, and a bra's
+// ket list is its range of every bucket, one after another: only its last chunk
+// of 64 is partial.  Up to kKetBuckets buckets, one per occurring count where
+// those are few (bucket_tops).  Busy lanes of the primitive loop, from the pair
+// lists: 592-function cluster of 3-primitive shells 0.70-0.80 (Schwarz order)
+// -> 0.93-0.98, 24 H2O in cc-pVDZ 0.77-0.80 (fixed buckets 1, 4, 9, 27 with a
+// list and a partial chunk each) -> 0.83-0.94, 8 H2O 0.53-0.66 -> 0.66-0.82.
+constexpr int kKetBuckets = 10;
 
 // Fixed device work array of qbx_density_purify_noalloc: P, Q, T (n x n, padded to
 // a multiple of 32) and the auxiliary values (row intervals, state, shares of 32 x
@@ -119,7 +123,35 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch_addr[kMaxDevices] = {};
 
-inline int ket_bucket(int ppn) { return ppn <= 1 ? 0 : ppn <= 4 ? 1 : ppn <= 9 ? 2 : ppn <= 27 ? 3 : 4; }
+// Largest primitive-pair count of every bucket, descending: a bucket per
+// occurring count, the neighbours merged that raise the padded total least
+// until kKetBuckets remain.
+inline std::vector<int> bucket_tops(const std::vector<int>& ppn)
+{
+    std::map<int, int64_t, std::greater<int>> count;
+    for (int v : ppn) ++count[v];
+    std::vector<std::pair<int, int64_t>> g(count.begin(), count.end());
+    while ((int)g.size() > kKetBuckets) {
+        size_t at = 0;
+        int64_t least = INT64_MAX;
+        for (size_t k = 0; k + 1 < g.size(); ++k) {
+            const int64_t pad = (int64_t)(g[k].first - g[k + 1].first) * g[k + 1].second;
+            if (pad < least) { least = pad; at = k; }
+        }
+        g[at].second += g[at + 1].second;
+        g.erase(g.begin() + at + 1);
+    }
+    std::vector<int> tops;
+    for (const auto& v : g) tops.push_back(v.first);
+    return tops;
+}
+
+inline int ket_bucket(const std::vector<int>& tops, int ppn)
+{
+    int k = 0;
+    while (k + 1 < (int)tops.size() && ppn <= tops[k + 1]) ++k;
+    return k;
+}
 
 }  // namespace
 
@@ -173,29 +205,30 @@ struct PairClass {
     std::vector<double> Q, AB;
     std::vector<int> rank, bstart;
     int nbk = 1;               // ket buckets of this class (1: plain Schwarz order)
-    std::unique_ptr<PairClass> plain;   // bucketed classes: the same pairs in plain Schwarz order
+    std::vector<int> btop;     // largest primitive-pair count of each bucket
+    std::unique_ptr<PairClass> plain;   // bucketed classes beside f or g shells: the same pairs in plain Schwarz order
     DevBuf<int> d_shA, d_shB, d_ppo, d_ppn;
     DevBuf<double> d_Q, d_AB;
     int n() const { return (int)shA.size(); }
 };
 
+// Ket lists and tasks of one ERI class and precision, in the basis's list pool.
 struct TaskSet {
-    DevBuf<int64_t> prefix;
-    DevBuf<int> koff;
-    DevBuf<int> cpre;          // waves (chunks of 64 kets) per bra, prefix sums
-    DevBuf<int> spre;          // K-row blocks (chunks chunks) per bra, prefix sums
+    const int* klist = nullptr;       // see KetList
+    const int* cpre = nullptr;        // waves (chunks of 64 kets) per bra, prefix sums
+    const RowTask* rtask = nullptr;   // K-row tasks
     int nsuper = 0;
-    int chunks = ROW_CHUNKS;   // chunks per K-row task
     int64_t total = 0;
     int nwave = 0;
     int nbra = 0;
 };
 
-// Twin-bra groups of one ERI class and precision (see TWIN_MAX): task prefix
-// and, per group, TWIN_MAX records (bra, first ket, end of kets).
+// Twin-bra groups of one ERI class (see TWIN_MAX): their ket lists, their
+// TWIN_MAX member bras and their tasks.
 struct TwinSet {
-    DevBuf<int> gpre;
-    DevBuf<int> gmem;
+    const int* klist = nullptr;
+    const int* gmem = nullptr;
+    const RowTask* rtask = nullptr;
     int ngroup = 0, ntask = 0, twmax = 0;
 };
 
@@ -233,8 +266,9 @@ struct qbx_basis {
     // the groups' own
     std::vector<std::vector<int>> twins[QBX_N_PAIR_CLASSES];
     bool use_twin[QBX_N_CLASSES] = {};
-    TaskSet s64[QBX_N_CLASSES], s32[QBX_N_CLASSES];
+    TaskSet s64[QBX_N_CLASSES];
     TwinSet w64[QBX_N_CLASSES];
+    DevBuf<int> d_lists;       // their arrays
     DevBuf<double> ws[QBX_N_CLASSES];   // staged-class workspaces
     // work buffers
     DevBuf<double> d_D, d_J, d_K, d_G;
@@ -705,24 +739,16 @@ EriLaunch schwarz_launcher(int la, int lb)
     return nullptr;
 }
 
-// The pair lists an ERI class runs over: the staged classes (few long waves
-// with a large fixed cost each, where the extra partial waves of the buckets
-// cost more than the even lanes save) take the plain Schwarz order of a
-// bucketed ket class, and of the bra class when it is the same pair class.
-const PairClass& pair_view(const qbx_basis* b, int cls, int side)
-{
-    const PairClass& P = b->pc[class_pc(cls, side)];
-    if (P.plain && qbx_class_ws[cls] > 0 && (side == 1 || X_is_Y(cls))) return *P.plain;
-    return P;
-}
+// Bra (side 0) or ket (side 1) pair class of an ERI class.
+const PairClass& pair_class(const qbx_basis* b, int cls, int side) { return b->pc[class_pc(cls, side)]; }
 
 EriArgs base_args(qbx_basis* b, int cls)
 {
     EriArgs a;
     std::memset(&a, 0, sizeof(a));
     const int X = class_pc(cls, 0), Y = class_pc(cls, 1);
-    a.bra = pcdev(pair_view(b, cls, 0));
-    a.ket = pcdev(pair_view(b, cls, 1));
+    a.bra = pcdev(pair_class(b, cls, 0));
+    a.ket = pcdev(pair_class(b, cls, 1));
     a.pp = b->d_pp.p;
     a.sh = b->d_sh.p;
     a.boys = b->ctx->boys.p;
@@ -731,11 +757,12 @@ EriArgs base_args(qbx_basis* b, int cls)
     a.boysl = b->ctx->boysl.p + (size_t)lt * QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE;
     a.same = X == Y;
     a.N = b->nbf;
-    a.nbk = pair_view(b, cls, 1).nbk;
+    a.nbk = pair_class(b, cls, 1).nbk;
     return a;
 }
 
-// Workspace of a staged class for up to `nwave` waves (kStageSlots at most).
+// Workspace of a staged class for up to `nwave` waves or blocks of shared
+// waves (kStageSlots at most).
 void attach_workspace(qbx_basis* b, int cls, int nwave, EriArgs& a)
 {
     const int wsv = qbx_class_ws[cls];
@@ -766,10 +793,14 @@ void find_twins(qbx_basis* b)
         if (it == fam_of.end()) it = fam_of.emplace(key, (int)fam_of.size()).first;
         fam[s] = it->second;
     }
+    std::vector<int> copies(fam_of.size(), 0);
+    bool any = false;
+    for (int f : fam) any = ++copies[f] > 1 || any;
     for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
         const PairClass& P = b->pc[c];
         std::map<std::vector<int>, std::vector<int>> sig;
-        for (int k = 0; k < P.n(); ++k) {
+        for (int k = 0; any && k < P.n(); ++k) {
+            if (copies[fam[P.shA[k]]] * copies[fam[P.shB[k]]] < 2) continue;   // no other pair of these families
             std::vector<int> key = {fam[P.shA[k]], fam[P.shB[k]], P.ppn[k]};
             for (int u = 0; u < P.ppn[k]; ++u) key.push_back(b->ppk[P.ppo[k] + u]);
             sig[key].push_back(k);
@@ -872,6 +903,7 @@ void ensure_schwarz(qbx_basis* b)
         if (n == 0) {
             P.nbk = 1;
             P.bstart.assign(2, 0);
+            P.btop.assign(1, 0);
             continue;
         }
         std::vector<double> Q(n);
@@ -882,39 +914,10 @@ void ensure_schwarz(qbx_basis* b)
         std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return Q[x] > Q[y]; });
         std::vector<int> qpos(n);
         for (int k = 0; k < n; ++k) qpos[perm[k]] = k;
-        // buckets where they make the lanes of a wave markedly more even:
-        // busy fraction of the primitive loop over chunks of 64 pairs, in
-        // Schwarz order and within buckets.  Measured: 24 H2O in cc-pVDZ
-        // gains 1.9-2.8x on this estimate for its s/p pair classes and its
-        // Fock build drops 80 -> 54 ms; the 592-function cluster of
-        // 3-primitive shells gains at most 1.29x, and bucketing its (pp)
-        // kets at that ratio made (pp|pp) 1.55 -> 2.17 ms (extra partial
-        // waves per bra), so the bar is 1.5x.
-        auto busy = [&](const std::vector<int>& order, bool by_bucket) {
-            double work = 0.0, span = 0.0;
-            int mx = 0, fill = 0, prev = -1;
-            for (size_t k = 0; k < order.size(); ++k) {
-                const int pn = P.ppn[order[k]];
-                const int bk = by_bucket ? ket_bucket(pn) : 0;
-                if (fill == 64 || (fill > 0 && bk != prev)) {   // chunk full, or a bucket starts its own
-                    span += 64.0 * mx;
-                    mx = 0;
-                    fill = 0;
-                }
-                prev = bk;
-                work += pn;
-                mx = std::max(mx, pn);
-                ++fill;
-            }
-            span += 64.0 * mx;
-            return span > 0.0 ? work / span : 1.0;
-        };
-        const double busy_plain = busy(perm, false);
-        std::vector<int> bperm = perm;
-        std::stable_sort(bperm.begin(), bperm.end(),
-                         [&](int x, int y) { return ket_bucket(P.ppn[x]) < ket_bucket(P.ppn[y]); });
-        const bool bucketed = b->ctx->ket_buckets && busy(bperm, true) >= 1.5 * busy_plain;
-        if (bucketed) {
+        const std::vector<int> tops = b->ctx->ket_buckets ? bucket_tops(P.ppn) : std::vector<int>(1, INT32_MAX);
+        const bool bucketed = tops.size() > 1;
+        auto bucket = [&](int x) { return ket_bucket(tops, P.ppn[x]); };
+        if (bucketed && b->has_high) {
             std::unique_ptr<PairClass> pl(new PairClass());
             for (int k = 0; k < n; ++k) {
                 const int o = perm[k];
@@ -934,15 +937,18 @@ void ensure_schwarz(qbx_basis* b)
             pl->d_AB.upload(pl->AB, st);
             pl->d_Q.upload(pl->Q, st);
             P.plain = std::move(pl);
-            perm.swap(bperm);
         }
+        if (bucketed) std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return bucket(x) < bucket(y); });
         PairClass S;
-        S.nbk = bucketed ? kKetBuckets : 1;
+        S.nbk = (int)tops.size();
+        S.btop.assign(S.nbk, 0);
         S.bstart.assign(S.nbk + 1, 0);
         for (int k = 0; k < n; ++k) {
             const int o = perm[k];
             S.rank.push_back(qpos[o]);
-            ++S.bstart[(bucketed ? ket_bucket(P.ppn[o]) : 0) + 1];
+            const int bk = bucket(o);
+            ++S.bstart[bk + 1];
+            S.btop[bk] = std::max(S.btop[bk], P.ppn[o]);
             S.shA.push_back(P.shA[o]);
             S.shB.push_back(P.shB[o]);
             S.ppo.push_back(P.ppo[o]);
@@ -960,6 +966,7 @@ void ensure_schwarz(qbx_basis* b)
         P.rank.swap(S.rank);
         P.bstart.swap(S.bstart);
         P.nbk = S.nbk;
+        P.btop.swap(S.btop);
         P.d_shA.upload(P.shA, st);
         P.d_shB.upload(P.shB, st);
         P.d_ppo.upload(P.ppo, st);
@@ -981,164 +988,316 @@ int count_ge(const std::vector<double>& q, double v)
 // Screened task lists: for bra i of class X, kets j of class Y with
 // Q_i Q_j >= thr (and j before or at i in Schwarz order when X == Y).  Under
 // mixed precision the surviving kets split at Q_i Q_j >= cut into an FP64 head
-// and an FP32 tail.  One task range per (bra, ket bucket): task t = i nbk + k.
-struct TaskCounts {
-    std::vector<int64_t> p64, p32;
-    std::vector<int> k64, k32;
-    std::vector<int> w64, w32;   // waves of 64 kets per task range, prefix sums
-    std::vector<int> s64, s32;   // K-row blocks per task range, prefix sums
-    int ntb = 0;                 // task ranges (bras x buckets)
-    int rc = ROW_CHUNKS;         // chunks per K-row block
+// and an FP32 tail.  One range per (bra, ket bucket), t = i nbk + k: FP64 [0,
+// c64), FP32 [c64, cnt), relative to the bucket's first position.
+struct RangeCounts {
+    std::vector<int> cnt, head;   // head: mixed precision only
+    const std::vector<int>& c64() const { return head.empty() ? cnt : head; }
 };
 
-// Surviving kets of bra i in ket bucket k: FP64 [0, c64), FP32 [c64, cnt),
-// relative to the bucket's first position.
-void bra_range(const qbx_basis* b, int cls, int i, int k, double thr, int mode, double cut, int& c64, int& cnt)
+// Within a bucket of bras the thresholds only rise, so the counts are found by
+// stepping back.
+RangeCounts range_counts(const qbx_basis* b, int cls, double thr, int mode, double cut)
 {
-    const int X = class_pc(cls, 0), Y = class_pc(cls, 1);
-    const PairClass& PX = pair_view(b, cls, 0);
-    const PairClass& PY = pair_view(b, cls, 1);
-    const int s0 = PY.bstart[k], s1 = PY.bstart[k + 1];
-    const double qi = PX.Q[i];
-    auto ge = [&](double v) {
-        return (int)(std::upper_bound(PY.Q.begin() + s0, PY.Q.begin() + s1, v,
-                                      [](double x, double y) { return x > y; }) - (PY.Q.begin() + s0));
-    };
-    if (thr <= 0.0) cnt = s1 - s0;
-    else cnt = qi > 0.0 ? ge(thr / qi) : 0;
-    if (X == Y)
-        cnt = std::min(cnt, (int)(std::upper_bound(PY.rank.begin() + s0, PY.rank.begin() + s1, PX.rank[i]) -
-                                  (PY.rank.begin() + s0)));
-    c64 = cnt;
-    if (mode == QBX_PREC_MIXED) c64 = std::min(cnt, qi > 0.0 ? ge(cut / qi) : 0);
-}
-
-// chunks of 64 kets per K-row task of class cls
-int task_chunks(int cls)
-{
-    if (qbx_class_ws[cls] == 0) return ROW_CHUNKS;
-    return qbx_class_split[cls] > 1 && qbx_class_split_chunks[cls] > 0 ? qbx_class_split_chunks[cls]
-                                                                       : STAGED_ROW_CHUNKS;
-}
-
-// start64: per task range, the first FP64 ket left to these lists (the twin
-// groups take the kets before it); null: all of them
-void task_counts(const qbx_basis* b, int cls, double thr, int mode, double cut, TaskCounts& tc,
-                 const std::vector<int>* start64 = nullptr)
-{
-    const int nx = b->pc[class_pc(cls, 0)].n();
-    const PairClass& PY = pair_view(b, cls, 1);
+    const bool same = X_is_Y(cls);
+    const PairClass& PX = pair_class(b, cls, 0);
+    const PairClass& PY = pair_class(b, cls, 1);
     const int nk = PY.nbk;
-    const int nt = nx * nk;
-    const int rc = task_chunks(cls);   // chunks per K-row task
-    tc.ntb = nt;
-    tc.rc = rc;
-    tc.p64.assign(nt + 1, 0);
-    tc.p32.assign(nt + 1, 0);
-    tc.k64.assign(std::max(nt, 1), 0);
-    tc.k32.assign(std::max(nt, 1), 0);
-    tc.w64.assign(nt + 1, 0);
-    tc.w32.assign(nt + 1, 0);
-    tc.s64.assign(nt + 1, 0);
-    tc.s32.assign(nt + 1, 0);
-    for (int i = 0; i < nx; ++i)
+    const bool mixed = mode == QBX_PREC_MIXED;
+    const int nx = PX.n();
+    // least ket bound that bra i keeps, and keeps in FP64
+    std::vector<double> least(nx), least64(mixed ? nx : 0);
+    for (int i = 0; i < nx; ++i) {
+        const double qi = PX.Q[i];
+        least[i] = qi > 0.0 ? thr / qi : HUGE_VAL;
+        if (mixed) least64[i] = qi > 0.0 ? cut / qi : HUGE_VAL;
+    }
+    RangeCounts r;
+    r.cnt.resize((size_t)nx * nk);
+    if (mixed) r.head.resize((size_t)nx * nk);
+    std::vector<int> all(nk), head(nk), upto(nk);
+    for (int kx = 0; kx < PX.nbk; ++kx) {
         for (int k = 0; k < nk; ++k) {
-            const int t = i * nk + k;
-            int c64, cnt;
-            bra_range(b, cls, i, k, thr, mode, cut, c64, cnt);
-            const int k0 = start64 ? std::min((*start64)[t], c64) : 0;
-            const int s0 = PY.bstart[k];
-            tc.k64[t] = s0 + k0;
-            tc.k32[t] = s0 + c64;
-            tc.p64[t + 1] = tc.p64[t] + (c64 - k0);
-            tc.p32[t + 1] = tc.p32[t] + (cnt - c64);
-            tc.w64[t + 1] = tc.w64[t] + (c64 - k0 + 63) / 64;
-            tc.w32[t + 1] = tc.w32[t] + (cnt - c64 + 63) / 64;
-            tc.s64[t + 1] = tc.s64[t] + ((c64 - k0 + 63) / 64 + rc - 1) / rc;
-            tc.s32[t + 1] = tc.s32[t] + ((cnt - c64 + 63) / 64 + rc - 1) / rc;
+            all[k] = head[k] = PY.bstart[k + 1] - PY.bstart[k];
+            upto[k] = 0;
         }
+        for (int i = PX.bstart[kx]; i < PX.bstart[kx + 1]; ++i)
+            for (int k = 0; k < nk; ++k) {
+                const double* q = PY.Q.data() + PY.bstart[k];
+                if (thr > 0.0)
+                    while (all[k] > 0 && !(q[all[k] - 1] >= least[i])) --all[k];
+                int cnt = all[k];
+                if (same) {
+                    const int* rank = PY.rank.data() + PY.bstart[k];
+                    while (upto[k] < PY.bstart[k + 1] - PY.bstart[k] && rank[upto[k]] <= PX.rank[i]) ++upto[k];
+                    cnt = std::min(cnt, upto[k]);
+                }
+                r.cnt[(size_t)i * nk + k] = cnt;
+                if (mixed) {
+                    while (head[k] > 0 && !(q[head[k] - 1] >= least64[i])) --head[k];
+                    r.head[(size_t)i * nk + k] = std::min(cnt, head[k]);
+                }
+            }
+    }
+    return r;
 }
 
-void upload_tasks(TaskSet& t64, TaskSet& t32, const TaskCounts& tc, hipStream_t st)
-{
-    const int nt = tc.ntb;
-    t64.prefix.upload(tc.p64, st);
-    t64.koff.upload(tc.k64, st);
-    t64.cpre.upload(tc.w64, st);
-    t64.spre.upload(tc.s64, st);
-    t64.nsuper = tc.s64[nt];
-    t64.chunks = tc.rc;
-    t64.total = tc.p64[nt];
-    t64.nwave = tc.w64[nt];
-    t64.nbra = nt;
-    t32.prefix.upload(tc.p32, st);
-    t32.koff.upload(tc.k32, st);
-    t32.cpre.upload(tc.w32, st);
-    t32.spre.upload(tc.s32, st);
-    t32.nsuper = tc.s32[nt];
-    t32.chunks = tc.rc;
-    t32.total = tc.p32[nt];
-    t32.nwave = tc.w32[nt];
-    t32.nbra = nt;
-}
+// The device lists of a basis in one allocation: arrays are appended on the
+// host, then uploaded together, and the pointers set.
+class ListPool {
+public:
+    explicit ListPool(size_t guess) { host_.reserve(guess); }
+    // n more values, zeroed, for the device pointer *where; returns their place
+    template <typename T> size_t add(size_t n, const T** where)
+    {
+        static_assert(sizeof(T) % sizeof(int) == 0 && alignof(T) <= alignof(int), "an array of ints");
+        const size_t at = host_.size();
+        slots_.push_back({(const void**)where, at});
+        host_.resize(at + n * (sizeof(T) / sizeof(int)));
+        return at;
+    }
+    template <typename T> void add(const std::vector<T>& v, const T** where)
+    {
+        const size_t at = add(v.size(), where);
+        if (!v.empty()) std::memcpy(&host_[at], v.data(), v.size() * sizeof(T));
+    }
+    int* data(size_t at) { return host_.data() + at; }
+    void upload(DevBuf<int>& dst, hipStream_t st)
+    {
+        dst.upload(host_, st);
+        QBX_HIP(hipStreamSynchronize(st));
+        for (const Slot& w : slots_) *w.where = dst.p + w.at;
+    }
 
-// Task lists of the twin groups of class cls: the FP64 kets that every member
-// of a group keeps, [0, common), in chunks of 64, ROW_CHUNKS chunks a task.
-// Each member's kets beyond the common prefix, and all FP32 kets, stay with
-// the per-bra lists (start64 receives the common prefix of every member), so
-// the shared evaluation never covers a ket that a member would not.
-void twin_tasks(const qbx_basis* b, int cls, double thr, int mode, double cut, TwinSet& w64,
-                std::vector<int>& start64, hipStream_t st)
-{
-    const std::vector<std::vector<int>>& groups = b->twins[class_pc(cls, 0)];
-    const PairClass& PY = pair_view(b, cls, 1);
-    std::vector<int> pre(1, 0), mem;
-    int twmax = 0;
-    for (const std::vector<int>& m : groups)
-        for (int k = 0; k < PY.nbk; ++k) {
-            int common = INT32_MAX;
-            for (int i : m) {
-                int c64, cnt;
-                bra_range(b, cls, i, k, thr, mode, cut, c64, cnt);
-                common = std::min(common, c64);
-            }
-            if (common <= 0) continue;
-            twmax = std::max(twmax, (int)m.size());
-            const int s0 = PY.bstart[k];
-            for (size_t t = 0; t < (size_t)TWIN_MAX; ++t) {
-                const bool in = t < m.size();
-                mem.push_back(in ? m[t] : -1);
-                mem.push_back(in ? s0 : 0);
-                mem.push_back(in ? s0 + common : 0);
-                if (in) start64[m[t] * PY.nbk + k] = common;
-            }
-            const int ch = (common + 63) / 64;
-            pre.push_back(pre.back() + (ch + ROW_CHUNKS - 1) / ROW_CHUNKS);
+private:
+    struct Slot {
+        const void** where;
+        size_t at;
+    };
+    std::vector<int> host_;
+    std::vector<Slot> slots_;
+};
+
+// Ket lists in the kernels' layout (KetList), and the prefix sums of their
+// 64-ket waves, in a pool.
+class KetLists {
+public:
+    // room for n lists; the device pointers go to *klist and (unless null) *cpre
+    KetLists(ListPool& pool, const PairClass& ket, size_t n, const int** klist, const int** cpre)
+        : pool_(pool), ket_(ket), kl_(pool.add(n * (2 * ket.nbk + 1), klist)), cpre_(cpre ? pool.add(n + 1, cpre) : 0),
+          has_cpre_(cpre != nullptr)
+    {
+    }
+    // one more list: of bucket k, the kets [lo[k], hi[k]) (lo null: from 0)
+    void add(const int* lo, const int* hi)
+    {
+        int* p = pool_.data(kl_) + (size_t)nl * (2 * ket_.nbk + 1);
+        int n = 0;
+        for (int k = 0; k < ket_.nbk; ++k) {
+            const int l = lo ? std::min(lo[k], hi[k]) : 0;
+            *p++ = n;
+            *p++ = ket_.bstart[k] + l - n;
+            n += hi[k] - l;
         }
-    const int ng = (int)pre.size() - 1;
-    w64.gpre.upload(pre, st);
-    if (ng > 0) w64.gmem.upload(mem, st);
-    w64.ngroup = ng;
-    w64.ntask = pre.back();
-    w64.twmax = twmax;
+        *p = n;
+        nwave += (n + 63) / 64;
+        total += n;
+        ++nl;
+        if (has_cpre_) pool_.data(cpre_)[nl] = nwave;
+    }
+    const int* list(size_t i) const { return pool_.data(kl_) + i * (2 * ket_.nbk + 1); }
+    int64_t total = 0;
+    int nl = 0, nwave = 0;
+
+private:
+    ListPool& pool_;
+    const PairClass& ket_;
+    size_t kl_, cpre_;
+    bool has_cpre_;
+};
+
+// the lists of every bra of class cls: bucket k's kets [lo, hi) (per range; lo
+// null: from 0)
+void bra_lists(const qbx_basis* b, int cls, const int* lo, const std::vector<int>& hi, KetLists& L)
+{
+    const int nx = pair_class(b, cls, 0).n(), nk = pair_class(b, cls, 1).nbk;
+    for (size_t i = 0; i < (size_t)nx; ++i) L.add(lo ? lo + i * nk : nullptr, &hi[i * nk]);
 }
 
 // Estimated work of a class's task lists: primitive shell quartets and
 // contracted shell quartets weighted by the class's cost per unit.
-double class_cost(const qbx_basis* b, int cls, const TaskCounts& tc)
+double class_cost(const qbx_basis* b, int cls, const RangeCounts& r)
 {
-    const PairClass& PX = pair_view(b, cls, 0);
-    const PairClass& PY = pair_view(b, cls, 1);
+    const PairClass& PX = pair_class(b, cls, 0);
+    const PairClass& PY = pair_class(b, cls, 1);
     std::vector<int64_t> kp(PY.n() + 1, 0);
     for (int j = 0; j < PY.n(); ++j) kp[j + 1] = kp[j] + PY.ppn[j];
     double prim = 0.0, quart = 0.0;
-    for (int t = 0; t < tc.ntb; ++t) {
-        const int n64 = (int)(tc.p64[t + 1] - tc.p64[t]), n32 = (int)(tc.p32[t + 1] - tc.p32[t]);
-        const int64_t kets = (kp[tc.k64[t] + n64] - kp[tc.k64[t]]) + (kp[tc.k32[t] + n32] - kp[tc.k32[t]]);
-        prim += (double)PX.ppn[t / PY.nbk] * (double)kets;
-        quart += n64 + n32;
-    }
+    for (int i = 0; i < PX.n(); ++i)
+        for (int k = 0; k < PY.nbk; ++k) {
+            const int cnt = r.cnt[(size_t)i * PY.nbk + k], s0 = PY.bstart[k];
+            prim += (double)PX.ppn[i] * (double)(kp[s0 + cnt] - kp[s0]);
+            quart += cnt;
+        }
     return prim * qbx_class_cost_prim[cls] + quart * qbx_class_cost_quartet[cls];
+}
+
+// Sizes of K-row tasks, in operations of the cost model per lane: an item (a
+// chunk, or a part of one) is cut to about `item`, a wave's share of a task to
+// about `task`.  cost: the class's estimate, total: all classes' (over 64 lanes).
+// A chunk is split where it would take a wave longer than half of the time that
+// its class needs on a full chip, or than an eighth of what the build does: the
+// few chunks of contracted core pairs (81 x 81 primitive quartets against a mean
+// of 82 in 24 H2O) otherwise end each class's launch on a few waves.  Below
+// kLeastItem operations and four times the digest's, an item's fixed part
+// outweighs what it shares.  A wave's share of a task is at most its share of
+// the class.  Measured per build with the chunks of one bucket and 32 chunks a
+// task before: 8 H2O UHF 5.45 -> 3.34 ms, 24 H2O 45.9 -> 35.5, the 592-function
+// cluster 33.4 -> 28.3, 64 atoms of s/p 2.19 -> 1.73; halving or doubling any of
+// the factors moves them by at most 3%.
+struct TaskCaps {
+    double item, task;
+};
+constexpr double kLeastItem = 1500.0;
+
+TaskCaps task_caps(int cls, double cost, double total)
+{
+    const double cp = qbx_class_cost_prim[cls];
+    const double waves = 1024.0 * (cp < 300 ? 4 : cp < 1200 ? 2 : 1);   // resident on the chip, by register use
+    const double least = kLeastItem + 4.0 * qbx_class_cost_quartet[cls];
+    TaskCaps c;
+    c.item = std::max(least, std::max(cost / (64 * 2 * waves), total / (64 * 8 * 4096.0)));
+    c.task = std::max(least, cost / (64 * waves));
+    return c;
+}
+
+// Cuts ket lists into tasks: `waves` waves a block, at most max_items items a
+// task; cp, cq: cost of a primitive quartet and of a quartet.
+class TaskCutter {
+public:
+    TaskCutter(const PairClass& ket, double cp, double cq, const TaskCaps& cap, int waves, int max_items)
+        : ket_(ket), cp_(cp), cq_(cq), cap_(cap), waves_(waves), max_items_(max_items) {}
+    // adds the tasks of list `list` (layout of KetList) for a bra of bn primitive pairs
+    void add(int list, const int* kl, int bn, std::vector<RowTask>& out)
+    {
+        if (bn <= 0) return;
+        const int nbk = ket_.nbk;
+        const Cut* cut = cuts(bn);
+        RowTask cur{list, 0, 0, 0, 0};
+        double cost = 0.0;
+        auto close = [&] {
+            if (cur.item1 > cur.item0) out.push_back(cur);
+            cur.item0 = cur.item1;
+            cost = 0.0;
+        };
+        int chunk = 0;
+        for (int k = 0; k < nbk; ++k) {
+            // the chunks up to this bucket's end whose first ket lies in it
+            const int end = ((k + 1 < nbk ? kl[2 * (k + 1)] : kl[2 * nbk]) + 63) / 64;
+            if (end <= chunk) continue;
+            const Cut& c = cut[k];
+            if (c.parts != cur.parts) {
+                close();
+                cur = RowTask{list, chunk, c.parts, 0, 0};
+            }
+            int left = (end - chunk) * c.parts;
+            while (left > 0) {
+                const int have = cur.item1 - cur.item0;
+                const int fit = (int)std::min((double)max_items_, std::max(1.0, (waves_ * cap_.task - cost) * c.inv));
+                const int even = (have + fit + waves_ - 1) / waves_ * waves_ - have;   // no wave of the block idle
+                const int take = std::min(left, std::max(1, std::min(max_items_ - have, even)));
+                cur.item1 += take;
+                cost += take * c.cost;
+                left -= take;
+                if (cur.item1 - cur.item0 >= max_items_ || cost >= waves_ * cap_.task) close();
+            }
+            chunk = end;
+        }
+        close();
+    }
+
+private:
+    // parts of a chunk of one ket bucket, cost of an item and its inverse
+    struct Cut {
+        int parts;
+        double cost, inv;
+    };
+    const Cut* cuts(int bn)
+    {
+        std::vector<Cut>& v = by_bn_[bn];
+        if (v.empty())
+            for (int top : ket_.btop) {
+                const double whole = (double)bn * top * cp_;
+                const int want = std::max(1, (int)std::min((double)bn, whole / cap_.item + 0.5));
+                const int per = (bn + want - 1) / want, parts = (bn + per - 1) / per;
+                const double c = whole / parts + cq_;
+                v.push_back({parts, c, 1.0 / c});
+            }
+        return v.data();
+    }
+    const PairClass& ket_;
+    double cp_, cq_;
+    TaskCaps cap_;
+    int waves_, max_items_;
+    std::map<int, std::vector<Cut>> by_bn_;
+};
+
+// K-row tasks of class cls over the ket lists L of its bras
+std::vector<RowTask> row_tasks(const qbx_basis* b, int cls, const KetLists& L, TaskCaps cap)
+{
+    const PairClass& PX = pair_class(b, cls, 0);
+    const PairClass& PY = pair_class(b, cls, 1);
+    int waves = ROW_WAVES, items = ROW_ITEMS;
+    if (qbx_class_ws[cls] > 0) {
+        items = STAGED_ROW_ITEMS;
+        if (qbx_class_split[cls] > 1 && qbx_class_split_chunks[cls] > 0) {   // the block shares each item
+            waves = 1;
+            items = qbx_class_split_chunks[cls];
+            cap.item *= qbx_class_split[cls];
+            cap.task *= qbx_class_split[cls];
+        }
+    }
+    TaskCutter cutter(PY, qbx_class_cost_prim[cls], qbx_class_cost_quartet[cls], cap, waves, items);
+    std::vector<RowTask> out;
+    for (int i = 0; i < PX.n(); ++i) cutter.add(i, L.list(i), PX.ppn[i], out);
+    return out;
+}
+
+// Ket lists and tasks of the twin groups of class cls: the FP64 kets that every
+// member of a group keeps, [0, common) of each bucket.
+// Each member's kets beyond the common prefix, and all FP32 kets, stay with
+// the per-bra lists (start64 receives the common prefix of every member), so
+// the shared evaluation never covers a ket that a member would not.
+void add_twins(const qbx_basis* b, int cls, const RangeCounts& r, const TaskCaps& cap, ListPool& pool, TwinSet& w64,
+               std::vector<int>& start64)
+{
+    const PairClass& PX = pair_class(b, cls, 0);
+    const PairClass& PY = pair_class(b, cls, 1);
+    const int nk = PY.nbk;
+    const std::vector<std::vector<int>>& groups = b->twins[class_pc(cls, 0)];
+    KetLists L(pool, PY, groups.size(), &w64.klist, nullptr);
+    std::vector<int> mem, common(nk);
+    std::vector<RowTask> task;
+    w64.ngroup = w64.ntask = w64.twmax = 0;
+    TaskCutter cutter(PY, qbx_class_cost_prim[cls], qbx_class_cost_quartet[cls] * TWIN_MAX, cap, TWIN_WAVES, ROW_ITEMS);
+    for (const std::vector<int>& m : groups) {
+        int any = 0;
+        for (int k = 0; k < nk; ++k) {
+            common[k] = INT32_MAX;
+            for (int i : m) common[k] = std::min(common[k], r.c64()[(size_t)i * nk + k]);
+            any = std::max(any, common[k]);
+        }
+        if (any == 0) continue;
+        for (int i : m) std::copy(common.begin(), common.end(), start64.begin() + (size_t)i * nk);
+        for (size_t t = 0; t < (size_t)TWIN_MAX; ++t) mem.push_back(t < m.size() ? m[t] : -1);
+        L.add(nullptr, common.data());
+        cutter.add(w64.ngroup, L.list(w64.ngroup), PX.ppn[m[0]], task);
+        w64.twmax = std::max(w64.twmax, (int)m.size());
+        ++w64.ngroup;
+    }
+    w64.ntask = (int)task.size();
+    pool.add(mem, &w64.gmem);
+    pool.add(task, &w64.rtask);
 }
 
 void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
@@ -1148,14 +1307,32 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
     // the lists are rewritten (and may be reallocated) on the context stream:
     // the last build, on whatever stream it ran, must be done reading them
     if (b->built) QBX_HIP(hipEventSynchronize(b->ev_done));
-    hipStream_t st = b->ctx->stream;
+    b->tasks_valid = false;
+    std::vector<RangeCounts> rc(QBX_N_CLASSES);
+    double total = 0.0;
     for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
-        TaskCounts tc;
-        task_counts(b, cls, thr, mode, cut, tc);
+        rc[cls] = range_counts(b, cls, thr, mode, cut);
+        total += b->class_cost[cls] = class_cost(b, cls, rc[cls]);
+    }
+    size_t guess = 0;
+    for (const RangeCounts& r : rc) guess += (mode == QBX_PREC_MIXED ? 6 : 4) * r.cnt.size();
+    ListPool pool(guess);
+    for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
+        const RangeCounts& r = rc[cls];
         const int X = class_pc(cls, 0);
-        const int nx = b->pc[X].n();
-        upload_tasks(b->t64[cls], b->t32[cls], tc, st);
-        b->class_cost[cls] = class_cost(b, cls, tc);
+        const TaskCaps cap = task_caps(cls, b->class_cost[cls], total);
+        auto add = [&](TaskSet& t, const int* lo, const std::vector<int>& hi) {
+            KetLists L(pool, pair_class(b, cls, 1), pair_class(b, cls, 0).n(), &t.klist, &t.cpre);
+            bra_lists(b, cls, lo, hi, L);
+            const std::vector<RowTask> tasks = row_tasks(b, cls, L, cap);
+            pool.add(tasks, &t.rtask);
+            t.nsuper = (int)tasks.size();
+            t.total = L.total;
+            t.nwave = L.nwave;
+            t.nbra = L.nl;
+        };
+        add(b->t64[cls], nullptr, r.c64());
+        if (mode == QBX_PREC_MIXED) add(b->t32[cls], r.c64().data(), r.cnt);
         b->use_twin[cls] = false;
         // only where bra and ket classes differ: within one pair class a bra's
         // kets end at its own Schwarz-sorted position, so the members' common
@@ -1163,17 +1340,15 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
         // (measured on 24 H2O in cc-pVDZ: (ps|ss) 27.8 -> 24.7 ms, while
         // (ss|ss) 15.2 -> 16.0 and (ps|ps) 11.3 -> 12.0 ms)
         if (b->ctx->twins && qbx_class_twin[cls] && X != class_pc(cls, 1) && !b->twins[X].empty()) {
-            std::vector<int> start64((size_t)nx * pair_view(b, cls, 1).nbk, 0);
-            twin_tasks(b, cls, thr, mode, cut, b->w64[cls], start64, st);
+            std::vector<int> start64(r.cnt.size(), 0);
+            add_twins(b, cls, r, cap, pool, b->w64[cls], start64);
             if (b->w64[cls].ngroup > 0) {
-                TaskCounts ts;
-                task_counts(b, cls, thr, mode, cut, ts, &start64);
-                upload_tasks(b->s64[cls], b->s32[cls], ts, st);
+                add(b->s64[cls], start64.data(), r.c64());
                 b->use_twin[cls] = true;
             }
         }
     }
-    QBX_HIP(hipStreamSynchronize(st));
+    pool.upload(b->d_lists, b->ctx->stream);
     b->tasks_valid = true;
     b->task_thr = thr;
     b->task_mode = mode;
@@ -1456,18 +1631,17 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
             twin = rows <= (size_t)ROW_LDS_MAX && rows + boys <= (size_t)ctx->lds_max;
         }
         auto set_tasks = [&](const TaskSet& t, const TwinSet* w) {
-            a.prefix = t.prefix.p;
-            a.koff = t.koff.p;
-            a.cpre = t.cpre.p;
+            a.klist = t.klist;
+            a.cpre = t.cpre;
             // no K-row task lists: the one-wave-per-chunk kernels run
-            a.spre = ctx->jk_rows ? t.spre.p : nullptr;
+            a.rtask = ctx->jk_rows ? t.rtask : nullptr;
             a.nsuper = t.nsuper;
-            a.tchunks = t.chunks;
             a.total = t.total;
             a.nwave = t.nwave;
             a.nbra = t.nbra;
-            a.gpre = w ? w->gpre.p : nullptr;
-            a.gmem = w ? w->gmem.p : nullptr;
+            a.gklist = w ? w->klist : nullptr;
+            a.gmem = w ? w->gmem : nullptr;
+            a.gtask = w ? w->rtask : nullptr;
             a.ngroup = w ? w->ngroup : 0;
             a.ntwtask = w ? w->ntask : 0;
             a.twmax = w ? w->twmax : 0;
@@ -1476,7 +1650,10 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
         a.split = ctx->staged_split ? 1 : 0;
         const TaskSet& t64 = twin ? b->s64[cls] : b->t64[cls];
         set_tasks(t64, twin ? &b->w64[cls] : nullptr);
-        attach_workspace(b, cls, std::max(t64.nwave, mode == QBX_PREC_MIXED ? b->t32[cls].nwave : 0), a);
+        const TaskSet& t32 = b->t32[cls];
+        int slots = std::max(t64.nwave, ROW_WAVES * t64.nsuper);
+        if (mode == QBX_PREC_MIXED) slots = std::max(slots, std::max(t32.nwave, ROW_WAVES * t32.nsuper));
+        attach_workspace(b, cls, slots, a);
         k_jk64[cls](a, ls);
         if (mode == QBX_PREC_MIXED) {
             set_tasks(b->t32[cls], nullptr);
@@ -2008,38 +2185,28 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
         // each class's task lists (host and device) stay alive until the one
         // synchronization below; the classes write disjoint elements and run
         // concurrently on the auxiliary streams
-        struct DenseTasks {
-            TaskCounts tc;
-            DevBuf<int64_t> pre;
-            DevBuf<int> ko, cw;
-        };
-        std::vector<std::unique_ptr<DenseTasks>> lists;
+        DevBuf<int> lists;
+        ListPool pool(0);
         std::vector<EriArgs> args(QBX_N_CLASSES);
         std::vector<int> order;
         double cost[QBX_N_CLASSES] = {};
         for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
-            auto L = std::make_unique<DenseTasks>();
-            TaskCounts& tc = L->tc;
-            task_counts(b, cls, 0.0, QBX_PREC_FP64, 0.0, tc);
-            const int nt = tc.ntb;
-            if (tc.p64[nt] == 0) continue;
-            L->pre.upload(tc.p64, st);
-            L->ko.upload(tc.k64, st);
-            L->cw.upload(tc.w64, st);
+            const RangeCounts r = range_counts(b, cls, 0.0, QBX_PREC_FP64, 0.0);
+            if (r.cnt.empty()) continue;
             EriArgs& a = args[cls] = base_args(b, cls);
-            a.prefix = L->pre.p;
-            a.koff = L->ko.p;
-            a.cpre = L->cw.p;
-            a.total = tc.p64[nt];
-            a.nwave = tc.w64[nt];
-            a.nbra = nt;
+            KetLists L(pool, pair_class(b, cls, 1), pair_class(b, cls, 0).n(), &a.klist, &a.cpre);
+            bra_lists(b, cls, nullptr, r.cnt, L);
+            if (L.total == 0) continue;
+            a.total = L.total;
+            a.nwave = L.nwave;
+            a.nbra = L.nl;
             a.scratch_stream = (void*)st;
             attach_workspace(b, cls, a.nwave, a);
             a.eri = d.p;
-            cost[cls] = class_cost(b, cls, tc);
+            cost[cls] = class_cost(b, cls, r);
             order.push_back(cls);
-            lists.push_back(std::move(L));
         }
+        pool.upload(lists, st);
         ensure_hl_tasks(b, 0.0);
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
         QBX_HIP(hipEventRecord(ctx->ev_fork, st));
@@ -2311,10 +2478,9 @@ int qbx_jk_stats(qbx_ctx* ctx, qbx_basis* b, double thr, double cut, int64_t* sh
         QBX_HIP(hipSetDevice(ctx->device));
         ensure_schwarz(b);
         for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
-            TaskCounts tc;
-            task_counts(b, cls, thr, cut > 0.0 ? QBX_PREC_MIXED : QBX_PREC_FP64, cut, tc);
-            const PairClass& PX = pair_view(b, cls, 0);
-            const PairClass& PY = pair_view(b, cls, 1);
+            const RangeCounts r = range_counts(b, cls, thr, cut > 0.0 ? QBX_PREC_MIXED : QBX_PREC_FP64, cut);
+            const PairClass& PX = pair_class(b, cls, 0);
+            const PairClass& PY = pair_class(b, cls, 1);
             const int nx = PX.n();
             // prefix sums over kets (sorted order) of primitive-pair counts and of
             // unique basis-function pairs (n(n+1)/2 for a diagonal shell pair)
@@ -2332,9 +2498,7 @@ int qbx_jk_stats(qbx_ctx* ctx, qbx_basis* b, double thr, double cut, int64_t* sh
             for (int i = 0; i < nx; ++i)
                 for (int k = 0; k < PY.nbk; ++k) {
                     const int t = i * PY.nbk + k;
-                    const int64_t n64 = tc.p64[t + 1] - tc.p64[t];
-                    const int64_t n32 = tc.p32[t + 1] - tc.p32[t];
-                    const int64_t cnt = n64 + n32;
+                    const int64_t n64 = r.c64()[t], cnt = r.cnt[t];
                     const int s0 = PY.bstart[k];
                     sq += cnt;
                     s64 += n64;
@@ -2647,9 +2811,8 @@ void hf_gradient(qbx_ctx* ctx, qbx_basis* b, const double* Dt, const double* Da,
             a.boysl = boys_order(ctx, lt + 1);
             a.D = dD.p;
             a.nset = uhf ? 2 : 1;
-            a.prefix = t64.prefix.p;
-            a.koff = t64.koff.p;
-            a.cpre = t64.cpre.p;
+            a.klist = t64.klist;
+            a.cpre = t64.cpre;
             a.total = t64.total;
             a.nwave = t64.nwave;
             a.nbra = t64.nbra;

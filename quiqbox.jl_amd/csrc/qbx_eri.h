@@ -34,6 +34,43 @@ namespace qbx {
 template <typename T> using cptr = const __attribute__((address_space(4))) T*;
 template <typename T> __device__ __forceinline__ cptr<T> cst(const T* p) { return (cptr<T>)p; }
 
+// Ket list i (a bra's, or a twin group's): its ranges of the ket buckets, one
+// after another, as nb pairs (first position, ket - position) and the length.
+// Only the list's last chunk of 64 is partial, and most others hold kets of one
+// primitive-pair count.
+struct KetList {
+    cptr<int> r;
+    int nbk, n;
+    __device__ __forceinline__ KetList(const int* klist, int nb, int i)
+        : r(cst(klist) + (size_t)i * (2 * nb + 1)), nbk(nb), n(r[2 * nb]) {}
+    // ket at position 0 <= pos < n
+    __device__ __forceinline__ int ket(int pos) const
+    {
+        int d = r[1];
+        for (int b = 1; b < nbk; ++b) d = pos >= r[2 * b] ? r[2 * b + 1] : d;
+        return pos + d;
+    }
+};
+
+// Items of a K-row task: chunk and range [u0, u0 + un) of the bra's primitive pairs.
+struct RowItem {
+    int chunk, u0, un;
+    __device__ __forceinline__ RowItem(const cptr<RowTask>& t, int j, int bn)
+    {
+        const int parts = t->parts;
+        if (parts == 1) {
+            chunk = t->chunk0 + j;
+            u0 = 0;
+            un = bn;
+        } else {
+            const int c = j / parts, per = (bn + parts - 1) / parts;
+            chunk = t->chunk0 + c;
+            u0 = (j - c * parts) * per;
+            un = min(per, bn - u0);
+        }
+    }
+};
+
 // J/K accumulation.  With per-XCD copies every writer of a copy runs on one
 // XCD, so the add only has to be atomic within that XCD's L2: workgroup scope
 // keeps it there instead of sending each 8-byte add out to memory.
@@ -280,11 +317,11 @@ __global__ __launch_bounds__(eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC)) void er
         const int mid = (lo + hi) >> 1;
         if (cpre[mid] <= wave) lo = mid; else hi = mid;
     }
-    const int tb = lo, bi = tb / a.nbk;
-    const int nk = (int)(cst(a.prefix)[tb + 1] - cst(a.prefix)[tb]);
-    const int pos = (wave - cpre[tb]) * 64 + lane;
-    const bool inrange = pos < nk;
-    const int ki = cst(a.koff)[tb] + (inrange ? pos : 0);
+    const int bi = lo;
+    const KetList kl(a.klist, a.nbk, bi);
+    const int pos = (wave - cpre[bi]) * 64 + lane;
+    const bool inrange = pos < kl.n;
+    const int ki = kl.ket(inrange ? pos : 0);
 
     const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
     const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
@@ -609,8 +646,8 @@ __device__ __forceinline__ void digest_rows(const EriArgs& a, const R* kacc, con
 }
 
 // ---------------------------------------------------------------------------
-// J/K with the bra's K rows in LDS.  A block of ROW_WAVES waves takes one bra
-// and up to ROW_CHUNKS of its 64-ket chunks.  Every K update of a quartet has
+// J/K with the bra's K rows in LDS.  A block of ROW_WAVES waves takes one task
+// (RowTask), its waves every ROW_WAVES-th item.  Every K update of a quartet has
 // one index on the bra (K_ac, K_ad on the rows of A's functions; K_bc, K_bd on
 // B's), so the block sums them in LDS rows [set][A and B functions][N] with
 // LDS atomics and sends each nonzero row element to J/K once, instead of one
@@ -666,18 +703,11 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
 
     const int lane = (int)threadIdx.x & 63;
     const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    // bra and superchunk of this block
-    const cptr<int> spre = cst(a.spre);
-    const int task = (int)blockIdx.x;
-    int lo = 0, hi = a.nbra;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (spre[mid] <= task) lo = mid; else hi = mid;
-    }
-    const int tb = lo, bi = tb / a.nbk;
-    const int sc = task - spre[tb];
-    const int nk = (int)(cst(a.prefix)[tb + 1] - cst(a.prefix)[tb]);
-    const int k0 = cst(a.koff)[tb];
+    const cptr<RowTask> task = cst(a.rtask + blockIdx.x);
+    const int bi = task->list;
+    const KetList kl(a.klist, a.nbk, bi);
+    const cptr<PrimPair> BP = cst(a.pp + cst(a.bra.ppo)[bi]);
+    const int bn = cst(a.bra.ppn)[bi];
     const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
     const cptr<DevShell> SA = cst(a.sh + sA);
     const cptr<DevShell> SB = cst(a.sh + sB);
@@ -690,12 +720,11 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
     for (int n = 0; n < NB; ++n) fb[n] = SB->bf[n] < 0 ? 0 : SB->bf[n];
     const JKSink sink(a);
 
-    for (int r = 0; r < ROW_CHUNKS / ROW_WAVES; ++r) {
-        const int chunk = (sc * (ROW_CHUNKS / ROW_WAVES) + r) * ROW_WAVES + wib;
-        if (chunk * 64 >= nk) break;
-        const int pos = chunk * 64 + lane;
-        const bool inrange = pos < nk;
-        const int ki = k0 + (inrange ? pos : 0);
+    for (int j = task->item0 + wib; j < task->item1; j += ROW_WAVES) {
+        const RowItem it(task, j, bn);
+        const int pos = it.chunk * 64 + lane;
+        const bool inrange = pos < kl.n;
+        const int ki = kl.ket(inrange ? pos : 0);
         const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
         int kn = inrange ? a.ket.ppn[ki] : 0;
         if (a.pdmax) {
@@ -712,8 +741,7 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
         R acc[Cls::NACC];
 #pragma unroll
         for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
-        prim_loop<Cls, LT, R, PREFETCH, -1>(acc, cst(a.pp + cst(a.bra.ppo)[bi]), cst(a.bra.ppn)[bi],
-                                            a.pp + a.ket.ppo[ki], kn, sb);
+        prim_loop<Cls, LT, R, PREFETCH, -1>(acc, BP + it.u0, it.un, a.pp + a.ket.ppo[ki], kn, sb);
         const double* CDp = a.ket.AB + 3 * ki;
         R kacc[Cls::NE * NCD];
         Cls::hrr_ket(acc, kacc, (R)CDp[0], (R)CDp[1], (R)CDp[2]);
@@ -730,13 +758,11 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
 }
 
 // ---------------------------------------------------------------------------
-// J/K for a group of twin bras.  A block of TWIN_WAVES waves takes one group
-// and up to ROW_CHUNKS 64-ket chunks of the union of its members' ket ranges
-// (each member's range is a prefix of the same sorted ket list, or its FP32
-// tail).  The geometry and Boys values of every primitive quartet are computed
-// once, from the first member's primitive pairs; each member accumulates them
-// with its own c_a c_b factor (Kp) where the ket lies in its range.  Each
-// member then goes through the digest with its own shells and LDS K rows
+// J/K for a group of twin bras.  A block of TWIN_WAVES waves takes one task of
+// the group's ket list, the kets that every member keeps.  The geometry and Boys
+// values of every primitive quartet are computed once, from the first member's
+// primitive pairs; each member accumulates them with its own c_a c_b factor (Kp)
+// and goes through the digest with its own shells and LDS K rows
 // [set][member][A and B functions][N].
 // ---------------------------------------------------------------------------
 template <int LA, int LB, int LC, int LD, typename R>
@@ -749,7 +775,6 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
     constexpr int NCD = qbx_ncart(LC) * qbx_ncart(LD);
     constexpr int NROW = NA + NB;
     constexpr int TW = TWIN_MAX;
-    static_assert(ROW_CHUNKS % TWIN_WAVES == 0, "chunks per task must split evenly over the waves");
     __shared__ double2 sboys[BOYS_HEAD2 + boys_rows(LT) * QBX_BOYSL_STRIDE / 2];
     extern __shared__ double krow[];    // [nset][twmax][NROW][N]
     const int Ni = a.N;
@@ -762,31 +787,18 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
 
     const int lane = (int)threadIdx.x & 63;
     const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const cptr<int> gpre = cst(a.gpre);
-    const int task = (int)blockIdx.x;
-    int lo = 0, hi = a.ngroup;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (gpre[mid] <= task) lo = mid; else hi = mid;
-    }
-    const int g = lo;
-    const int sc = task - gpre[g];
-    const cptr<int> gm = cst(a.gmem + 3 * TW * g);
-    int bi[TW], klo[TW], khi[TW], sA[TW], sB[TW], ppo[TW];
-    int ulo = 0x7fffffff, uhi = 0;
+    const cptr<RowTask> task = cst(a.gtask + blockIdx.x);
+    const int g = task->list;
+    const KetList kl(a.gklist, a.nbk, g);
+    const cptr<int> gm = cst(a.gmem + TW * g);
+    int bi[TW], sA[TW], sB[TW], ppo[TW];
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
-        bi[t] = t < tw ? gm[3 * t] : -1;
-        klo[t] = t < tw ? gm[3 * t + 1] : 0;
-        khi[t] = t < tw ? gm[3 * t + 2] : 0;
+        bi[t] = t < tw ? gm[t] : -1;
         const int b = bi[t] < 0 ? bi[0] : bi[t];
         sA[t] = cst(a.bra.shA)[b];
         sB[t] = cst(a.bra.shB)[b];
         ppo[t] = cst(a.bra.ppo)[b];
-        if (bi[t] >= 0 && khi[t] > klo[t]) {
-            ulo = min(ulo, klo[t]);
-            uhi = max(uhi, khi[t]);
-        }
     }
     const int bn = cst(a.bra.ppn)[bi[0]];
     const cptr<PrimPair> BP = cst(a.pp + ppo[0]);
@@ -794,18 +806,17 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
     const R ABx = (R)ABp[0], ABy = (R)ABp[1], ABz = (R)ABp[2];
     const JKSink sink(a);
 
-    for (int r = 0; r < ROW_CHUNKS / TWIN_WAVES; ++r) {
-        const int chunk = (sc * (ROW_CHUNKS / TWIN_WAVES) + r) * TWIN_WAVES + wib;
-        if (ulo >= uhi || ulo + chunk * 64 >= uhi) break;
-        const int pos = ulo + chunk * 64 + lane;
-        const bool inrange = pos < uhi;
-        const int ki = inrange ? pos : ulo;
+    for (int j = task->item0 + wib; j < task->item1; j += TWIN_WAVES) {
+        const RowItem it(task, j, bn);
+        const int pos = it.chunk * 64 + lane;
+        const bool inrange = pos < kl.n;
+        const int ki = kl.ket(inrange ? pos : 0);
         const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
         bool live[TW];
         bool any = false;
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
-            bool l = inrange && bi[t] >= 0 && pos >= klo[t] && pos < khi[t];
+            bool l = inrange && bi[t] >= 0;
             if (l && a.pdmax) {
                 const double* dm = a.pdmax;
                 const int ns = a.nshell;
@@ -828,7 +839,7 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
         const PrimPair* KP = a.pp + a.ket.ppo[ki];
         for (int v = 0; v < kn; ++v) {
             const KetPrim Q = load_ket(KP + v);
-            for (int u = 0; u < bn; ++u) {
+            for (int u = it.u0; u < it.u0 + it.un; ++u) {
                 const double p = BP[u].p, inv2p = BP[u].inv2p;
                 const double PQx = BP[u].Px - Q.Qx, PQy = BP[u].Py - Q.Qy, PQz = BP[u].Pz - Q.Qz;
                 const double pq = p + Q.q;
@@ -887,7 +898,7 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
         const int t = rem / (NROW * Ni);
         rem -= t * NROW * Ni;
         const int row = rem / Ni, col = rem - row * Ni;
-        const int b = gm[3 * t];
+        const int b = gm[t];
         const int sh = row < NA ? cst(a.bra.shA)[b] : cst(a.bra.shB)[b];
         const int fr = max(a.sh[sh].bf[row < NA ? row : row - NA], 0);
         sink.add(sink.K + (size_t)s * N * N + (size_t)fr * N + col, v);
@@ -967,19 +978,18 @@ __device__ __forceinline__ void staged_groups(std::integer_sequence<int, Gs...>,
 // every W-th group, then one W-th of the (a b| rows of the digest); every
 // wave of the block must call with the same task.
 template <int LA, int LB, int LC, int LD, typename R, int MODE, class KOut, int W = 1>
-__device__ __forceinline__ void staged_chunk(const EriArgs& a, int tb, int chunk, int lane, const WsSlot<R>& ws,
-                                             const double* sb, const KOut& kout, int wib = 0)
+__device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, int chunk, int u0, int un, int lane,
+                                             const WsSlot<R>& ws, const double* sb, const KOut& kout, int wib = 0)
 {
     using Cls = EriClass<LA, LB, LC, LD, R>;
     constexpr int NA = qbx_ncart(LA), NB = qbx_ncart(LB), NC = qbx_ncart(LC), ND = qbx_ncart(LD);
     constexpr int LT = LA + LB + LC + LD;
     constexpr int NCD = NC * ND;
     const size_t N = (size_t)a.N;
-    const int bi = tb / a.nbk;
-    const int nk = (int)(cst(a.prefix)[tb + 1] - cst(a.prefix)[tb]);
+    const KetList kl(a.klist, a.nbk, bi);
     const int pos = chunk * 64 + lane;
-    const bool inrange = pos < nk;
-    const int ki = cst(a.koff)[tb] + (inrange ? pos : 0);
+    const bool inrange = pos < kl.n;
+    const int ki = kl.ket(inrange ? pos : 0);
     const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
     const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
     int kn = inrange ? a.ket.ppn[ki] : 0;
@@ -996,7 +1006,7 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int tb, int chunk
 
     const double* CDp = a.ket.AB + 3 * ki;
     staged_groups<Cls, LT, R, W>(std::make_integer_sequence<int, Cls::NGRP>{}, wib,
-                                 cst(a.pp + cst(a.bra.ppo)[bi]), cst(a.bra.ppn)[bi],
+                                 cst(a.pp + cst(a.bra.ppo)[bi]) + u0, un,
                                  a.pp + a.ket.ppo[ki], kn, sb, (R)CDp[0], (R)CDp[1], (R)CDp[2], ws);
     if constexpr (W > 1) {
         static_assert(MODE == MODE_JK, "split staged tasks digest J/K only");
@@ -1193,7 +1203,7 @@ void eri_staged_kernel(EriArgs a)
             const int mid = (lo + hi) >> 1;
             if (cpre[mid] <= wave) lo = mid; else hi = mid;
         }
-        staged_chunk<LA, LB, LC, LD, R, MODE>(a, lo, wave - cpre[lo], lane, ws, sb, kout);
+        staged_chunk<LA, LB, LC, LD, R, MODE>(a, lo, wave - cpre[lo], 0, cst(a.bra.ppn)[lo], lane, ws, sb, kout);
     }
 }
 
@@ -1227,14 +1237,14 @@ void eri_staged_split_kernel(EriArgs a)
             const int mid = (lo + hi) >> 1;
             if (cpre[mid] <= task) lo = mid; else hi = mid;
         }
-        staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToGlobal, W>(a, lo, task - cpre[lo], lane, ws, sb, kout, wib);
+        staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToGlobal, W>(a, lo, task - cpre[lo], 0, cst(a.bra.ppn)[lo], lane, ws,
+                                                               sb, kout, wib);
         __syncthreads();    // the slot is rewritten by the next task
     }
 }
 
 // Staged J/K with the bra's K rows in LDS: a persistent grid of blocks, each
-// taking one (bra, up to a.tchunks chunks) task at a time; its waves share
-// the task's chunks, K goes to the rows, and the rows are flushed to K once
+// taking one task (RowTask) at a time; its waves share the task's items, K goes to the rows, and the rows are flushed to K once
 // per task.
 template <int LA, int LB, int LC, int LD, typename R>
 __global__ __launch_bounds__(64 * STAGE_WAVES_PER_BLOCK) __attribute__((amdgpu_waves_per_eu(EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD, EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD)))
@@ -1259,24 +1269,16 @@ void eri_staged_rows_kernel(EriArgs a)
     const int lane = (int)threadIdx.x & 63;
     const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const WsSlot<R> ws((R*)a.ws + (size_t)((int)blockIdx.x * W + wib) * WSV * 64, WSV, lane);
-    const cptr<int> spre = cst(a.spre);
     const JKSink sink(a);
     const KToRows<NROW> kout{krow, Ni};
 
-    for (int task = (int)blockIdx.x; task < a.nsuper; task += (int)gridDim.x) {
-        int lo = 0, hi = a.nbra;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (spre[mid] <= task) lo = mid; else hi = mid;
-        }
-        const int tb = lo, bi = tb / a.nbk;
-        const int sc = task - spre[tb];
-        const int nk = (int)(cst(a.prefix)[tb + 1] - cst(a.prefix)[tb]);
-        // wave wib takes chunks wib, wib + W, ... of the task's a.tchunks
-        for (int j = wib; j < a.tchunks; j += W) {
-            const int chunk = sc * a.tchunks + j;
-            if (chunk * 64 >= nk) break;
-            staged_chunk<LA, LB, LC, LD, R, MODE_JK>(a, tb, chunk, lane, ws, sb, kout);
+    for (int t = (int)blockIdx.x; t < a.nsuper; t += (int)gridDim.x) {
+        const cptr<RowTask> task = cst(a.rtask + t);
+        const int bi = task->list, bn = cst(a.bra.ppn)[bi];
+        // wave wib takes items wib, wib + W, ... of the task
+        for (int j = task->item0 + wib; j < task->item1; j += W) {
+            const RowItem it(task, j, bn);
+            staged_chunk<LA, LB, LC, LD, R, MODE_JK>(a, bi, it.chunk, it.u0, it.un, lane, ws, sb, kout);
         }
         __syncthreads();
         const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
@@ -1287,9 +1289,8 @@ void eri_staged_rows_kernel(EriArgs a)
 
 // Staged J/K with the bra's K rows in LDS and each 64-ket chunk shared by
 // the Cls::SPLIT waves of a block (groups, then digest rows, spread over the
-// waves; one workspace slot per block).  A task is one (bra, up to
-// a.tchunks chunks) range, its chunks taken one after another by the
-// whole block, so no wave idles when a bra has fewer chunks than the block
+// waves; one workspace slot per block).  A task's items are taken one after
+// another by the whole block, so no wave idles when a bra has fewer chunks than the block
 // has waves; the rows are flushed to K once per task.
 template <int LA, int LB, int LC, int LD, typename R>
 __global__ __launch_bounds__((64 * EriClass<LA, LB, LC, LD, R>::SPLIT)) __attribute__((amdgpu_waves_per_eu(EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD, EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD)))
@@ -1314,24 +1315,17 @@ void eri_staged_split_rows_kernel(EriArgs a)
     const int lane = (int)threadIdx.x & 63;
     const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const WsSlot<R> ws((R*)a.ws + (size_t)blockIdx.x * WSV * 64, WSV, lane);
-    const cptr<int> spre = cst(a.spre);
     const JKSink sink(a);
     const KToRows<NROW> kout{krow, Ni};
 
-    for (int task = (int)blockIdx.x; task < a.nsuper; task += (int)gridDim.x) {
-        int lo = 0, hi = a.nbra;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (spre[mid] <= task) lo = mid; else hi = mid;
-        }
-        const int tb = lo, bi = tb / a.nbk;
-        const int sc = task - spre[tb];
-        const int nk = (int)(cst(a.prefix)[tb + 1] - cst(a.prefix)[tb]);
-        for (int r = 0; r < a.tchunks; ++r) {
-            const int chunk = sc * a.tchunks + r;
-            if (chunk * 64 >= nk) break;
-            staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToRows<NROW>, W>(a, tb, chunk, lane, ws, sb, kout, wib);
-            __syncthreads();    // the slot is rewritten by the next chunk
+    for (int t = (int)blockIdx.x; t < a.nsuper; t += (int)gridDim.x) {
+        const cptr<RowTask> task = cst(a.rtask + t);
+        const int bi = task->list, bn = cst(a.bra.ppn)[bi];
+        for (int j = task->item0; j < task->item1; ++j) {
+            const RowItem it(task, j, bn);
+            staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToRows<NROW>, W>(a, bi, it.chunk, it.u0, it.un, lane, ws, sb, kout,
+                                                                       wib);
+            __syncthreads();    // the slot is rewritten by the next item
         }
         const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
         flush_rows<NA, TPB>(krow, nrowel, NROW, Ni, a.sh[sA].bf, a.sh[sB].bf, sink, true);
@@ -1410,7 +1404,7 @@ void launch_eri(const EriArgs& a, hipStream_t s)
                 (void)hipGetLastError();
                 return ok;
             }();
-            if ((EriClass<LA, LB, LC, LD, R>::SPLIT == 1 || !a.split) && rows_ok && a.spre &&
+            if ((EriClass<LA, LB, LC, LD, R>::SPLIT == 1 || !a.split) && rows_ok && a.rtask &&
                 shm <= (size_t)ROW_LDS_MAX && shm + boys_lds <= (size_t)a.lds_max) {
                 if (a.nsuper <= 0) return;
                 const int max_blocks = a.ws_slots / STAGE_WAVES_PER_BLOCK;
@@ -1433,7 +1427,7 @@ void launch_eri(const EriArgs& a, hipStream_t s)
                 (void)hipGetLastError();
                 return ok;
             }();
-            if (a.split && srows_ok && a.spre && shm <= (size_t)ROW_LDS_MAX && shm + boys_lds <= (size_t)a.lds_max) {
+            if (a.split && srows_ok && a.rtask && shm <= (size_t)ROW_LDS_MAX && shm + boys_lds <= (size_t)a.lds_max) {
                 if (a.nsuper <= 0) return;
                 // one slot per block
                 const int blocks = a.nsuper < a.ws_slots ? a.nsuper : a.ws_slots;
@@ -1494,7 +1488,7 @@ void launch_eri(const EriArgs& a, hipStream_t s)
                 (void)hipGetLastError();
                 return ok;
             }();
-            if (rows_ok && a.spre && shm <= (size_t)ROW_LDS_MAX && shm + boys_lds <= (size_t)a.lds_max) {
+            if (rows_ok && a.rtask && shm <= (size_t)ROW_LDS_MAX && shm + boys_lds <= (size_t)a.lds_max) {
                 if (a.nsuper <= 0) return;
                 static const size_t scratch = [] {
                     hipFuncAttributes fa;

@@ -7,22 +7,28 @@
 namespace qbx {
 enum EriMode { MODE_JK = 0, MODE_DENSE = 1, MODE_SCHWARZ = 2 };
 
-// J/K kernel with the bra's K rows in LDS: ROW_WAVES waves per block, up to
-// ROW_CHUNKS chunks of 64 kets of one bra per block, at most ROW_LDS_MAX bytes
-// of rows (larger bases use the one-wave-per-chunk kernel).
+// J/K kernel with the bra's K rows in LDS: ROW_WAVES waves per block, at most
+// ROW_LDS_MAX bytes of rows (larger bases use the one-wave-per-chunk kernel).
 #ifndef QBX_ROW_WAVES
 #define QBX_ROW_WAVES 4
 #endif
 constexpr int ROW_WAVES = QBX_ROW_WAVES;
-// Chunks per task of the low-L K-row and twin kernels: fewer, larger tasks
-// (fewer K-row flushes) measured 50.9 -> 49.6 ms per Fock build of 24 H2O in
-// cc-pVDZ at 32 instead of 16, the 592-function cluster unchanged; at 64 the
-// cluster lost (38.6 -> 39.4 ms).
-constexpr int ROW_CHUNKS = 32;
-// Chunks per task of the staged K-row kernel: its waves are long, and smaller
-// tasks balance better (592-function cluster: (dp|pp) 5.05 -> 4.33 ms, build
-// 41.0 -> 40.1 ms against 16; water's low-L classes lost 4% at 8).
-constexpr int STAGED_ROW_CHUNKS = 8;
+// One K-row task (one block): items item0 .. item1 - 1 of a list (a bra, or a
+// group of twin bras).  Item j is the 64-ket chunk chunk0 + j / parts with part
+// j % parts of the bra's primitive pairs: the digest is linear in the integrals,
+// so the waves that share a heavy chunk each digest the integrals of their own
+// primitive pairs.
+struct RowTask {
+    int list, chunk0, parts, item0, item1;
+};
+// Most items per task of the low-L K-row and twin kernels, and of the staged
+// K-row kernel (whose waves are long, so that smaller tasks balance better).
+// Fewer and larger tasks flush fewer K rows: with chunks alone as items, 24 H2O
+// in cc-pVDZ took 50.9 ms per build at 16 and 49.6 at 32, the 592-function
+// cluster lost at 64 (38.6 -> 39.4 ms), and its (dp|pp) took 5.05 ms at 16 and
+// 4.33 at 8.
+constexpr int ROW_ITEMS = 32;
+constexpr int STAGED_ROW_ITEMS = 8;
 constexpr int ROW_LDS_MAX = 64 * 1024;
 // Twin bras: shell pairs of one pair class with the same primitive geometry
 // and primitive pairs, differing only in contraction coefficients (shells
@@ -50,18 +56,17 @@ struct EriArgs {
     const double* boys;
     const double* bexp;
     const double* boysl;      // per-order Boys rows of the class's total L
-    const int64_t* prefix;    // [nbra+1] prefix over bras of the screened ket counts
-    const int* koff;          // [nbra] first ket of each bra
+    const int* klist;         // [nbra][2 nbk + 1]: ket lists of the bras (KetList)
     const int* cpre;          // [nbra+1] prefix over bras of ceil(kets / 64): waves
-    const int* spre;          // [nbra+1] prefix over bras of ceil(waves / tchunks): K-row blocks
-    int nsuper;               // number of K-row blocks
-    int tchunks;              // chunks per K-row task of the staged kernels (spre)
-    const int* gpre;          // [ngroup+1] twin groups: prefix of tasks (ROW_CHUNKS chunks of the union range)
-    const int* gmem;          // [ngroup][TWIN_MAX][3]: bra, first ket, end of kets (bra < 0: no member)
+    const RowTask* rtask;     // K-row tasks of the bras (null: the one-wave-per-chunk kernels run)
+    int nsuper;               // their number
+    const int* gklist;        // [ngroup][2 nbk + 1]: ket lists of the twin groups
+    const int* gmem;          // [ngroup][TWIN_MAX] bras of a group (-1: no member)
+    const RowTask* gtask;     // tasks of the twin groups
     int ngroup;               // twin groups of this class (0: none)
     int ntwtask;              // their tasks
     int twmax;                // largest group (LDS rows per set)
-    int nbk;                  // ket buckets per bra: task t is bra t / nbk, bucket t % nbk
+    int nbk;                  // ket buckets of the class
     int lds_max;              // LDS bytes a block may use on this device
     int64_t total;            // Schwarz mode: number of diagonal pairs
     int nwave;                // J/K and dense modes: number of waves
