@@ -96,6 +96,12 @@ constexpr int kStageSlots = 2048;
 // by at most 3e-12, their energies by 3e-11 Eh; the water build has 20%
 // fewer primitive quartets.
 constexpr double QBX_PRIM_PAIR_CUT = 1e-20;
+// Basis functions from which J's ket sums go through the pair-order buffer
+// (JKSink::add_ket).  Water boxes in cc-pVDZ: 100 functions 967 -> 961 us per
+// build, 250 3740 -> 3610, 600 35.3 -> 32.6 ms; at 25 and 50 functions the
+// kernel that adds the sums to J costs what the atomics gain (771 against 773,
+// 796 against 804 us).
+constexpr int kPairSumMin = 64;
 // Ket buckets.  A wave's lanes take consecutive kets of one bra and the wave
 // runs as long as its lane with the most primitive pairs; in Schwarz order,
 // contracted core pairs (81 primitive pairs in cc-pVDZ oxygen) sit among
@@ -271,7 +277,7 @@ struct qbx_basis {
     DevBuf<int> d_lists;       // their arrays
     DevBuf<double> ws[QBX_N_CLASSES];   // staged-class workspaces
     // work buffers
-    DevBuf<double> d_D, d_J, d_K, d_G;
+    DevBuf<double> d_D, d_JK, d_G;   // d_JK: J, K, and the ket sums in pair order
     DevBuf<double> d_pdmax;        // shell-pair max |D| for density screening
     // end of the last Fock build (recorded on its stream after the
     // symmetrization) and that stream: a build on another stream, and every
@@ -667,6 +673,37 @@ __global__ void symmetrize_kernel(const double* J, const double* K, double* G, i
         v += 0.5 * (Js[i * N + j] + Js[j * N + i]) - 0.5 * (Ks[i * N + j] + Ks[j * N + i]);
     }
     G[g] = v;
+}
+
+// Ket sums in pair order (the blocks of the low pair classes one after another,
+// each [component][pair]; `copies` copies of nset sets), added to J (copy 0).
+// Every element of J belongs to one component of one pair.
+struct KetSumArgs {
+    size_t at[QBX_N_LOW_PAIR_CLASSES + 1];
+    const int* shA[QBX_N_LOW_PAIR_CLASSES];
+    const int* shB[QBX_N_LOW_PAIR_CLASSES];
+    int n[QBX_N_LOW_PAIR_CLASSES], nb[QBX_N_LOW_PAIR_CLASSES];
+    const DevShell* sh;
+    const double* jp;
+    double* J;
+    int N, nset, copies;
+};
+
+__global__ void ket_sum_kernel(KetSumArgs a)
+{
+    const size_t total = a.at[QBX_N_LOW_PAIR_CLASSES];
+    const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= total * a.nset) return;
+    const size_t s = g / total, e = g - s * total;
+    int c = 0;
+    while (e >= a.at[c + 1]) ++c;
+    const size_t r = e - a.at[c];
+    const int cd = (int)(r / a.n[c]), k = (int)(r - (size_t)cd * a.n[c]);
+    const int fa = a.sh[a.shA[c][k]].bf[cd / a.nb[c]], fb = a.sh[a.shB[c][k]].bf[cd % a.nb[c]];
+    if (fa < 0 || fb < 0) return;
+    double v = 0.0;
+    for (int i = 0; i < a.copies; ++i) v += a.jp[((size_t)i * a.nset + s) * total + e];
+    a.J[(s * a.N + fa) * a.N + fb] += v;
 }
 
 // Which XCD runs each block (one write per block).
@@ -1575,10 +1612,23 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
     ensure_hl_tasks(b, thr);
     const size_t NN = (size_t)b->nbf * b->nbf;
     const int copies = ctx->xcd_local ? QBX_MAX_XCD : 1;
-    b->d_J.ensure(NN * nset * copies);
-    b->d_K.ensure(NN * nset * copies);
-    zero_async(b->d_J.p, NN * nset * copies, st);
-    zero_async(b->d_K.p, NN * nset * copies, st);
+    KetSumArgs ks;
+    ks.at[0] = 0;
+    for (int c = 0; c < QBX_N_LOW_PAIR_CLASSES; ++c) {
+        const PairClass& P = b->pc[c];
+        ks.n[c] = P.n();
+        ks.nb[c] = qbx_ncart(qbx_pair_class_l[c][1]);
+        ks.shA[c] = P.d_shA.p;
+        ks.shB[c] = P.d_shB.p;
+        ks.at[c + 1] = ks.at[c] + (size_t)P.n() * qbx_ncart(qbx_pair_class_l[c][0]) * ks.nb[c];
+    }
+    const size_t npair_el = b->nbf >= kPairSumMin ? ks.at[QBX_N_LOW_PAIR_CLASSES] : 0;
+    const size_t jk_el = NN * nset * copies, jp_el = npair_el * nset * copies;
+    b->d_JK.ensure(2 * jk_el + jp_el);
+    double* const dJ = b->d_JK.p;
+    double* const dK = dJ + jk_el;
+    double* const dP = dK + jk_el;
+    zero_async(b->d_JK.p, 2 * jk_el + jp_el, st);
     // timing 1: every class on the main stream, one after another, bracketed
     // by events; timing 2: the concurrent build as it runs untimed, each
     // class bracketed by events on the stream it is launched on
@@ -1616,10 +1666,13 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
         a.nshell = ns;
         a.dthr = ctx->density_thr;
         a.D = dD;
-        a.J = b->d_J.p;
-        a.K = b->d_K.p;
+        a.J = dJ;
+        a.K = dK;
         a.xcd_local = ctx->xcd_local ? 1 : 0;
         a.jk_stride = NN * nset;
+        a.jp = npair_el > 0 ? dP + ks.at[class_pc(cls, 1)] : nullptr;
+        a.jp_set = npair_el;
+        a.jp_stride = npair_el * nset;
         a.nset = nset;
         // twin groups where their LDS rows ([set][member][A and B][N]) fit a block
         bool twin = b->use_twin[cls] && ctx->jk_rows;
@@ -1677,8 +1730,8 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
     if (b->has_high)
         launch_high(b, MODE_JK, fork ? ctx->aux : &st, fork ? kStreams : 1, [&](GenArgs& g) {
             g.D = dD;
-            g.J = b->d_J.p;
-            g.K = b->d_K.p;
+            g.J = dJ;
+            g.K = dK;
             g.xcd_local = ctx->xcd_local ? 1 : 0;
             g.jk_stride = NN * nset;
             g.nset = nset;
@@ -1705,9 +1758,19 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
             QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
         }
     }
+    if (npair_el > 0) {
+        ks.sh = b->d_sh.p;
+        ks.jp = dP;
+        ks.J = dJ;
+        ks.N = b->nbf;
+        ks.nset = nset;
+        ks.copies = copies;
+        hipLaunchKernelGGL(ket_sum_kernel, dim3((unsigned)((npair_el * nset + 255) / 256)), dim3(256), 0, st, ks);
+        QBX_HIP(hipGetLastError());
+    }
     const size_t tot = NN * nset;
     hipLaunchKernelGGL(symmetrize_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st,
-                       b->d_J.p, b->d_K.p, dG, b->nbf, nset, copies);
+                       dJ, dK, dG, b->nbf, nset, copies);
     QBX_HIP(hipGetLastError());
     QBX_HIP(hipEventRecord(b->ev_done, st));
     b->last_stream = st;

@@ -77,13 +77,26 @@ struct RowItem {
 struct JKSink {
     double* J;
     double* K;
+    double* P;          // ket sums in pair order, or null
+    size_t pset;
+    int npair;
     bool local;
     __device__ __forceinline__ JKSink(const EriArgs& a)
     {
         local = a.xcd_local != 0;
-        const size_t off = local ? (size_t)qbx_xcc_id() * a.jk_stride : 0;
-        J = a.J + off;
-        K = a.K + off;
+        const size_t copy = local ? (size_t)qbx_xcc_id() : 0;
+        J = a.J + copy * a.jk_stride;
+        K = a.K + copy * a.jk_stride;
+        P = a.jp ? a.jp + copy * a.jp_stride : nullptr;
+        pset = a.jp_set;
+        npair = a.ket.n;
+    }
+    // J_cd of component cd of ket ki: in pair order the 64 lanes' kets are
+    // neighbours, so a wave's atomics go to a few cache lines; in J every lane's
+    // element lies on its own line (24 H2O in cc-pVDZ: (ps|ps) 5.6 -> 4.2 ms).
+    __device__ __forceinline__ void add_ket(int s, int cd, int ki, double* Jcd, double v) const
+    {
+        add(P ? P + s * pset + (size_t)cd * npair + ki : Jcd, v);
     }
     __device__ __forceinline__ void add(double* p, double v) const
     {
@@ -484,7 +497,7 @@ __global__ __launch_bounds__(eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC)) void er
 #pragma unroll
             for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
-                for (int id = 0; id < ND; ++id) sink.add(Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
+                for (int id = 0; id < ND; ++id) sink.add_ket(s, ic * ND + id, ki, Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
 #pragma unroll
             for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -543,8 +556,8 @@ __device__ __forceinline__ void flush_rows(double* krow, int nrowel, int nrow, i
 // B functions][N].  f is the quartet's degeneracy weight (0 for dead lanes).
 template <int LA, int LB, int LC, int LD, typename R>
 __device__ __forceinline__ void digest_rows(const EriArgs& a, const R* kacc, const int* fa, const int* fb,
-                                            cptr<DevShell> SA, cptr<DevShell> SB, R ABx, R ABy, R ABz, int sC,
-                                            int sD, double f, bool live, double* rows0, int rstride,
+                                            cptr<DevShell> SA, cptr<DevShell> SB, R ABx, R ABy, R ABz, int ki,
+                                            int sC, int sD, double f, bool live, double* rows0, int rstride,
                                             const JKSink& sink, int lane)
 {
     using Cls = EriClass<LA, LB, LC, LD, R>;
@@ -632,7 +645,7 @@ __device__ __forceinline__ void digest_rows(const EriArgs& a, const R* kacc, con
 #pragma unroll
             for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
-                for (int id = 0; id < ND; ++id) sink.add(Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
+                for (int id = 0; id < ND; ++id) sink.add_ket(s, ic * ND + id, ki, Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
 #pragma unroll
             for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -750,7 +763,7 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
         if (sA == sB) f *= 0.5;
         if (sC == sD) f *= 0.5;
         if (a.same && bi == ki) f *= 0.5;
-        digest_rows<LA, LB, LC, LD, R>(a, kacc, fa, fb, SA, SB, ABx, ABy, ABz, sC, sD, f, live, krow, NROW * Ni,
+        digest_rows<LA, LB, LC, LD, R>(a, kacc, fa, fb, SA, SB, ABx, ABy, ABz, ki, sC, sD, f, live, krow, NROW * Ni,
                                        sink, lane);
     }
     __syncthreads();
@@ -883,7 +896,7 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
             if (sA[t] == sB[t]) f *= 0.5;
             if (sC == sD) f *= 0.5;
             if (a.same && bi[t] == ki) f *= 0.5;
-            digest_rows<LA, LB, LC, LD, R>(a, kacc, fa, fb, SA, SB, ABx, ABy, ABz, sC, sD, f, live[t],
+            digest_rows<LA, LB, LC, LD, R>(a, kacc, fa, fb, SA, SB, ABx, ABy, ABz, ki, sC, sD, f, live[t],
                                            krow + t * NROW * Ni, tw * NROW * Ni, sink, lane);
         }
     }
@@ -1171,7 +1184,7 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, int chunk
 #pragma unroll
             for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
-                for (int id = 0; id < ND; ++id) sink.add(Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
+                for (int id = 0; id < ND; ++id) sink.add_ket(s, ic * ND + id, ki, Js + fc[ic] * N + fd[id], fj * jcd[ic * ND + id]);
         }
     }
 }

@@ -80,6 +80,10 @@ struct EriArgs {
     // atomics, which the XCD's L2 resolves; otherwise one copy, device scope
     int xcd_local;
     size_t jk_stride;
+    // ket sums J_cd in pair order (null: straight to J): the ket class's block
+    // [component cd][pair], per density set (stride jp_set) and copy (jp_stride)
+    double* jp;
+    size_t jp_set, jp_stride;
     int nset;
     int N;
     double* eri;       // dense mode, N^4
