@@ -1220,7 +1220,7 @@ public:
         if (bn <= 0) return;
         const int nbk = ket_.nbk;
         const Cut* cut = cuts(bn);
-        RowTask cur{list, 0, 0, 0, 0};
+        RowTask cur{list, 0, 0, 0, 0, 0};
         double cost = 0.0;
         auto close = [&] {
             if (cur.item1 > cur.item0) out.push_back(cur);
@@ -1233,11 +1233,11 @@ public:
             const int end = ((k + 1 < nbk ? kl[2 * (k + 1)] : kl[2 * nbk]) + 63) / 64;
             if (end <= chunk) continue;
             const Cut& c = cut[k];
-            if (c.parts != cur.parts) {
+            if (c.kparts != cur.kparts || c.bparts != cur.bparts) {
                 close();
-                cur = RowTask{list, chunk, c.parts, 0, 0};
+                cur = RowTask{list, chunk, c.kparts, c.bparts, 0, 0};
             }
-            int left = (end - chunk) * c.parts;
+            int left = (end - chunk) * c.kparts * c.bparts;
             while (left > 0) {
                 const int have = cur.item1 - cur.item0;
                 const int fit = (int)std::min((double)max_items_, std::max(1.0, (waves_ * cap_.task - cost) * c.inv));
@@ -1256,7 +1256,7 @@ public:
 private:
     // parts of a chunk of one ket bucket, cost of an item and its inverse
     struct Cut {
-        int parts;
+        int kparts, bparts;
         double cost, inv;
     };
     const Cut* cuts(int bn)
@@ -1265,10 +1265,18 @@ private:
         if (v.empty())
             for (int top : ket_.btop) {
                 const double whole = (double)bn * top * cp_;
-                const int want = std::max(1, (int)std::min((double)bn, whole / cap_.item + 0.5));
-                const int per = (bn + want - 1) / want, parts = (bn + per - 1) / per;
-                const double c = whole / parts + cq_;
-                v.push_back({parts, c, 1.0 / c});
+                // n things cut into about m equal parts: their number
+                auto cut = [](int n, int m) {
+                    const int per = (n + m - 1) / m;
+                    return (n + per - 1) / per;
+                };
+                // the bra's primitive pairs first, down to 4 (a ket's pair is loaded
+                // once for all of them), then the ket's
+                const int want = std::max(1, (int)std::min((double)bn * top, whole / cap_.item + 0.5));
+                const int bparts = cut(bn, std::min(want, std::max(1, bn / 4)));
+                const int kparts = cut(std::max(top, 1), std::min(std::max(top, 1), (want + bparts / 2) / bparts));
+                const double c = whole / (kparts * bparts) + cq_;
+                v.push_back({kparts, bparts, c, 1.0 / c});
             }
         return v.data();
     }
@@ -1358,7 +1366,10 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
         const RangeCounts& r = rc[cls];
         const int X = class_pc(cls, 0);
         const TaskCaps cap = task_caps(cls, b->class_cost[cls], total);
-        auto add = [&](TaskSet& t, const int* lo, const std::vector<int>& hi) {
+        // whole chunks in the FP32 lists: an FP32 integral is one sum, its
+        // rounding the same whatever else the lists hold
+        const TaskCaps whole = {HUGE_VAL, cap.task};
+        auto add = [&](TaskSet& t, const int* lo, const std::vector<int>& hi, const TaskCaps& cap) {
             KetLists L(pool, pair_class(b, cls, 1), pair_class(b, cls, 0).n(), &t.klist, &t.cpre);
             bra_lists(b, cls, lo, hi, L);
             const std::vector<RowTask> tasks = row_tasks(b, cls, L, cap);
@@ -1368,8 +1379,8 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
             t.nwave = L.nwave;
             t.nbra = L.nl;
         };
-        add(b->t64[cls], nullptr, r.c64());
-        if (mode == QBX_PREC_MIXED) add(b->t32[cls], r.c64().data(), r.cnt);
+        add(b->t64[cls], nullptr, r.c64(), cap);
+        if (mode == QBX_PREC_MIXED) add(b->t32[cls], r.c64().data(), r.cnt, whole);
         b->use_twin[cls] = false;
         // only where bra and ket classes differ: within one pair class a bra's
         // kets end at its own Schwarz-sorted position, so the members' common
@@ -1380,7 +1391,7 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
             std::vector<int> start64(r.cnt.size(), 0);
             add_twins(b, cls, r, cap, pool, b->w64[cls], start64);
             if (b->w64[cls].ngroup > 0) {
-                add(b->s64[cls], start64.data(), r.c64());
+                add(b->s64[cls], start64.data(), r.c64(), cap);
                 b->use_twin[cls] = true;
             }
         }

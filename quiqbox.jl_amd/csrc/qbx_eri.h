@@ -52,21 +52,34 @@ struct KetList {
     }
 };
 
-// Items of a K-row task: chunk and range [u0, u0 + un) of the bra's primitive pairs.
+// Item of a K-row task: its chunk, the range [u0, u0 + un) of the bra's primitive
+// pairs and part kpart of kparts of each ket's.
 struct RowItem {
-    int chunk, u0, un;
+    int chunk, u0, un, kpart, kparts;
     __device__ __forceinline__ RowItem(const cptr<RowTask>& t, int j, int bn)
+        : chunk(t->chunk0 + j), u0(0), un(bn), kpart(0), kparts(t->kparts)
     {
-        const int parts = t->parts;
-        if (parts == 1) {
-            chunk = t->chunk0 + j;
-            u0 = 0;
-            un = bn;
-        } else {
-            const int c = j / parts, per = (bn + parts - 1) / parts;
+        const int bparts = t->bparts, parts = kparts * bparts;
+        if (parts > 1) {
+            const int c = j / parts, r = j - c * parts, iu = r / kparts;
+            const int per = (bn + bparts - 1) / bparts;
             chunk = t->chunk0 + c;
-            u0 = (j - c * parts) * per;
+            u0 = iu * per;
             un = min(per, bn - u0);
+            kpart = r - iu * kparts;
+        }
+    }
+    // the whole chunk
+    __device__ __forceinline__ RowItem(int chunk, int bn) : chunk(chunk), u0(0), un(bn), kpart(0), kparts(1) {}
+    // this item's share of a ket's kn primitive pairs: first one and number
+    __device__ __forceinline__ void ket_part(int kn, int& v0, int& vn) const
+    {
+        v0 = 0;
+        vn = kn;
+        if (kparts > 1) {
+            const int per = (kn + kparts - 1) / kparts;
+            v0 = min(kpart * per, kn);
+            vn = min(per, kn - v0);
         }
     }
 };
@@ -754,7 +767,9 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
         R acc[Cls::NACC];
 #pragma unroll
         for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
-        prim_loop<Cls, LT, R, PREFETCH, -1>(acc, BP + it.u0, it.un, a.pp + a.ket.ppo[ki], kn, sb);
+        int v0, vn;
+        it.ket_part(kn, v0, vn);
+        prim_loop<Cls, LT, R, PREFETCH, -1>(acc, BP + it.u0, it.un, a.pp + a.ket.ppo[ki] + v0, vn, sb);
         const double* CDp = a.ket.AB + 3 * ki;
         R kacc[Cls::NE * NCD];
         Cls::hrr_ket(acc, kacc, (R)CDp[0], (R)CDp[1], (R)CDp[2]);
@@ -849,8 +864,10 @@ __global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
         for (int t = 0; t < TW; ++t)
 #pragma unroll
             for (int n = 0; n < Cls::NACC; ++n) acc[t][n] = (R)0;
-        const PrimPair* KP = a.pp + a.ket.ppo[ki];
-        for (int v = 0; v < kn; ++v) {
+        int v0, vn;
+        it.ket_part(kn, v0, vn);
+        const PrimPair* KP = a.pp + a.ket.ppo[ki] + v0;
+        for (int v = 0; v < vn; ++v) {
             const KetPrim Q = load_ket(KP + v);
             for (int u = it.u0; u < it.u0 + it.un; ++u) {
                 const double p = BP[u].p, inv2p = BP[u].inv2p;
@@ -991,7 +1008,7 @@ __device__ __forceinline__ void staged_groups(std::integer_sequence<int, Gs...>,
 // every W-th group, then one W-th of the (a b| rows of the digest); every
 // wave of the block must call with the same task.
 template <int LA, int LB, int LC, int LD, typename R, int MODE, class KOut, int W = 1>
-__device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, int chunk, int u0, int un, int lane,
+__device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, const RowItem& it, int lane,
                                              const WsSlot<R>& ws, const double* sb, const KOut& kout, int wib = 0)
 {
     using Cls = EriClass<LA, LB, LC, LD, R>;
@@ -1000,7 +1017,7 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, int chunk
     constexpr int NCD = NC * ND;
     const size_t N = (size_t)a.N;
     const KetList kl(a.klist, a.nbk, bi);
-    const int pos = chunk * 64 + lane;
+    const int pos = it.chunk * 64 + lane;
     const bool inrange = pos < kl.n;
     const int ki = kl.ket(inrange ? pos : 0);
     const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
@@ -1017,10 +1034,12 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, int chunk
     if (__ballot(kn > 0) == 0) return;
     const bool live = kn > 0;
 
+    int v0, vn;
+    it.ket_part(kn, v0, vn);
     const double* CDp = a.ket.AB + 3 * ki;
     staged_groups<Cls, LT, R, W>(std::make_integer_sequence<int, Cls::NGRP>{}, wib,
-                                 cst(a.pp + cst(a.bra.ppo)[bi]) + u0, un,
-                                 a.pp + a.ket.ppo[ki], kn, sb, (R)CDp[0], (R)CDp[1], (R)CDp[2], ws);
+                                 cst(a.pp + cst(a.bra.ppo)[bi]) + it.u0, it.un,
+                                 a.pp + a.ket.ppo[ki] + v0, vn, sb, (R)CDp[0], (R)CDp[1], (R)CDp[2], ws);
     if constexpr (W > 1) {
         static_assert(MODE == MODE_JK, "split staged tasks digest J/K only");
         __syncthreads();    // every group's [e|cd) is in the slot
@@ -1216,7 +1235,7 @@ void eri_staged_kernel(EriArgs a)
             const int mid = (lo + hi) >> 1;
             if (cpre[mid] <= wave) lo = mid; else hi = mid;
         }
-        staged_chunk<LA, LB, LC, LD, R, MODE>(a, lo, wave - cpre[lo], 0, cst(a.bra.ppn)[lo], lane, ws, sb, kout);
+        staged_chunk<LA, LB, LC, LD, R, MODE>(a, lo, RowItem(wave - cpre[lo], cst(a.bra.ppn)[lo]), lane, ws, sb, kout);
     }
 }
 
@@ -1250,7 +1269,7 @@ void eri_staged_split_kernel(EriArgs a)
             const int mid = (lo + hi) >> 1;
             if (cpre[mid] <= task) lo = mid; else hi = mid;
         }
-        staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToGlobal, W>(a, lo, task - cpre[lo], 0, cst(a.bra.ppn)[lo], lane, ws,
+        staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToGlobal, W>(a, lo, RowItem(task - cpre[lo], cst(a.bra.ppn)[lo]), lane, ws,
                                                                sb, kout, wib);
         __syncthreads();    // the slot is rewritten by the next task
     }
@@ -1291,7 +1310,7 @@ void eri_staged_rows_kernel(EriArgs a)
         // wave wib takes items wib, wib + W, ... of the task
         for (int j = task->item0 + wib; j < task->item1; j += W) {
             const RowItem it(task, j, bn);
-            staged_chunk<LA, LB, LC, LD, R, MODE_JK>(a, bi, it.chunk, it.u0, it.un, lane, ws, sb, kout);
+            staged_chunk<LA, LB, LC, LD, R, MODE_JK>(a, bi, it, lane, ws, sb, kout);
         }
         __syncthreads();
         const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
@@ -1336,7 +1355,7 @@ void eri_staged_split_rows_kernel(EriArgs a)
         const int bi = task->list, bn = cst(a.bra.ppn)[bi];
         for (int j = task->item0; j < task->item1; ++j) {
             const RowItem it(task, j, bn);
-            staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToRows<NROW>, W>(a, bi, it.chunk, it.u0, it.un, lane, ws, sb, kout,
+            staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToRows<NROW>, W>(a, bi, it, lane, ws, sb, kout,
                                                                        wib);
             __syncthreads();    // the slot is rewritten by the next item
         }

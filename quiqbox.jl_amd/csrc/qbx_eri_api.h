@@ -14,12 +14,12 @@ enum EriMode { MODE_JK = 0, MODE_DENSE = 1, MODE_SCHWARZ = 2 };
 #endif
 constexpr int ROW_WAVES = QBX_ROW_WAVES;
 // One K-row task (one block): items item0 .. item1 - 1 of a list (a bra, or a
-// group of twin bras).  Item j is the 64-ket chunk chunk0 + j / parts with part
-// j % parts of the bra's primitive pairs: the digest is linear in the integrals,
-// so the waves that share a heavy chunk each digest the integrals of their own
-// primitive pairs.
+// group of twin bras).  Item j is the 64-ket chunk chunk0 + j / (kparts bparts)
+// with one of kparts parts of every ket's primitive pairs and one of bparts parts
+// of the bra's: the digest is linear in the integrals, so the waves that share a
+// heavy chunk each digest the integrals of their own primitive quartets.
 struct RowTask {
-    int list, chunk0, parts, item0, item1;
+    int list, chunk0, kparts, bparts, item0, item1;
 };
 // Most items per task of the low-L K-row and twin kernels, and of the staged
 // K-row kernel (whose waves are long, so that smaller tasks balance better).
