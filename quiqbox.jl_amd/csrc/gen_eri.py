@@ -94,8 +94,10 @@ STAGE_ONE_WAVE = {(2, 2, 2, 2): 62}
 # too few tasks to give every SIMD more than one wave), (dd|dp) 3.89 -> 2.66
 # ms, (dp|dp) 2.50 -> 2.14 ms; (dp|pp) 3.72 -> 4.29, (dd|pp) 1.47 -> 1.61 and
 # (dd|ds) 1.13 -> 1.27 ms lost (many tasks already fill the chip, and the
-# extra barriers cost).
-STAGE_SPLIT = {(2, 2, 2, 2): 4, (2, 2, 2, 1): 4, (2, 1, 2, 1): 4}
+# extra barriers cost): those three share chunks only where there are few of them
+# (kSplitChunks in qbx.hip).
+STAGE_SPLIT = {c: 4 for c in STAGED}
+STAGE_SPLIT_ALWAYS = {(2, 2, 2, 2), (2, 2, 2, 1), (2, 1, 2, 1)}
 # 64-ket chunks per task (one bra, its K rows flushed once per task) of the
 # classes of STAGE_SPLIT.  Each chunk already occupies a whole block, so small
 # tasks balance best.  Measured on the 592-function cluster against 8 chunks a
@@ -103,7 +105,8 @@ STAGE_SPLIT = {(2, 2, 2, 2): 4, (2, 2, 2, 1): 4, (2, 1, 2, 1): 4}
 # 2.55 -> 1.60 ms at two (1.45 at one), (dp|dp) 2.11 -> 1.87 ms at two (2.00 at
 # one); the concurrent build was 0.5-1 ms slower with one-chunk tasks for all
 # three than with two (more K-row flushes among the other classes' atomics).
-STAGE_SPLIT_CHUNKS = {(2, 2, 2, 2): 1, (2, 2, 2, 1): 2, (2, 1, 2, 1): 2}
+STAGE_SPLIT_CHUNKS = {(2, 2, 2, 2): 1, (2, 2, 2, 1): 2, (2, 1, 2, 1): 2, (2, 1, 1, 1): 2, (2, 2, 1, 1): 2,
+                      (2, 2, 2, 0): 2}
 # Classes whose K-row J/K kernel is compiled for two waves per SIMD (256
 # registers, the rest spilled to scratch) instead of the compiler's choice of
 # one wave with AGPRs.  Measured on the 592-function cluster, serialized:
@@ -1023,6 +1026,9 @@ def main(outdir):
              "static const int qbx_class_split_chunks[%d] = {%s};" % (
                  len(classes), ", ".join(str(STAGE_SPLIT_CHUNKS[c] if c in STAGED and STAGE_SPLIT.get(c, 1) > 1
                                              else 0) for c in classes)),
+             "// classes whose chunks are shared however many there are",
+             "static const int qbx_class_split_always[%d] = {%s};" % (
+                 len(classes), ", ".join("1" if c in STAGE_SPLIT_ALWAYS else "0" for c in classes)),
              "// classes launched after all others in a Fock build",
              "static const int qbx_class_last[%d] = {%s};" % (
                  len(classes), ", ".join("1" if c in LAUNCH_LAST else "0" for c in classes)),

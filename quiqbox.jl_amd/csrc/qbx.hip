@@ -102,6 +102,15 @@ constexpr double QBX_PRIM_PAIR_CUT = 1e-20;
 // kernel that adds the sums to J costs what the atomics gain (771 against 773,
 // 796 against 804 us).
 constexpr int kPairSumMin = 64;
+// Chunks of 64 kets up to which every staged class shares them among the waves of
+// a block: a class of few chunks takes as long as one of them, and four waves do one
+// in less than half the time.  8 H2O UHF (154 chunks of (dd|pp), 125 of (dd|ds)):
+// 0.48 -> 0.21 and 0.35 -> 0.15 ms, build 3.22 -> 2.95 ms; builds of 25, 50 and 100
+// functions 549 -> 487, 601 -> 505, 735 -> 674 us.  Shared up to 3500 chunks, single
+// classes still gained ((dd|pp) of the 592-function cluster 1.50 -> 1.22 ms), but the
+// concurrent builds lost: 8 H2O 2.95 -> 3.16 ms ((dp|pp), 1409 chunks), 24 H2O
+// 32.8 -> 33.4.
+constexpr int kSplitChunks = 512;
 // Ket buckets.  A wave's lanes take consecutive kets of one bra and the wave
 // runs as long as its lane with the most primitive pairs; in Schwarz order,
 // contracted core pairs (81 primitive pairs in cc-pVDZ oxygen) sit among
@@ -195,7 +204,7 @@ struct qbx_ctx {
     bool ket_buckets = true;       // kets bucketed by primitive-pair count (QBX_KET_BUCKETS=0: off)
     bool jk_rows = true;           // LDS K-row and twin kernels in the J/K build (QBX_JK_ROWS=0: off, the
                                    // one-wave-per-chunk kernels run everywhere)
-    bool staged_split = true;      // (dd|dd), (dd|dp), (dp|dp): 64-ket chunks shared by a block's waves (QBX_STAGED_SPLIT=0: off)
+    bool staged_split = true;      // staged classes: 64-ket chunks shared by a block's waves (QBX_STAGED_SPLIT=0: off)
     DevBuf<double> la_X, la_F, la_P, la_Q, la_T, la_aux;   // density purification
     double* scratch = nullptr;     // this device's address of the fixed work array
     rocblas_handle blas = nullptr; // rocSOLVER's handle (qbx_fock_solve), created on first use
@@ -224,6 +233,7 @@ struct TaskSet {
     const int* cpre = nullptr;        // waves (chunks of 64 kets) per bra, prefix sums
     const RowTask* rtask = nullptr;   // K-row tasks
     int nsuper = 0;
+    bool split = false;               // staged class: chunks shared by a block's waves
     int64_t total = 0;
     int nwave = 0;
     int nbra = 0;
@@ -1288,14 +1298,14 @@ private:
 };
 
 // K-row tasks of class cls over the ket lists L of its bras
-std::vector<RowTask> row_tasks(const qbx_basis* b, int cls, const KetLists& L, TaskCaps cap)
+std::vector<RowTask> row_tasks(const qbx_basis* b, int cls, const KetLists& L, TaskCaps cap, bool split)
 {
     const PairClass& PX = pair_class(b, cls, 0);
     const PairClass& PY = pair_class(b, cls, 1);
     int waves = ROW_WAVES, items = ROW_ITEMS;
     if (qbx_class_ws[cls] > 0) {
         items = STAGED_ROW_ITEMS;
-        if (qbx_class_split[cls] > 1 && qbx_class_split_chunks[cls] > 0) {   // the block shares each item
+        if (split) {   // the block shares each item
             waves = 1;
             items = qbx_class_split_chunks[cls];
             cap.item *= qbx_class_split[cls];
@@ -1372,7 +1382,9 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
         auto add = [&](TaskSet& t, const int* lo, const std::vector<int>& hi, const TaskCaps& cap) {
             KetLists L(pool, pair_class(b, cls, 1), pair_class(b, cls, 0).n(), &t.klist, &t.cpre);
             bra_lists(b, cls, lo, hi, L);
-            const std::vector<RowTask> tasks = row_tasks(b, cls, L, cap);
+            t.split = b->ctx->staged_split && qbx_class_split[cls] > 1 &&
+                      (qbx_class_split_always[cls] || L.nwave <= kSplitChunks);
+            const std::vector<RowTask> tasks = row_tasks(b, cls, L, cap, t.split);
             pool.add(tasks, &t.rtask);
             t.nsuper = (int)tasks.size();
             t.total = L.total;
@@ -1700,6 +1712,7 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
             // no K-row task lists: the one-wave-per-chunk kernels run
             a.rtask = ctx->jk_rows ? t.rtask : nullptr;
             a.nsuper = t.nsuper;
+            a.split = t.split ? 1 : 0;
             a.total = t.total;
             a.nwave = t.nwave;
             a.nbra = t.nbra;
@@ -1711,7 +1724,6 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
             a.twmax = w ? w->twmax : 0;
         };
         a.lds_max = ctx->lds_max;
-        a.split = ctx->staged_split ? 1 : 0;
         const TaskSet& t64 = twin ? b->s64[cls] : b->t64[cls];
         set_tasks(t64, twin ? &b->w64[cls] : nullptr);
         const TaskSet& t32 = b->t32[cls];
