@@ -36,6 +36,7 @@
 
 #include "qbx_common.h"
 #include "qbx_eri_api.h"
+#include "qbx_hostcopy.h"
 #include "qbx_linalg.h"
 #include "qbx_one_e.h"
 #include "gen/eri_table.inc"
@@ -206,6 +207,7 @@ struct qbx_ctx {
                                    // one-wave-per-chunk kernels run everywhere)
     bool staged_split = true;      // staged classes: 64-ket chunks shared by a block's waves (QBX_STAGED_SPLIT=0: off)
     DevBuf<double> la_X, la_F, la_P, la_Q, la_T, la_aux;   // density purification
+    HostCopier copier;             // large host arrays
     double* scratch = nullptr;     // this device's address of the fixed work array
     rocblas_handle blas = nullptr; // rocSOLVER's handle (qbx_fock_solve), created on first use
     std::mutex mu;
@@ -2303,8 +2305,7 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
             QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
             QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
         }
-        QBX_HIP(hipMemcpyAsync(eri, d.p, N4 * sizeof(double), hipMemcpyDeviceToHost, st));
-        QBX_HIP(hipStreamSynchronize(st));
+        ctx->copier.to_host(ctx->device, eri, d.p, N4 * sizeof(double), st);
     });
 }
 
@@ -2502,14 +2503,13 @@ int qbx_mo_transform(qbx_ctx* ctx, int32_t rank, int32_t n_ao, int32_t n_mo, con
         buf[0].ensure(big);
         buf[1].ensure(big);
         dC.upload(std::vector<double>(C, C + (size_t)n_ao * n_mo), st);
-        QBX_HIP(hipMemcpyAsync(buf[0].p, ints, n_in * sizeof(double), hipMemcpyHostToDevice, st));
+        ctx->copier.to_device(ctx->device, buf[0].p, ints, n_in * sizeof(double), st);
         for (int q = 0; q < rank; ++q) {
             const int M = (int)rows[q];
             gemm_f64(true, false, M, n_mo, n_ao, 1.0, buf[q & 1].p, M, dC.p, n_mo, 0.0, nullptr, 0,
                      buf[(q + 1) & 1].p, n_mo, st);
         }
-        QBX_HIP(hipMemcpyAsync(out, buf[rank & 1].p, n_out * sizeof(double), hipMemcpyDeviceToHost, st));
-        QBX_HIP(hipStreamSynchronize(st));
+        ctx->copier.to_host(ctx->device, out, buf[rank & 1].p, n_out * sizeof(double), st);
     });
 }
 
@@ -2527,7 +2527,7 @@ int qbx_mo_coulomb_ab(qbx_ctx* ctx, int32_t n_ao, int32_t n1, int32_t n2, const 
         hipStream_t st = ctx->stream;
         DevBuf<double> dE, dC1, dC2, K1, K2, P, dJ;
         dE.ensure(nn * nn);
-        QBX_HIP(hipMemcpyAsync(dE.p, eri, nn * nn * sizeof(double), hipMemcpyHostToDevice, st));
+        ctx->copier.to_device(ctx->device, dE.p, eri, nn * nn * sizeof(double), st);
         dC1.upload(std::vector<double>(C1, C1 + (size_t)n_ao * n1), st);
         dC2.upload(std::vector<double>(C2, C2 + (size_t)n_ao * n2), st);
         K1.ensure(nn * n1);
