@@ -1745,8 +1745,14 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
     };
     // Without serialized timing, the class kernels run concurrently on the
     // auxiliary streams (staged classes first, then largest work first);
-    // they only meet in the J/K atomics.
-    const bool fork = ctx->timing != 1;
+    // they only meet in the J/K atomics.  One occupied class stays on the main
+    // stream (H10 in STO-3G: the two rounds of events took 20 of 107 us).
+    auto occupied = [&](int cls) {
+        return b->t64[cls].nwave > 0 || (mode == QBX_PREC_MIXED && b->t32[cls].nwave > 0);
+    };
+    size_t parallel = b->has_high ? b->hl.sets.size() : 0;
+    for (int cls = 0; cls < QBX_N_CLASSES; ++cls) parallel += occupied(cls);
+    const bool fork = ctx->timing != 1 && parallel > 1;
     if (fork) {
         QBX_HIP(hipEventRecord(ctx->ev_fork, st));
         for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
@@ -1776,7 +1782,9 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
         if (sx != sy) return sx;
         return b->class_cost[x] > b->class_cost[y];
     });
-    for (int oi = 0; oi < QBX_N_CLASSES; ++oi) launch_class(order[oi], fork ? ctx->aux[oi % kStreams] : st);
+    int lane = 0;
+    for (int cls : order)
+        if (ctx->timing != 0 || occupied(cls)) launch_class(cls, fork ? ctx->aux[lane++ % kStreams] : st);
     if (fork) {
         for (int k = 0; k < kStreams; ++k) {
             QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
