@@ -1299,6 +1299,13 @@ private:
     std::map<int, std::vector<Cut>> by_bn_;
 };
 
+// whether the waves of a block share each of the class's nwave chunks
+bool split_chunks(const qbx_basis* b, int cls, int nwave)
+{
+    return b->ctx->staged_split && qbx_class_split[cls] > 1 &&
+           (qbx_class_split_always[cls] || nwave <= kSplitChunks);
+}
+
 // K-row tasks of class cls over the ket lists L of its bras
 std::vector<RowTask> row_tasks(const qbx_basis* b, int cls, const KetLists& L, TaskCaps cap, bool split)
 {
@@ -1384,8 +1391,7 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
         auto add = [&](TaskSet& t, const int* lo, const std::vector<int>& hi, const TaskCaps& cap) {
             KetLists L(pool, pair_class(b, cls, 1), pair_class(b, cls, 0).n(), &t.klist, &t.cpre);
             bra_lists(b, cls, lo, hi, L);
-            t.split = b->ctx->staged_split && qbx_class_split[cls] > 1 &&
-                      (qbx_class_split_always[cls] || L.nwave <= kSplitChunks);
+            t.split = split_chunks(b, cls, L.nwave);
             const std::vector<RowTask> tasks = row_tasks(b, cls, L, cap, t.split);
             pool.add(tasks, &t.rtask);
             t.nsuper = (int)tasks.size();
@@ -2296,6 +2302,7 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
             a.total = L.total;
             a.nwave = L.nwave;
             a.nbra = L.nl;
+            a.split = split_chunks(b, cls, L.nwave) ? 1 : 0;
             a.scratch_stream = (void*)st;
             attach_workspace(b, cls, a.nwave, a);
             a.eri = d.p;

@@ -216,11 +216,12 @@ __device__ __forceinline__ void boys_lds(double T, double* __restrict__ F, const
 // Copy the head constants and the Boys rows of the class's total angular
 // momentum into LDS (dst holds BOYS_HEAD2 + ROWS * QBX_BOYSL_STRIDE / 2 double2).
 template <int TPB, int ROWS = QBX_BOYSL_ROWS>
-__device__ __forceinline__ void stage_boys(double2* __restrict__ dst, const double* __restrict__ src)
+__device__ __forceinline__ void stage_boys(double2* __restrict__ dst, const double* __restrict__ src,
+                                           int threads = TPB)
 {
     if (threadIdx.x < BOYS_HEAD) ((double*)dst)[threadIdx.x] = kBoysExp[threadIdx.x];
     const double2* s = (const double2*)src;
-    for (int i = threadIdx.x; i < ROWS * QBX_BOYSL_STRIDE / 2; i += TPB) dst[BOYS_HEAD2 + i] = s[i];
+    for (int i = threadIdx.x; i < ROWS * QBX_BOYSL_STRIDE / 2; i += threads) dst[BOYS_HEAD2 + i] = s[i];
 }
 
 // The ket-pair quantities one primitive quartet reads; Kq carries the quartet's
@@ -318,8 +319,127 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// J/K digest and dense tensor: one wave per (bra, chunk of 64 kets).
-template <int LA, int LB, int LC, int LD, typename R, int MODE>
+// Waves of a dense block: as many as the registers of the class leave room for.
+__host__ __device__ constexpr int dense_waves(int nacc) { return nacc <= 9 ? 16 : nacc <= 36 ? 8 : 4; }
+
+// Dense tensor of the classes whose accumulators stay in registers.  The tensors
+// that fit a device are of small molecules: few chunks of 64 kets, each up to
+// thousands of primitive quartets long (64 x 64 for the contracted s pairs of N2 in
+// cc-pVTZ, whose (ss|ss) has 36 chunks).  So the W = blockDim.x / 64 waves of a
+// block share a chunk: each sums its parts of the bra's and the kets' primitive
+// pairs, the sums are added in LDS in wave order (the tensor comes out the same
+// on every run), and the waves share the components of A in the transfer and the
+// stores.  A persistent grid over the chunks.  N2 in cc-pVTZ, against one wave a
+// chunk: the whole tensor with its copy to the host 15.5 -> 10.3 ms ((ss|ss) alone
+// 3.2 ms before).
+template <int LA, int LB, int LC, int LD, typename R>
+__global__ __launch_bounds__(64 * dense_waves(EriClass<LA, LB, LC, LD, R>::NACC)) void eri_dense_kernel(EriArgs a)
+{
+    using Cls = EriClass<LA, LB, LC, LD, R>;
+    constexpr int NA = qbx_ncart(LA), NB = qbx_ncart(LB), NC = qbx_ncart(LC), ND = qbx_ncart(LD);
+    constexpr int LT = LA + LB + LC + LD;
+    constexpr int NCD = NC * ND;
+    constexpr bool PREFETCH = Cls::NACC <= 18;
+    __shared__ double2 sboys[BOYS_HEAD2 + boys_rows(LT) * QBX_BOYSL_STRIDE / 2];
+    __shared__ R sums[Cls::NACC][64];
+    stage_boys<0, boys_rows(LT)>(sboys, a.boysl, (int)blockDim.x);
+    __syncthreads();
+    const double* sb = (const double*)sboys + BOYS_HEAD;
+
+    const int lane = (int)threadIdx.x & 63;
+    const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int W = (int)blockDim.x >> 6;
+    const cptr<int> cpre = cst(a.cpre);
+    const size_t N = (size_t)a.N;
+    for (int chunk = (int)blockIdx.x; chunk < a.nwave; chunk += (int)gridDim.x) {
+        int lo = 0, hi = a.nbra;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (cpre[mid] <= chunk) lo = mid; else hi = mid;
+        }
+        const int bi = lo;
+        const KetList kl(a.klist, a.nbk, bi);
+        const int pos = (chunk - cpre[bi]) * 64 + lane;
+        const bool live = pos < kl.n;
+        const int ki = kl.ket(live ? pos : 0);
+        const int kn = live ? a.ket.ppn[ki] : 0;
+        const int bn = cst(a.bra.ppn)[bi];
+        // bparts x kparts = W: the bra's primitive pairs down to 4 a part, then the kets'
+        int bparts = 1;
+        while (bparts < W && bn >= 8 * bparts) bparts *= 2;
+        RowItem it(0, bn);
+        const int per = (bn + bparts - 1) / bparts;
+        it.u0 = min((wib % bparts) * per, bn);
+        it.un = min(per, bn - it.u0);
+        it.kpart = wib / bparts;
+        it.kparts = W / bparts;
+        int v0, vn;
+        it.ket_part(kn, v0, vn);
+        R acc[Cls::NACC];
+#pragma unroll
+        for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
+        prim_loop<Cls, LT, R, PREFETCH, -1>(acc, cst(a.pp + cst(a.bra.ppo)[bi]) + it.u0, it.un,
+                                            a.pp + a.ket.ppo[ki] + v0, vn, sb);
+        if (W > 1) {
+            for (int w = 0; w < W; ++w) {
+                __syncthreads();    // also: the last chunk's sums are read
+                if (w != wib) continue;
+#pragma unroll
+                for (int n = 0; n < Cls::NACC; ++n) sums[n][lane] = w == 0 ? acc[n] : sums[n][lane] + acc[n];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int n = 0; n < Cls::NACC; ++n) acc[n] = sums[n][lane];
+        }
+        if (live && wib < NA) {
+            const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
+            const cptr<double> ABp = cst(a.bra.AB + 3 * bi);
+            const double* CDp = a.ket.AB + 3 * ki;
+            R kacc[Cls::NE * NCD];
+            Cls::hrr_ket(acc, kacc, (R)CDp[0], (R)CDp[1], (R)CDp[2]);
+            const R ABx = (R)ABp[0], ABy = (R)ABp[1], ABz = (R)ABp[2];
+            const cptr<DevShell> SA = cst(a.sh + sA);
+            const cptr<DevShell> SB = cst(a.sh + sB);
+            const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
+            const DevShell* SC = a.sh + sC;
+            const DevShell* SD = a.sh + sD;
+            const bool diag = a.same && bi == ki;
+#pragma unroll
+            for (int ia = 0; ia < NA; ++ia) {
+                if (ia % W != wib) continue;
+                R out[NB * NCD];
+                Cls::hrr_bra(ia, kacc, out, ABx, ABy, ABz);
+#pragma unroll
+                for (int ib = 0; ib < NB; ++ib)
+#pragma unroll
+                    for (int ic = 0; ic < NC; ++ic)
+#pragma unroll
+                        for (int id = 0; id < ND; ++id) {
+                            if (SA->bf[ia] < 0 || SB->bf[ib] < 0 || SC->bf[ic] < 0 || SD->bf[id] < 0) continue;
+                            // an element that several components reach (A = B, C = D, bra = ket)
+                            // is written by one
+                            if ((sA == sB && ia < ib) || (sC == sD && ic < id) ||
+                                (diag && ia * NB + ib < ic * ND + id))
+                                continue;
+                            const size_t i = SA->bf[ia], j = SB->bf[ib], k = SC->bf[ic], l = SD->bf[id];
+                            const double v = (double)out[ib * NCD + ic * ND + id] * (SA->sc[ia] * SB->sc[ib]) *
+                                             (SC->sc[ic] * SD->sc[id]);
+                            a.eri[((i * N + j) * N + k) * N + l] = v;
+                            a.eri[((j * N + i) * N + k) * N + l] = v;
+                            a.eri[((i * N + j) * N + l) * N + k] = v;
+                            a.eri[((j * N + i) * N + l) * N + k] = v;
+                            a.eri[((k * N + l) * N + i) * N + j] = v;
+                            a.eri[((l * N + k) * N + i) * N + j] = v;
+                            a.eri[((k * N + l) * N + j) * N + i] = v;
+                            a.eri[((l * N + k) * N + j) * N + i] = v;
+                        }
+            }
+        }
+    }
+}
+
+// J/K digest: one wave per (bra, chunk of 64 kets).
+template <int LA, int LB, int LC, int LD, typename R>
 __global__ __launch_bounds__(eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC)) void eri_kernel(EriArgs a)
 {
     using Cls = EriClass<LA, LB, LC, LD, R>;
@@ -352,7 +472,7 @@ __global__ __launch_bounds__(eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC)) void er
     const int sA = cst(a.bra.shA)[bi], sB = cst(a.bra.shB)[bi];
     const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
     int kn = inrange ? a.ket.ppn[ki] : 0;
-    if (MODE == MODE_JK && a.pdmax) {
+    if (a.pdmax) {
         // Haser-Ahlrichs bound with the densities of this build
         const double* dm = a.pdmax;
         const int ns = a.nshell;
@@ -393,34 +513,6 @@ __global__ __launch_bounds__(eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC)) void er
         for (int id = 0; id < ND; ++id) scd[ic * ND + id] = SC->sc[ic] * SD->sc[id];
 
     const size_t N = (size_t)a.N;
-    if (MODE == MODE_DENSE) {
-        if (!live) return;
-#pragma unroll
-        for (int ia = 0; ia < NA; ++ia) {
-            R out[NB * NCD];
-            Cls::hrr_bra(ia, kacc, out, ABx, ABy, ABz);
-#pragma unroll
-            for (int ib = 0; ib < NB; ++ib)
-#pragma unroll
-                for (int ic = 0; ic < NC; ++ic)
-#pragma unroll
-                    for (int id = 0; id < ND; ++id) {
-                        if (SA->bf[ia] < 0 || SB->bf[ib] < 0 || fc[ic] < 0 || fd[id] < 0) continue;
-                        const size_t i = SA->bf[ia], j = SB->bf[ib], k = fc[ic], l = fd[id];
-                        const double v = (double)out[ib * NCD + ic * ND + id] * (SA->sc[ia] * SB->sc[ib]) *
-                                         scd[ic * ND + id];
-                        a.eri[((i * N + j) * N + k) * N + l] = v;
-                        a.eri[((j * N + i) * N + k) * N + l] = v;
-                        a.eri[((i * N + j) * N + l) * N + k] = v;
-                        a.eri[((j * N + i) * N + l) * N + k] = v;
-                        a.eri[((k * N + l) * N + i) * N + j] = v;
-                        a.eri[((l * N + k) * N + i) * N + j] = v;
-                        a.eri[((k * N + l) * N + j) * N + i] = v;
-                        a.eri[((l * N + k) * N + j) * N + i] = v;
-                    }
-        }
-        return;
-    }
 
     // ---- MODE_JK: digest, one bra component a at a time, with the
     //      degeneracy of the unique shell quartet ----
@@ -1041,7 +1133,6 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, const Row
                                  cst(a.pp + cst(a.bra.ppo)[bi]) + it.u0, it.un,
                                  a.pp + a.ket.ppo[ki] + v0, vn, sb, (R)CDp[0], (R)CDp[1], (R)CDp[2], ws);
     if constexpr (W > 1) {
-        static_assert(MODE == MODE_JK, "split staged tasks digest J/K only");
         __syncthreads();    // every group's [e|cd) is in the slot
     }
 
@@ -1060,20 +1151,24 @@ __device__ __forceinline__ void staged_chunk(const EriArgs& a, int bi, const Row
 
     if (MODE == MODE_DENSE) {
         if (!live) return;
+        // all rows, or this wave's share
 #pragma unroll 1
-        for (int iab = 0; iab < NA * NB; ++iab) {
+        for (int iab = W == 1 ? 0 : wib * NA * NB / W; iab < (W == 1 ? NA * NB : (wib + 1) * NA * NB / W); ++iab) {
             const int ia = iab / NB, ib = iab - ia * NB;
             R out[NCD];
             Cls::hrr_bra_ab(iab, ws, out, ABx, ABy, ABz);
             const int fa_ = SA->bf[ia], fb_ = SB->bf[ib];
-            if (fa_ < 0 || fb_ < 0) continue;
+            // an element that several components reach (A = B, C = D, bra = ket) is written by one
+            if (fa_ < 0 || fb_ < 0 || (sA == sB && ia < ib)) continue;
             const double sab = SA->sc[ia] * SB->sc[ib];
             const size_t i = fa_, j = fb_;
 #pragma unroll
             for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
                 for (int id = 0; id < ND; ++id) {
-                    if (fc[ic] < 0 || fd[id] < 0) continue;
+                    if (fc[ic] < 0 || fd[id] < 0 || (sC == sD && ic < id) ||
+                        (a.same && bi == ki && iab < ic * ND + id))
+                        continue;
                     const size_t k = fc[ic], l = fd[id];
                     const double v = (double)out[ic * ND + id] * sab * (scc[ic] * scdd[id]);
                     a.eri[((i * N + j) * N + k) * N + l] = v;
@@ -1239,10 +1334,10 @@ void eri_staged_kernel(EriArgs a)
     }
 }
 
-// Staged J/K with each wave task shared by the Cls::SPLIT waves of a block
-// (classes with few tasks: their latency, not the throughput of a full chip,
-// sets the time).  A persistent grid of blocks, one workspace slot each.
-template <int LA, int LB, int LC, int LD, typename R>
+// Staged J/K or dense tensor with each wave task shared by the Cls::SPLIT waves
+// of a block (classes with few tasks: their latency, not the throughput of a full
+// chip, sets the time).  A persistent grid of blocks, one workspace slot each.
+template <int LA, int LB, int LC, int LD, typename R, int MODE>
 __global__ __launch_bounds__((64 * EriClass<LA, LB, LC, LD, R>::SPLIT)) __attribute__((amdgpu_waves_per_eu(EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD, EriClass<LA, LB, LC, LD, R>::WAVES_PER_SIMD)))
 void eri_staged_split_kernel(EriArgs a)
 {
@@ -1269,7 +1364,7 @@ void eri_staged_split_kernel(EriArgs a)
             const int mid = (lo + hi) >> 1;
             if (cpre[mid] <= task) lo = mid; else hi = mid;
         }
-        staged_chunk<LA, LB, LC, LD, R, MODE_JK, KToGlobal, W>(a, lo, RowItem(task - cpre[lo], cst(a.bra.ppn)[lo]), lane, ws,
+        staged_chunk<LA, LB, LC, LD, R, MODE, KToGlobal, W>(a, lo, RowItem(task - cpre[lo], cst(a.bra.ppn)[lo]), lane, ws,
                                                                sb, kout, wib);
         __syncthreads();    // the slot is rewritten by the next task
     }
@@ -1365,7 +1460,14 @@ void eri_staged_split_rows_kernel(EriArgs a)
     }
 }
 
-// Schwarz bounds: one thread per diagonal shell pair (ab|ab).
+// Lanes that share a diagonal shell pair in the Schwarz kernel.
+__host__ __device__ constexpr int schwarz_lanes(int nacc) { return nacc <= 9 ? 64 : nacc <= 100 ? 16 : 1; }
+
+// Schwarz bounds: schwarz_lanes lanes per diagonal shell pair (ab|ab), each with
+// its part of the bra's primitive pairs; the [e0|f0] sums meet through lane
+// exchanges.  One lane a pair took as long as its longest pair, 64 x 64 primitive
+// quartets in cc-pVTZ: N2, (ss) 1.75 ms, (ps) 0.86, (pp) 0.51; the first tensor of a
+// basis 21.6 -> 13.0 ms with the dense kernels, the first build of 8 H2O 9.3 -> 6.3.
 template <int LA, int LB, typename R>
 __global__ __launch_bounds__(256) void eri_schwarz_kernel(EriArgs a)
 {
@@ -1373,18 +1475,28 @@ __global__ __launch_bounds__(256) void eri_schwarz_kernel(EriArgs a)
     constexpr int NA = qbx_ncart(LA), NB = qbx_ncart(LB);
     constexpr int LT = 2 * (LA + LB);
     constexpr int NCD = NA * NB;
+    constexpr int G = schwarz_lanes(Cls::NACC);
     __shared__ double2 sboys[BOYS_HEAD2 + boys_rows(LT) * QBX_BOYSL_STRIDE / 2];
     stage_boys<256, boys_rows(LT)>(sboys, a.boysl);
     __syncthreads();
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.total) return;
-    const int bi = (int)t;
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G;
+    const int part = (int)threadIdx.x % G;
+    const bool on = t < a.total;
+    const int bi = on ? (int)t : 0;
     R acc[Cls::NACC];
 #pragma unroll
     for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
     const PrimPair* P = a.pp + a.bra.ppo[bi];
-    const int n = a.bra.ppn[bi];
-    prim_loop<Cls, LT, R, false, -1>(acc, P, n, P, n, (const double*)sboys + BOYS_HEAD);
+    const int n = on ? a.bra.ppn[bi] : 0;
+    const int per = (n + G - 1) / G, u0 = min(part * per, n);
+    prim_loop<Cls, LT, R, false, -1>(acc, P + u0, min(per, n - u0), P, n, (const double*)sboys + BOYS_HEAD);
+    if constexpr (G > 1) {
+#pragma unroll
+        for (int k = 0; k < Cls::NACC; ++k)
+#pragma unroll
+            for (int o = G / 2; o >= 1; o >>= 1) acc[k] += __shfl_xor(acc[k], o, 64);
+    }
+    if (!on || part != 0) return;
     const double* AB = a.bra.AB + 3 * bi;
     R kacc[Cls::NE * NCD];
     Cls::hrr_ket(acc, kacc, (R)AB[0], (R)AB[1], (R)AB[2]);
@@ -1412,7 +1524,8 @@ void launch_eri(const EriArgs& a, hipStream_t s)
     if constexpr (MODE == MODE_SCHWARZ) {
         static_assert(LA == LC && LB == LD, "Schwarz bounds need a diagonal class");
         if (a.total <= 0) return;
-        const int64_t blocks = (a.total + 255) / 256;
+        constexpr int PAIRS = 256 / schwarz_lanes(EriClass<LA, LB, LC, LD, R>::NACC);
+        const int64_t blocks = (a.total + PAIRS - 1) / PAIRS;
         hipLaunchKernelGGL((eri_schwarz_kernel<LA, LB, R>), dim3((unsigned)blocks), dim3(256), 0, s, a);
         QBX_HIP(hipGetLastError());
     } else if constexpr (EriClass<LA, LB, LC, LD, R>::STAGED) {
@@ -1468,10 +1581,12 @@ void launch_eri(const EriArgs& a, hipStream_t s)
                 QBX_HIP(hipGetLastError());
                 return;
             }
+        }
+        if constexpr (EriClass<LA, LB, LC, LD, R>::SPLIT > 1) {
             if (a.split) {
                 // one slot per block
                 const int blocks = a.nwave < a.ws_slots ? a.nwave : a.ws_slots;
-                hipLaunchKernelGGL((eri_staged_split_kernel<LA, LB, LC, LD, R>), dim3((unsigned)blocks),
+                hipLaunchKernelGGL((eri_staged_split_kernel<LA, LB, LC, LD, R, MODE>), dim3((unsigned)blocks),
                                    dim3(64 * EriClass<LA, LB, LC, LD, R>::SPLIT), 0, s, a);
                 QBX_HIP(hipGetLastError());
                 return;
@@ -1536,19 +1651,38 @@ void launch_eri(const EriArgs& a, hipStream_t s)
             }
         }
         if (a.nwave <= 0) return;
-        // Kernels that spill to scratch run on the caller's main stream only:
-        // each extra hardware queue would need its own scratch allocation.
-        static const size_t scratch = [] {
-            hipFuncAttributes fa;
-            if (hipFuncGetAttributes(&fa, (const void*)eri_kernel<LA, LB, LC, LD, R, MODE>) != hipSuccess)
-                return (size_t)1;
-            return (size_t)fa.localSizeBytes;
-        }();
-        hipStream_t use = (scratch > 0 && a.scratch_stream) ? (hipStream_t)a.scratch_stream : s;
-        constexpr int TPB = eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC);
-        const int64_t blocks = ((int64_t)a.nwave + TPB / 64 - 1) / (TPB / 64);
-        hipLaunchKernelGGL((eri_kernel<LA, LB, LC, LD, R, MODE>), dim3((unsigned)blocks), dim3(TPB), 0, use, a);
-        QBX_HIP(hipGetLastError());
+        if constexpr (MODE == MODE_DENSE) {
+            static const size_t scratch = [] {
+                hipFuncAttributes fa;
+                if (hipFuncGetAttributes(&fa, (const void*)eri_dense_kernel<LA, LB, LC, LD, R>) != hipSuccess)
+                    return (size_t)1;
+                return (size_t)fa.localSizeBytes;
+            }();
+            hipStream_t use = (scratch > 0 && a.scratch_stream) ? (hipStream_t)a.scratch_stream : s;
+            // waves a chunk: enough to fill the chip's 4096 or so wave slots
+            constexpr int WMAX = dense_waves(EriClass<LA, LB, LC, LD, R>::NACC);
+            int waves = 1;
+            while (waves < WMAX && (int64_t)a.nwave * waves < 4096) waves *= 2;
+            const int blocks = a.nwave < 8192 / waves ? a.nwave : 8192 / waves;
+            hipLaunchKernelGGL((eri_dense_kernel<LA, LB, LC, LD, R>), dim3((unsigned)blocks), dim3(64 * waves), 0, use,
+                               a);
+            QBX_HIP(hipGetLastError());
+            return;
+        } else {
+            // Kernels that spill to scratch run on the caller's main stream only:
+            // each extra hardware queue would need its own scratch allocation.
+            static const size_t scratch = [] {
+                hipFuncAttributes fa;
+                if (hipFuncGetAttributes(&fa, (const void*)eri_kernel<LA, LB, LC, LD, R>) != hipSuccess)
+                    return (size_t)1;
+                return (size_t)fa.localSizeBytes;
+            }();
+            hipStream_t use = (scratch > 0 && a.scratch_stream) ? (hipStream_t)a.scratch_stream : s;
+            constexpr int TPB = eri_tpb(EriClass<LA, LB, LC, LD, R>::NACC);
+            const int64_t blocks = ((int64_t)a.nwave + TPB / 64 - 1) / (TPB / 64);
+            hipLaunchKernelGGL((eri_kernel<LA, LB, LC, LD, R>), dim3((unsigned)blocks), dim3(TPB), 0, use, a);
+            QBX_HIP(hipGetLastError());
+        }
     }
 }
 
