@@ -512,6 +512,9 @@ __global__ __launch_bounds__(TS * W) void eri_md_kernel(GenArgs a)
             if (MODE == MODE_SCHWARZ) {
                 if (ab == c0 + c) qmax = fmax(qmax, fabs(val));
             } else if (MODE == MODE_DENSE) {
+                // an element that several components reach (A = B, C = D, bra = ket) is written by one
+                if ((sA == sB && ia < ib) || (sC == sD && ic < id) || (a.same && bi == ki && ab < c0 + c))
+                    continue;
                 const size_t i = fa, j = fb, kk = fc, l = fd;
                 a.eri[((i * N + j) * N + kk) * N + l] = val;
                 a.eri[((j * N + i) * N + kk) * N + l] = val;

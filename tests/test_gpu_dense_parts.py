@@ -34,6 +34,18 @@ def test_dense_parts_match_oracle(sets):
     assert err < 1e-12
 
 
+def test_dense_with_f_shells_same_on_every_run():
+    bs = random_spd_basis(97, n_atoms=2, box=2.0, lmax=3, nprim=(3, 2, 1, 2))[1]
+    gb = qb.GPUBasis(bs)
+    E = gb.eri_dense()
+    print("[gpu-test] s to f shells: n %d" % gb.n, flush=True)
+    for _ in range(3):
+        assert np.array_equal(gb.eri_dense(), E)
+    # the eight permutations of every element are one value
+    for p in ((1, 0, 2, 3), (0, 1, 3, 2), (2, 3, 0, 1)):
+        assert np.array_equal(E.transpose(p), E)
+
+
 def test_schwarz_bounds_of_uneven_contractions():
     rng = np.random.default_rng(4)
     bs = []
