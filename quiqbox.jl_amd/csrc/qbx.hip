@@ -112,6 +112,10 @@ constexpr int kPairSumMin = 64;
 // concurrent builds lost: 8 H2O 2.95 -> 3.16 ms ((dp|pp), 1409 chunks), 24 H2O
 // 32.8 -> 33.4.
 constexpr int kSplitChunks = 512;
+// Order from which qbx_fock_solve tridiagonalizes with tridiagonalize(); below it
+// the library reduces in one block (n = 64: 1.92 against 1.89 ms; 100: 1.94
+// against 1.70).
+constexpr int kTridiagMin = 96;
 // Ket buckets.  A wave's lanes take consecutive kets of one bra and the wave
 // runs as long as its lane with the most primitive pairs; in Schwarz order,
 // contracted core pairs (81 primitive pairs in cc-pVDZ oxygen) sit among
@@ -208,6 +212,7 @@ struct qbx_ctx {
     bool staged_split = true;      // staged classes: 64-ket chunks shared by a block's waves (QBX_STAGED_SPLIT=0: off)
     DevBuf<double> la_X, la_F, la_P, la_Q, la_T, la_aux;   // density purification
     HostCopier copier;             // large host arrays
+    DevBuf<uint64_t> la_x;         // exchange of the tridiagonalization
     double* scratch = nullptr;     // this device's address of the fixed work array
     rocblas_handle blas = nullptr; // rocSOLVER's handle (qbx_fock_solve), created on first use
     std::mutex mu;
@@ -2446,7 +2451,7 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
         ctx->la_P.ensure(nn);
         ctx->la_Q.ensure(nn);
         ctx->la_T.ensure(nn);
-        ctx->la_aux.ensure(3 * (size_t)n + 4);
+        ctx->la_aux.ensure(4 * (size_t)n + 4);
         double* dX = ctx->la_X.p;
         double* dF = ctx->la_F.p;
         double* dP = ctx->la_P.p;
@@ -2455,7 +2460,8 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
         double* dE = ctx->la_aux.p;             // eigenvalues (n)
         double* dOff = dE + n;                  // off-diagonal work of the tridiagonal form (n)
         double* dSgn = dOff + n;                // column signs (n)
-        rocblas_int* dInfo = (rocblas_int*)(dSgn + n);
+        double* dTau = dSgn + n;                // factors of the reflectors (n)
+        rocblas_int* dInfo = (rocblas_int*)(dTau + n);   // the solver's, then the tridiagonalization's
         QBX_HIP(hipMemcpyAsync(dX, X, nn * sizeof(double), hipMemcpyHostToDevice, st));
         QBX_HIP(hipMemcpyAsync(dF, F, nn * sizeof(double), hipMemcpyHostToDevice, st));
         // Fock matrix in the orthonormal basis: X' F X, symmetrized
@@ -2464,15 +2470,41 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
         symmetrize_square(dP, n, st);
         // eigenpairs, ascending; the column-major eigenvector matrix V read
         // row-major is V^T
-        if (rocsolver_dsyevd(ctx->blas, rocblas_evect_original, rocblas_fill_upper, n, dP, n, dE, dOff, dInfo) !=
-            rocblas_status_success)
-            throw QbxError(QBX_EINTERNAL, "rocsolver_dsyevd failed");
-        rocblas_int info = 0;
-        QBX_HIP(hipMemcpyAsync(&info, dInfo, sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
-        QBX_HIP(hipStreamSynchronize(st));
-        if (info != 0) throw QbxError(QBX_ENOCONV, "the symmetric eigensolver did not converge");
+        const double* dV = dP;
+        rocblas_int info[2] = {0, 0};
+        auto read_info = [&](int k) {
+            QBX_HIP(hipMemcpyAsync(info, dInfo, k * sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
+            QBX_HIP(hipStreamSynchronize(st));
+        };
+        bool own = false;
+        if (n >= kTridiagMin) {
+            ctx->la_x.ensure(tridiag_exchange(n));
+            zero_async(dQ, nn, st);
+            own = tridiagonalize(n, dP, dQ, dE, dOff, dTau, ctx->la_x.p, dInfo + 1, st);
+        }
+        if (own) {
+            double* back = dTau + (n - 1);   // there are n - 1 factors
+            tridiag_scale(n, dE, dOff, back, st);
+            if (rocsolver_dstedc(ctx->blas, rocblas_evect_tridiagonal, n, dE, dOff, dT, n, dInfo) !=
+                    rocblas_status_success ||
+                rocsolver_dormtr(ctx->blas, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none, n, n, dQ, n,
+                                 dTau, dT, n) != rocblas_status_success)
+                throw QbxError(QBX_EINTERNAL, "rocsolver_dstedc or rocsolver_dormtr failed");
+            tridiag_unscale(n, dE, back, st);
+            read_info(2);
+            own = info[1] == 0;   // else a block gave up waiting: the library's own reduction
+            dV = dT;
+        }
+        if (!own) {
+            if (rocsolver_dsyevd(ctx->blas, rocblas_evect_original, rocblas_fill_upper, n, dP, n, dE, dOff, dInfo) !=
+                rocblas_status_success)
+                throw QbxError(QBX_EINTERNAL, "rocsolver_dsyevd failed");
+            read_info(1);
+            dV = dP;
+        }
+        if (info[0] != 0) throw QbxError(QBX_ENOCONV, "the symmetric eigensolver did not converge");
         // C = X V with every column's first entry made non-negative
-        gemm_f64(false, true, n, n, n, 1.0, dX, n, dP, n, 0.0, nullptr, 0, dQ, n, st);
+        gemm_f64(false, true, n, n, n, 1.0, dX, n, dV, n, 0.0, nullptr, 0, dQ, n, st);
         fix_column_signs(dQ, n, dSgn, st);
         QBX_HIP(hipMemcpyAsync(C, dQ, nn * sizeof(double), hipMemcpyDeviceToHost, st));
         if (eps) QBX_HIP(hipMemcpyAsync(eps, dE, n * sizeof(double), hipMemcpyDeviceToHost, st));

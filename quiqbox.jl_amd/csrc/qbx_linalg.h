@@ -3,6 +3,8 @@
 // Row-major matrices, device pointers, launches on the given stream.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cstddef>
+#include <cstdint>
 
 namespace qbx {
 
@@ -55,5 +57,22 @@ void sp2_product(const double* P, double* Q, int n, int nocc, int k, double* sha
 
 // state and measures after k launches of sp2_product
 void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2Status* out, hipStream_t s);
+
+// Householder tridiagonalization of the symmetric n x n matrix A (LAPACK's lower
+// form): diagonal d (n), off-diagonal e (n - 1), reflector k (its first entry, 1,
+// left out) in V[k n + k + 2 ...], factors tau (n - 1).  exchange: tridiag_exchange(n)
+// values of work space.  false where the matrix does not fit the device's LDS or
+// the device cannot run the whole grid at once (nothing is launched then).  *status
+// (device) is 0, or 1 when a block gave up waiting for another: the outputs are
+// not valid then.
+size_t tridiag_exchange(int n);
+bool tridiagonalize(int n, const double* A, double* V, double* d, double* e, double* tau, uint64_t* exchange,
+                    int* status, hipStream_t s);
+
+// The tridiagonal matrix times a power of two, its largest entry in [1, 2) (the
+// divide and conquer solver drops what is small in absolute terms), and the
+// eigenvalues d brought back; back: one double of device memory.
+void tridiag_scale(int n, double* d, double* e, double* back, hipStream_t s);
+void tridiag_unscale(int n, double* d, const double* back, hipStream_t s);
 
 }  // namespace qbx

@@ -4,6 +4,8 @@
 // MFMA f64 16x16x4 operand layout (one wave): lane l holds A[l % 16][l / 16]
 // and B[l / 16][l % 16]; the four result registers r hold
 // D[4 r + l / 16][l % 16].
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "qbx_common.h"
@@ -636,6 +638,315 @@ void sp2_product(const double* P, double* Q, int n, int nocc, int k, double* sha
 void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2Status* out, hipStream_t s)
 {
     hipLaunchKernelGGL(sp2_status_kernel, dim3(1), dim3(256), 0, s, shares, sp2_blocks(n), state + (k & 1), out);
+    QBX_HIP(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------
+// Householder tridiagonalization.  A step needs the whole pivot column and the
+// whole product A v before any row can be updated, so a library that launches a
+// few kernels a column pays their latency 600 times over (n = 600: 6000 launches,
+// 9.7 of the 13.9 ms of a Fock solve).  Here one persistent grid holds the matrix in
+// LDS, rows dealt to the blocks in turn, and the blocks exchange two numbers per
+// row and step: p_r = (A v)_r and the next pivot column's element before the
+// step's update.  From those every block forms the update's w, the next column
+// and its reflector for itself, so one exchange a step is all; the latency of the
+// exchange and of two block-wide sums (4 to 5 us a step) bounds it.  A Fock solve of
+// n = 100, 250, 600, 1000 and 1800: 1.94 -> 1.70, 5.9 -> 3.4, 13.3 -> 7.5, 24.0 ->
+// 13.7 and 49.5 -> 32.3 ms.
+//
+// The exchange needs no barrier: every value has a place of its own, filled with
+// TRI_EMPTY before the launch, and a reader polls until it holds something else.
+// Values cross the XCDs, so they are stored and loaded at agent scope.  A NaN is
+// published as the plain quiet NaN, which is not TRI_EMPTY.  The launch is
+// cooperative (all blocks resident), and a block that has polled TRI_SPINS times
+// sets *status and ends; the others then end the same way.
+// ---------------------------------------------------------------------------
+constexpr uint64_t TRI_EMPTY = ~0ull;
+constexpr int TRI_SPINS = 1 << 20;
+constexpr int TRI_MAX_N = 2048;   // 1024 threads, two elements each
+
+size_t tridiag_exchange(int n) { return 2 * (size_t)n * n; }
+
+__global__ void tri_empty_kernel(uint64_t* p, size_t n, int* status)
+{
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = TRI_EMPTY;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *status = 0;
+}
+
+__device__ __forceinline__ void tri_put(uint64_t* p, double v)
+{
+    const uint64_t u = v != v ? 0x7ff8000000000000ull : __builtin_bit_cast(uint64_t, v);
+    __hip_atomic_store(p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t tri_get(const uint64_t* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ double tri_wave_sum(double v)
+{
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// E elements of every length-n vector per thread: element e of a thread is
+// threadIdx.x + e * blockDim.x.
+template <int E>
+__global__ __launch_bounds__(1024) void tridiag_kernel(int n, const double* A, double* V, double* d, double* e_out,
+                                                       double* tau_out, uint64_t* exchange, int* status)
+{
+    extern __shared__ double lds[];
+    __shared__ double red[3][16];
+    __shared__ int fail;
+    const int B = (int)gridDim.x, b = (int)blockIdx.x, T = (int)blockDim.x, tid = (int)threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6, nwave = T >> 6;
+    const int R = (n + B - 1) / B;
+    double* rows = lds;                  // rows b, b + B, ...
+    double* va = rows + (size_t)R * n;   // last step's reflector,
+    double* wa = va + n;                 // its w,
+    double* vb = wa + n;                 // this step's column, then reflector
+    for (int i = tid; i < R * n; i += T) {
+        const int r = b + (i / n) * B;
+        if (r < n) rows[i] = A[(size_t)r * n + i % n];
+    }
+    if (tid == 0) fail = 0;
+    auto block_sum = [&](double v, int which) {
+        v = tri_wave_sum(v);
+        if (lane == 0) red[which][wave] = v;
+        __syncthreads();
+        double sum = 0.0;
+        for (int w = 0; w < nwave; ++w) sum += red[which][w];
+        return sum;
+    };
+    double tau = 0.0;
+    for (int k = 0; k < n - 1; ++k) {
+        double x[E];
+        if (k == 0) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                x[q] = r < n ? A[r] : 0.0;
+            }
+        } else {
+            // last step's products and the column before its update
+            const uint64_t* in = exchange + (size_t)(k - 1) * 2 * n;
+            uint64_t up[E], ux[E];
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                const bool on = r >= k && r < n;
+                up[q] = on ? tri_get(in + r) : 0;
+                ux[q] = on ? tri_get(in + n + r) : 0;
+            }
+            bool ok = true;
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                for (int i = 0; i < TRI_SPINS && (up[q] == TRI_EMPTY || ux[q] == TRI_EMPTY); ++i) {
+                    up[q] = tri_get(in + r);
+                    ux[q] = tri_get(in + n + r);
+                }
+                ok = ok && up[q] != TRI_EMPTY && ux[q] != TRI_EMPTY;
+            }
+            if (!ok) fail = 1;
+            double dot = 0.0;
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                if (r >= k && r < n) dot += __builtin_bit_cast(double, up[q]) * va[r];
+            }
+            dot = block_sum(dot, 0);
+            if (fail) {     // uniform: written before block_sum's barrier, and never reset
+                if (tid == 0) *status = 1;
+                return;
+            }
+            // w = tau (p - tau/2 (p.v) v); A <- A - v w' - w v'
+            double w[E];
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                w[q] = 0.0;
+                if (r >= k && r < n) {
+                    w[q] = tau * (__builtin_bit_cast(double, up[q]) - 0.5 * tau * dot * va[r]);
+                    wa[r] = w[q];
+                }
+            }
+            __syncthreads();
+            const double wk = wa[k], vk = va[k];
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                x[q] = r >= k && r < n ? __builtin_bit_cast(double, ux[q]) - va[r] * wk - w[q] * vk : 0.0;
+            }
+        }
+        // reflector of the column's part below the diagonal
+        double ssq = 0.0, big = 0.0;
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int r = tid + q * T;
+            if (r >= k && r < n) vb[r] = x[q];
+            if (r == k && b == 0) d[k] = x[q];
+            if (r >= k + 2 && r < n) ssq += x[q] * x[q];
+        }
+        ssq = block_sum(ssq, 1);
+        const double alpha = vb[k + 1];
+        double norm = sqrt(alpha * alpha + ssq);
+        bool tail = true;    // entries below alpha
+        if (!(ssq > 1e-280 && norm < 1e140)) {
+            // no entries, or squares that may have lost digits or overflowed:
+            // scaled by the largest entry
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                if (r >= k + 2 && r < n) big = fmax(big, fabs(x[q]));
+            }
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+            if (lane == 0) red[2][wave] = big;
+            __syncthreads();
+            for (int w = 0; w < nwave; ++w) big = fmax(big, red[2][w]);
+            __syncthreads();
+            tail = big > 0.0;
+            big = fmax(big, fabs(alpha));
+            double y2 = 0.0;
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int r = tid + q * T;
+                const double y = tail && r >= k + 2 && r < n ? x[q] / big : 0.0;
+                y2 += y * y;
+            }
+            y2 = block_sum(y2, 2);
+            norm = tail ? big * sqrt(y2 + (alpha / big) * (alpha / big)) : fabs(alpha);
+        }
+        double beta = alpha, scale = 0.0, tau_k = 0.0;
+        if (tail) {
+            beta = alpha > 0.0 ? -norm : norm;
+            tau_k = (beta - alpha) / beta;
+            scale = 1.0 / (alpha - beta);
+        }
+        __syncthreads();    // alpha read
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int r = tid + q * T;
+            if (r < k + 1 || r >= n) continue;
+            const double v = r == k + 1 ? 1.0 : x[q] * scale;
+            vb[r] = v;
+            if (b == 0 && r > k + 1) V[(size_t)k * n + r] = v;
+        }
+        if (b == 0 && tid == 0) {
+            e_out[k] = beta;
+            tau_out[k] = tau_k;
+        }
+        __syncthreads();
+        // this block's rows: last step's update, and their products with the reflector
+        uint64_t* out = exchange + (size_t)k * 2 * n;
+        for (int rr = wave; rr < R; rr += nwave) {
+            const int r = b + rr * B;
+            if (r <= k || r >= n) continue;
+            double* row = rows + (size_t)rr * n;
+            const double vr = k > 0 ? va[r] : 0.0, wr = k > 0 ? wa[r] : 0.0;
+            double acc = 0.0, first = 0.0;
+            for (int c = k + 1 + lane; c < n; c += 64) {
+                double a = row[c];
+                if (k > 0) {
+                    a -= vr * wa[c] + wr * va[c];
+                    row[c] = a;
+                }
+                if (c == k + 1) first = a;
+                acc += a * vb[c];
+            }
+            acc = tri_wave_sum(acc);
+            if (lane == 0) {
+                tri_put(out + r, acc);
+                tri_put(out + n + r, first);
+                if (k == n - 2) d[n - 1] = first;
+            }
+        }
+        __syncthreads();
+        double* t = va;
+        va = vb;
+        vb = t;
+        tau = tau_k;
+    }
+}
+
+bool tridiagonalize(int n, const double* A, double* V, double* d, double* e, double* tau, uint64_t* exchange,
+                    int* status, hipStream_t s)
+{
+    if (n < 2 || n > TRI_MAX_N) return false;
+    int dev = 0, cus = 0, coop = 0, lds_max = 0;
+    QBX_HIP(hipGetDevice(&dev));
+    QBX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    QBX_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    QBX_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    if (!coop || cus <= 0) return false;
+    const int threads = std::min(1024, (n + 63) / 64 * 64);
+    const bool two = n > 1024;
+    const void* f = two ? (const void*)tridiag_kernel<2> : (const void*)tridiag_kernel<1>;
+    // the fewest blocks whose LDS holds the matrix: each value then has fewer readers
+    // (n = 600: 64, 128 and 256 blocks 7.47, 7.64 and 7.95 ms a solve)
+    int B = 64;
+    size_t shm = 0;
+    for (;; B *= 2) {
+        B = std::min(std::min(B, cus), n);
+        shm = ((size_t)((n + B - 1) / B) + 3) * n * sizeof(double);
+        if (shm + 1024 <= (size_t)lds_max) break;
+        if (B >= 256 || B >= cus || B >= n) return false;
+    }
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, threads, shm) != hipSuccess || per_cu * cus < B) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t nx = tridiag_exchange(n);
+    hipLaunchKernelGGL(tri_empty_kernel, dim3((unsigned)std::min<size_t>((nx + 255) / 256, 2048)), dim3(256), 0, s,
+                       exchange, nx, status);
+    QBX_HIP(hipGetLastError());
+    void* args[] = {&n, &A, &V, &d, &e, &tau, &exchange, &status};
+    if (hipLaunchCooperativeKernel(f, dim3(B), dim3(threads), args, (unsigned)shm, s) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// One block: d (n) and e (n - 1) times the power of two that brings their largest
+// entry into [1, 2); *back undoes it.
+__global__ void tri_scale_kernel(int n, double* d, double* e, double* back)
+{
+    __shared__ double red[16];
+    double big = 0.0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) big = fmax(big, fmax(fabs(d[i]), i < n - 1 ? fabs(e[i]) : 0.0));
+    for (int o = 32; o >= 1; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = big;
+    __syncthreads();
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) big = fmax(big, red[w]);
+    const int x = big > 0.0 && big < HUGE_VAL ? -ilogb(big) : 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        d[i] = ldexp(d[i], x);
+        if (i < n - 1) e[i] = ldexp(e[i], x);
+    }
+    if (threadIdx.x == 0) *back = (double)-x;
+}
+__global__ void tri_unscale_kernel(int n, double* d, const double* back)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) d[i] = ldexp(d[i], (int)*back);
+}
+
+void tridiag_scale(int n, double* d, double* e, double* back, hipStream_t s)
+{
+    hipLaunchKernelGGL(tri_scale_kernel, dim3(1), dim3(1024), 0, s, n, d, e, back);
+    QBX_HIP(hipGetLastError());
+}
+void tridiag_unscale(int n, double* d, const double* back, hipStream_t s)
+{
+    hipLaunchKernelGGL(tri_unscale_kernel, dim3(1), dim3(1024), 0, s, n, d, back);
     QBX_HIP(hipGetLastError());
 }
 
