@@ -123,7 +123,6 @@ ROWS_TWO_WAVES = {(2, 1, 1, 0), (2, 0, 1, 1)}
 # 32.30 -> 32.42 ms (five A/B pairs on the 592-function cluster, within the
 # run-to-run spread).
 LAUNCH_LAST = {(2, 1, 2, 0)}
-TWIN_MAX_ACC = 9   # must match qbx_eri_api.h
 
 
 def cart(L):
@@ -954,10 +953,8 @@ def main(outdir):
     os.makedirs(outdir, exist_ok=True)
     classes, pcl = class_list()
     flops = {}
-    twin_ok = []
     for (la, lb, lc, ld) in classes:
         code, fv, fh, nacc, fexec = gen_class(la, lb, lc, ld)
-        twin_ok.append(fexec is None and nacc <= TWIN_MAX_ACC)
         tag = "%d%d%d%d" % (la, lb, lc, ld)
         flops[tag] = {"vrr_per_prim_quartet": fv, "hrr_per_quartet": fh, "n_acc": nacc,
                       "staged": fexec is not None}
@@ -1032,9 +1029,6 @@ def main(outdir):
              "// classes launched after all others in a Fock build",
              "static const int qbx_class_last[%d] = {%s};" % (
                  len(classes), ", ".join("1" if c in LAUNCH_LAST else "0" for c in classes)),
-             "// classes with a twin-bra kernel (not staged, at most %d accumulators)" % TWIN_MAX_ACC,
-             "static const int qbx_class_twin[%d] = {%s};" % (
-                 len(classes), ", ".join("1" if t else "0" for t in twin_ok)),
              "// launch-order cost model: per primitive shell quartet (geometry and Boys"
              " values, about %d operations, plus the executed VRR) and per contracted"
              " shell quartet (executed HRR plus %d per Cartesian quartet for the digest)" % (COST_PRIM0, COST_DIGEST),

@@ -205,9 +205,8 @@ struct qbx_ctx {
     bool xcd_local = false;        // per-XCD J/K copies (set by the probe at init)
     int n_xcd = 1;
     int lds_max = 65536;           // LDS bytes per block on this device
-    bool twins = true;             // twin-bra groups in the J/K build (QBX_TWINS=0: off)
     bool ket_buckets = true;       // kets bucketed by primitive-pair count (QBX_KET_BUCKETS=0: off)
-    bool jk_rows = true;           // LDS K-row and twin kernels in the J/K build (QBX_JK_ROWS=0: off, the
+    bool jk_rows = true;           // LDS K-row kernels in the J/K build (QBX_JK_ROWS=0: off, the
                                    // one-wave-per-chunk kernels run everywhere)
     bool staged_split = true;      // staged classes: 64-ket chunks shared by a block's waves (QBX_STAGED_SPLIT=0: off)
     DevBuf<double> la_X, la_F, la_P, la_Q, la_T, la_aux;   // density purification
@@ -246,15 +245,6 @@ struct TaskSet {
     int nbra = 0;
 };
 
-// Twin-bra groups of one ERI class (see TWIN_MAX): their ket lists, their
-// TWIN_MAX member bras and their tasks.
-struct TwinSet {
-    const int* klist = nullptr;
-    const int* gmem = nullptr;
-    const RowTask* rtask = nullptr;
-    int ngroup = 0, ntask = 0, twmax = 0;
-};
-
 struct HostShell {
     double c[3];
     int L, nprim, poff;
@@ -284,14 +274,7 @@ struct qbx_basis {
     int task_mode = -1;
     TaskSet t64[QBX_N_CLASSES], t32[QBX_N_CLASSES];
     double class_cost[QBX_N_CLASSES] = {};   // estimated work of each class (launch order)
-    // twin bras: groups of positions in each (Schwarz-sorted) pair class; for
-    // the J/K build of a class with groups, the other bras' task lists and
-    // the groups' own
-    std::vector<std::vector<int>> twins[QBX_N_PAIR_CLASSES];
-    bool use_twin[QBX_N_CLASSES] = {};
-    TaskSet s64[QBX_N_CLASSES];
-    TwinSet w64[QBX_N_CLASSES];
-    DevBuf<int> d_lists;       // their arrays
+    DevBuf<int> d_lists;       // arrays of the task sets
     DevBuf<double> ws[QBX_N_CLASSES];   // staged-class workspaces
     // work buffers
     DevBuf<double> d_D, d_JK, d_G;   // d_JK: J, K, and the ket sums in pair order
@@ -828,50 +811,6 @@ void attach_workspace(qbx_basis* b, int cls, int nwave, EriArgs& a)
     a.ws_slots = (int)(b->ws[cls].n / ((size_t)wsv * 64));
 }
 
-// Schwarz bounds, then every pair class sorted by descending bound.
-// Twin bras.  Shells that share centre, L and exponents form a family (the
-// segmented copies of a general contraction); shell pairs of one pair class
-// whose shells come from the same two families and that kept the same
-// primitive pairs have identical primitive geometry and differ only in the
-// c_a c_b factors.  Groups of up to TWIN_MAX such pairs, in Schwarz order.
-void find_twins(qbx_basis* b)
-{
-    const int ns = (int)b->shells.size();
-    std::map<std::vector<double>, int> fam_of;
-    std::vector<int> fam(ns);
-    for (int s = 0; s < ns; ++s) {
-        const HostShell& H = b->shells[s];
-        std::vector<double> key = {H.c[0], H.c[1], H.c[2], (double)H.L, (double)H.nprim};
-        for (int k = 0; k < H.nprim; ++k) key.push_back(b->pexp[H.poff + k]);
-        auto it = fam_of.find(key);
-        if (it == fam_of.end()) it = fam_of.emplace(key, (int)fam_of.size()).first;
-        fam[s] = it->second;
-    }
-    std::vector<int> copies(fam_of.size(), 0);
-    bool any = false;
-    for (int f : fam) any = ++copies[f] > 1 || any;
-    for (int c = 0; c < QBX_N_PAIR_CLASSES; ++c) {
-        const PairClass& P = b->pc[c];
-        std::map<std::vector<int>, std::vector<int>> sig;
-        for (int k = 0; any && k < P.n(); ++k) {
-            if (copies[fam[P.shA[k]]] * copies[fam[P.shB[k]]] < 2) continue;   // no other pair of these families
-            std::vector<int> key = {fam[P.shA[k]], fam[P.shB[k]], P.ppn[k]};
-            for (int u = 0; u < P.ppn[k]; ++u) key.push_back(b->ppk[P.ppo[k] + u]);
-            sig[key].push_back(k);
-        }
-        b->twins[c].clear();
-        for (auto& kv : sig) {
-            const std::vector<int>& m = kv.second;
-            for (size_t o = 0; o + 1 < m.size(); o += TWIN_MAX) {
-                const size_t e = std::min(m.size(), o + (size_t)TWIN_MAX);
-                if (e - o >= 2) b->twins[c].emplace_back(m.begin() + o, m.begin() + e);
-            }
-        }
-        std::sort(b->twins[c].begin(), b->twins[c].end(),
-                  [](const std::vector<int>& x, const std::vector<int>& y) { return x[0] < y[0]; });
-    }
-}
-
 bool high_class(int c) { return qbx_pair_class_l[c][0] > QBX_GEN_LMAX; }
 
 // The pairs of a class in plain Schwarz order.
@@ -918,6 +857,7 @@ void high_class_schwarz(qbx_basis* b, int c, DevBuf<double>& q, DevBuf<int64_t>&
     launch_eri_generic(g, MODE_SCHWARZ, st);
 }
 
+// Schwarz bounds, then every pair class by ket bucket and descending bound.
 void ensure_schwarz(qbx_basis* b)
 {
     if (b->schwarz) return;
@@ -1030,7 +970,6 @@ void ensure_schwarz(qbx_basis* b)
     }
     QBX_HIP(hipStreamSynchronize(st));
     b->schwarz = true;
-    find_twins(b);
 }
 
 // number of leading entries of a descending array that are >= v
@@ -1136,10 +1075,9 @@ private:
 // 64-ket waves, in a pool.
 class KetLists {
 public:
-    // room for n lists; the device pointers go to *klist and (unless null) *cpre
+    // room for n lists; the device pointers go to *klist and *cpre
     KetLists(ListPool& pool, const PairClass& ket, size_t n, const int** klist, const int** cpre)
-        : pool_(pool), ket_(ket), kl_(pool.add(n * (2 * ket.nbk + 1), klist)), cpre_(cpre ? pool.add(n + 1, cpre) : 0),
-          has_cpre_(cpre != nullptr)
+        : pool_(pool), ket_(ket), kl_(pool.add(n * (2 * ket.nbk + 1), klist)), cpre_(pool.add(n + 1, cpre))
     {
     }
     // one more list: of bucket k, the kets [lo[k], hi[k]) (lo null: from 0)
@@ -1157,7 +1095,7 @@ public:
         nwave += (n + 63) / 64;
         total += n;
         ++nl;
-        if (has_cpre_) pool_.data(cpre_)[nl] = nwave;
+        pool_.data(cpre_)[nl] = nwave;
     }
     const int* list(size_t i) const { return pool_.data(kl_) + i * (2 * ket_.nbk + 1); }
     int64_t total = 0;
@@ -1167,7 +1105,6 @@ private:
     ListPool& pool_;
     const PairClass& ket_;
     size_t kl_, cpre_;
-    bool has_cpre_;
 };
 
 // the lists of every bra of class cls: bucket k's kets [lo, hi) (per range; lo
@@ -1332,43 +1269,6 @@ std::vector<RowTask> row_tasks(const qbx_basis* b, int cls, const KetLists& L, T
     return out;
 }
 
-// Ket lists and tasks of the twin groups of class cls: the FP64 kets that every
-// member of a group keeps, [0, common) of each bucket.
-// Each member's kets beyond the common prefix, and all FP32 kets, stay with
-// the per-bra lists (start64 receives the common prefix of every member), so
-// the shared evaluation never covers a ket that a member would not.
-void add_twins(const qbx_basis* b, int cls, const RangeCounts& r, const TaskCaps& cap, ListPool& pool, TwinSet& w64,
-               std::vector<int>& start64)
-{
-    const PairClass& PX = pair_class(b, cls, 0);
-    const PairClass& PY = pair_class(b, cls, 1);
-    const int nk = PY.nbk;
-    const std::vector<std::vector<int>>& groups = b->twins[class_pc(cls, 0)];
-    KetLists L(pool, PY, groups.size(), &w64.klist, nullptr);
-    std::vector<int> mem, common(nk);
-    std::vector<RowTask> task;
-    w64.ngroup = w64.ntask = w64.twmax = 0;
-    TaskCutter cutter(PY, qbx_class_cost_prim[cls], qbx_class_cost_quartet[cls] * TWIN_MAX, cap, TWIN_WAVES, ROW_ITEMS);
-    for (const std::vector<int>& m : groups) {
-        int any = 0;
-        for (int k = 0; k < nk; ++k) {
-            common[k] = INT32_MAX;
-            for (int i : m) common[k] = std::min(common[k], r.c64()[(size_t)i * nk + k]);
-            any = std::max(any, common[k]);
-        }
-        if (any == 0) continue;
-        for (int i : m) std::copy(common.begin(), common.end(), start64.begin() + (size_t)i * nk);
-        for (size_t t = 0; t < (size_t)TWIN_MAX; ++t) mem.push_back(t < m.size() ? m[t] : -1);
-        L.add(nullptr, common.data());
-        cutter.add(w64.ngroup, L.list(w64.ngroup), PX.ppn[m[0]], task);
-        w64.twmax = std::max(w64.twmax, (int)m.size());
-        ++w64.ngroup;
-    }
-    w64.ntask = (int)task.size();
-    pool.add(mem, &w64.gmem);
-    pool.add(task, &w64.rtask);
-}
-
 void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
 {
     if (mode != QBX_PREC_MIXED) cut = 0.0;
@@ -1388,7 +1288,6 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
     ListPool pool(guess);
     for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
         const RangeCounts& r = rc[cls];
-        const int X = class_pc(cls, 0);
         const TaskCaps cap = task_caps(cls, b->class_cost[cls], total);
         // whole chunks in the FP32 lists: an FP32 integral is one sum, its
         // rounding the same whatever else the lists hold
@@ -1406,20 +1305,6 @@ void ensure_tasks(qbx_basis* b, double thr, int mode, double cut)
         };
         add(b->t64[cls], nullptr, r.c64(), cap);
         if (mode == QBX_PREC_MIXED) add(b->t32[cls], r.c64().data(), r.cnt, whole);
-        b->use_twin[cls] = false;
-        // only where bra and ket classes differ: within one pair class a bra's
-        // kets end at its own Schwarz-sorted position, so the members' common
-        // prefix is short and the group's fixed cost per block outweighs it
-        // (measured on 24 H2O in cc-pVDZ: (ps|ss) 27.8 -> 24.7 ms, while
-        // (ss|ss) 15.2 -> 16.0 and (ps|ps) 11.3 -> 12.0 ms)
-        if (b->ctx->twins && qbx_class_twin[cls] && X != class_pc(cls, 1) && !b->twins[X].empty()) {
-            std::vector<int> start64(r.cnt.size(), 0);
-            add_twins(b, cls, r, cap, pool, b->w64[cls], start64);
-            if (b->w64[cls].ngroup > 0) {
-                add(b->s64[cls], start64.data(), r.c64(), cap);
-                b->use_twin[cls] = true;
-            }
-        }
     }
     pool.upload(b->d_lists, b->ctx->stream);
     b->tasks_valid = true;
@@ -1710,16 +1595,7 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
         a.jp_set = npair_el;
         a.jp_stride = npair_el * nset;
         a.nset = nset;
-        // twin groups where their LDS rows ([set][member][A and B][N]) fit a block
-        bool twin = b->use_twin[cls] && ctx->jk_rows;
-        if (twin) {
-            const size_t rows = (size_t)nset * b->w64[cls].twmax *
-                                (qbx_ncart(qbx_class_l[cls][0]) + qbx_ncart(qbx_class_l[cls][1])) * b->nbf *
-                                sizeof(double);
-            const size_t boys = (size_t)QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE * sizeof(double);
-            twin = rows <= (size_t)ROW_LDS_MAX && rows + boys <= (size_t)ctx->lds_max;
-        }
-        auto set_tasks = [&](const TaskSet& t, const TwinSet* w) {
+        auto set_tasks = [&](const TaskSet& t) {
             a.klist = t.klist;
             a.cpre = t.cpre;
             // no K-row task lists: the one-wave-per-chunk kernels run
@@ -1729,23 +1605,17 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
             a.total = t.total;
             a.nwave = t.nwave;
             a.nbra = t.nbra;
-            a.gklist = w ? w->klist : nullptr;
-            a.gmem = w ? w->gmem : nullptr;
-            a.gtask = w ? w->rtask : nullptr;
-            a.ngroup = w ? w->ngroup : 0;
-            a.ntwtask = w ? w->ntask : 0;
-            a.twmax = w ? w->twmax : 0;
         };
         a.lds_max = ctx->lds_max;
-        const TaskSet& t64 = twin ? b->s64[cls] : b->t64[cls];
-        set_tasks(t64, twin ? &b->w64[cls] : nullptr);
+        const TaskSet& t64 = b->t64[cls];
+        set_tasks(t64);
         const TaskSet& t32 = b->t32[cls];
         int slots = std::max(t64.nwave, ROW_WAVES * t64.nsuper);
         if (mode == QBX_PREC_MIXED) slots = std::max(slots, std::max(t32.nwave, ROW_WAVES * t32.nsuper));
         attach_workspace(b, cls, slots, a);
         k_jk64[cls](a, ls);
         if (mode == QBX_PREC_MIXED) {
-            set_tasks(b->t32[cls], nullptr);
+            set_tasks(b->t32[cls]);
             k_jk32[cls](a, ls);
         }
         if (ctx->timing == 1) QBX_HIP(hipEventRecord(ev[2 * cls + 1], st));
@@ -1975,8 +1845,6 @@ int qbx_init(int32_t device, qbx_ctx** out)
             c->xcd_local = ok && n >= 2 && !off;
         }
         {
-            const char* env = std::getenv("QBX_TWINS");
-            c->twins = !(env && env[0] == '0');
             const char* benv = std::getenv("QBX_KET_BUCKETS");
             c->ket_buckets = !(benv && benv[0] == '0');
             const char* renv = std::getenv("QBX_JK_ROWS");

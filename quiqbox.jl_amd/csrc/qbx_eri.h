@@ -34,7 +34,7 @@ namespace qbx {
 template <typename T> using cptr = const __attribute__((address_space(4))) T*;
 template <typename T> __device__ __forceinline__ cptr<T> cst(const T* p) { return (cptr<T>)p; }
 
-// Ket list i (a bra's, or a twin group's): its ranges of the ket buckets, one
+// Ket list of bra i: its ranges of the ket buckets, one
 // after another, as nb pairs (first position, ket - position) and the length.
 // Only the list's last chunk of 64 is partial, and most others hold kets of one
 // primitive-pair count.
@@ -878,156 +878,6 @@ __device__ __forceinline__ void jk_rows_body(const EriArgs& a)
 }
 
 // ---------------------------------------------------------------------------
-// J/K for a group of twin bras.  A block of TWIN_WAVES waves takes one task of
-// the group's ket list, the kets that every member keeps.  The geometry and Boys
-// values of every primitive quartet are computed once, from the first member's
-// primitive pairs; each member accumulates them with its own c_a c_b factor (Kp)
-// and goes through the digest with its own shells and LDS K rows
-// [set][member][A and B functions][N].
-// ---------------------------------------------------------------------------
-template <int LA, int LB, int LC, int LD, typename R>
-__global__ __launch_bounds__(64 * TWIN_WAVES) void eri_jk_twin_kernel(EriArgs a)
-{
-    using Cls = EriClass<LA, LB, LC, LD, R>;
-    constexpr int TPB = 64 * TWIN_WAVES;
-    constexpr int NA = qbx_ncart(LA), NB = qbx_ncart(LB);
-    constexpr int LT = LA + LB + LC + LD;
-    constexpr int NCD = qbx_ncart(LC) * qbx_ncart(LD);
-    constexpr int NROW = NA + NB;
-    constexpr int TW = TWIN_MAX;
-    __shared__ double2 sboys[BOYS_HEAD2 + boys_rows(LT) * QBX_BOYSL_STRIDE / 2];
-    extern __shared__ double krow[];    // [nset][twmax][NROW][N]
-    const int Ni = a.N;
-    const int tw = a.twmax;
-    const int nrowel = a.nset * tw * NROW * Ni;
-    stage_boys<TPB, boys_rows(LT)>(sboys, a.boysl);
-    for (int i = threadIdx.x; i < nrowel; i += TPB) krow[i] = 0.0;
-    __syncthreads();
-    const double* sb = (const double*)sboys + BOYS_HEAD;
-
-    const int lane = (int)threadIdx.x & 63;
-    const int wib = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const cptr<RowTask> task = cst(a.gtask + blockIdx.x);
-    const int g = task->list;
-    const KetList kl(a.gklist, a.nbk, g);
-    const cptr<int> gm = cst(a.gmem + TW * g);
-    int bi[TW], sA[TW], sB[TW], ppo[TW];
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-        bi[t] = t < tw ? gm[t] : -1;
-        const int b = bi[t] < 0 ? bi[0] : bi[t];
-        sA[t] = cst(a.bra.shA)[b];
-        sB[t] = cst(a.bra.shB)[b];
-        ppo[t] = cst(a.bra.ppo)[b];
-    }
-    const int bn = cst(a.bra.ppn)[bi[0]];
-    const cptr<PrimPair> BP = cst(a.pp + ppo[0]);
-    const cptr<double> ABp = cst(a.bra.AB + 3 * bi[0]);
-    const R ABx = (R)ABp[0], ABy = (R)ABp[1], ABz = (R)ABp[2];
-    const JKSink sink(a);
-
-    for (int j = task->item0 + wib; j < task->item1; j += TWIN_WAVES) {
-        const RowItem it(task, j, bn);
-        const int pos = it.chunk * 64 + lane;
-        const bool inrange = pos < kl.n;
-        const int ki = kl.ket(inrange ? pos : 0);
-        const int sC = a.ket.shA[ki], sD = a.ket.shB[ki];
-        bool live[TW];
-        bool any = false;
-#pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            bool l = inrange && bi[t] >= 0;
-            if (l && a.pdmax) {
-                const double* dm = a.pdmax;
-                const int ns = a.nshell;
-                double d = fmax(fmax(dm[sA[t] * ns + sB[t]], dm[sC * ns + sD]),
-                                fmax(dm[sA[t] * ns + sC], dm[sA[t] * ns + sD]));
-                d = fmax(d, fmax(dm[sB[t] * ns + sC], dm[sB[t] * ns + sD]));
-                if (cst(a.bra.Q)[bi[t]] * a.ket.Q[ki] * d < a.dthr) l = false;
-            }
-            live[t] = l;
-            any = any || l;
-        }
-        const int kn = any ? a.ket.ppn[ki] : 0;
-        if (__ballot(kn > 0) == 0) continue;
-
-        R acc[TW][Cls::NACC];
-#pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int n = 0; n < Cls::NACC; ++n) acc[t][n] = (R)0;
-        int v0, vn;
-        it.ket_part(kn, v0, vn);
-        const PrimPair* KP = a.pp + a.ket.ppo[ki] + v0;
-        for (int v = 0; v < vn; ++v) {
-            const KetPrim Q = load_ket(KP + v);
-            for (int u = it.u0; u < it.u0 + it.un; ++u) {
-                const double p = BP[u].p, inv2p = BP[u].inv2p;
-                const double PQx = BP[u].Px - Q.Qx, PQy = BP[u].Py - Q.Qy, PQz = BP[u].Pz - Q.Qz;
-                const double pq = p + Q.q;
-                const double s = rsqrt_pos(pq);
-                const double inv = s * s;
-                const double rho = p * Q.q * inv;
-                const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);
-                const double pref0 = Q.Kq * s;
-                double Fd[LT + 1];
-                boys_lds<LT>(T, Fd, sb);
-                const double rho_p = Q.q * inv, rho_q = p * inv;
-#pragma unroll
-                for (int t = 0; t < TW; ++t) {
-                    if (bi[t] < 0) continue;
-                    const double w = live[t] ? pref0 * cst(a.pp + ppo[t])[u].Kp : 0.0;
-                    R F[LT + 1];
-#pragma unroll
-                    for (int m = 0; m <= LT; ++m) F[m] = (R)(Fd[m] * w);
-                    Cls::vrr(F, acc[t], (R)BP[u].PAx, (R)BP[u].PAy, (R)BP[u].PAz,
-                             (R)(-rho_p * PQx), (R)(-rho_p * PQy), (R)(-rho_p * PQz),
-                             (R)Q.QCx, (R)Q.QCy, (R)Q.QCz,
-                             (R)(rho_q * PQx), (R)(rho_q * PQy), (R)(rho_q * PQz),
-                             (R)inv2p, (R)Q.inv2q, (R)(0.5 * inv), (R)rho_p, (R)rho_q);
-                }
-            }
-        }
-        const double* CDp = a.ket.AB + 3 * ki;
-#pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            if (bi[t] < 0 || __ballot(live[t]) == 0) continue;
-            R kacc[Cls::NE * NCD];
-            Cls::hrr_ket(acc[t], kacc, (R)CDp[0], (R)CDp[1], (R)CDp[2]);
-            const cptr<DevShell> SA = cst(a.sh + sA[t]);
-            const cptr<DevShell> SB = cst(a.sh + sB[t]);
-            int fa[NA], fb[NB];
-#pragma unroll
-            for (int n = 0; n < NA; ++n) fa[n] = SA->bf[n] < 0 ? 0 : SA->bf[n];
-#pragma unroll
-            for (int n = 0; n < NB; ++n) fb[n] = SB->bf[n] < 0 ? 0 : SB->bf[n];
-            double f = live[t] ? 1.0 : 0.0;
-            if (sA[t] == sB[t]) f *= 0.5;
-            if (sC == sD) f *= 0.5;
-            if (a.same && bi[t] == ki) f *= 0.5;
-            digest_rows<LA, LB, LC, LD, R>(a, kacc, fa, fb, SA, SB, ABx, ABy, ABz, ki, sC, sD, f, live[t],
-                                           krow + t * NROW * Ni, tw * NROW * Ni, sink, lane);
-        }
-    }
-    __syncthreads();
-    // each nonzero row element to K once
-    const size_t N = (size_t)Ni;
-    for (int i = threadIdx.x; i < nrowel; i += TPB) {
-        const double v = krow[i];
-        if (v == 0.0) continue;
-        const int s = i / (tw * NROW * Ni);
-        int rem = i - s * tw * NROW * Ni;
-        const int t = rem / (NROW * Ni);
-        rem -= t * NROW * Ni;
-        const int row = rem / Ni, col = rem - row * Ni;
-        const int b = gm[t];
-        const int sh = row < NA ? cst(a.bra.shA)[b] : cst(a.bra.shB)[b];
-        const int fr = max(a.sh[sh].bf[row < NA ? row : row - NA], 0);
-        sink.add(sink.K + (size_t)s * N * N + (size_t)fr * N + col, v);
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Staged classes: the [e0|f0] set is too large for the register file, so each
 // group of bra components e makes its own pass over the primitive quartets
 // (the intermediates shared between groups are recomputed), transfers its
@@ -1601,29 +1451,6 @@ void launch_eri(const EriArgs& a, hipStream_t s)
         QBX_HIP(hipGetLastError());
     } else {
         if constexpr (MODE == MODE_JK) {
-            if (a.ngroup > 0) {
-                if constexpr (EriClass<LA, LB, LC, LD, R>::NACC <= TWIN_MAX_ACC) {
-                    const size_t tshm =
-                        (size_t)a.nset * a.twmax * (qbx_ncart(LA) + qbx_ncart(LB)) * a.N * sizeof(double);
-                    static const bool twin_ok = [] {
-                        const bool ok = hipFuncSetAttribute((const void*)eri_jk_twin_kernel<LA, LB, LC, LD, R>,
-                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                            ROW_LDS_MAX) == hipSuccess;
-                        (void)hipGetLastError();
-                        return ok;
-                    }();
-                    if (!twin_ok || tshm > (size_t)ROW_LDS_MAX ||
-                        tshm + QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE * sizeof(double) > (size_t)a.lds_max)
-                        throw QbxError(QBX_EINTERNAL, "twin-bra groups given where their LDS rows do not fit");
-                    if (a.ntwtask > 0) {
-                        hipLaunchKernelGGL((eri_jk_twin_kernel<LA, LB, LC, LD, R>), dim3((unsigned)a.ntwtask),
-                                           dim3(64 * TWIN_WAVES), tshm, s, a);
-                        QBX_HIP(hipGetLastError());
-                    }
-                } else {
-                    throw QbxError(QBX_EINTERNAL, "twin-bra groups given to a class without a twin kernel");
-                }
-            }
             const size_t shm = (size_t)a.nset * (qbx_ncart(LA) + qbx_ncart(LB)) * a.N * sizeof(double);
             const size_t boys_lds = QBX_BOYSL_ROWS * QBX_BOYSL_STRIDE * sizeof(double);
             // the attribute call fails where the device cannot give a block

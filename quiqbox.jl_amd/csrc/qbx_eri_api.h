@@ -13,15 +13,14 @@ enum EriMode { MODE_JK = 0, MODE_DENSE = 1, MODE_SCHWARZ = 2 };
 #define QBX_ROW_WAVES 4
 #endif
 constexpr int ROW_WAVES = QBX_ROW_WAVES;
-// One K-row task (one block): items item0 .. item1 - 1 of a list (a bra, or a
-// group of twin bras).  Item j is the 64-ket chunk chunk0 + j / (kparts bparts)
+// One K-row task (one block): items item0 .. item1 - 1 of bra `list`.  Item j is the 64-ket chunk chunk0 + j / (kparts bparts)
 // with one of kparts parts of every ket's primitive pairs and one of bparts parts
 // of the bra's: the digest is linear in the integrals, so the waves that share a
 // heavy chunk each digest the integrals of their own primitive quartets.
 struct RowTask {
     int list, chunk0, kparts, bparts, item0, item1;
 };
-// Most items per task of the low-L K-row and twin kernels, and of the staged
+// Most items per task of the low-L K-row kernels, and of the staged
 // K-row kernel (whose waves are long, so that smaller tasks balance better).
 // Fewer and larger tasks flush fewer K rows: with chunks alone as items, 24 H2O
 // in cc-pVDZ took 50.9 ms per build at 16 and 49.6 at 32, the 592-function
@@ -30,15 +29,6 @@ struct RowTask {
 constexpr int ROW_ITEMS = 32;
 constexpr int STAGED_ROW_ITEMS = 8;
 constexpr int ROW_LDS_MAX = 64 * 1024;
-// Twin bras: shell pairs of one pair class with the same primitive geometry
-// and primitive pairs, differing only in contraction coefficients (shells
-// that share centre, L and exponents, as the 1s and 2s contractions of
-// cc-pVDZ oxygen).  A group of up to TWIN_MAX of them is evaluated together
-// by classes with at most TWIN_MAX_ACC accumulators.
-constexpr int TWIN_MAX = 4;
-constexpr int TWIN_WAVES = 8;   // waves per block of the twin kernel (its K rows take up to 61 KB of LDS)
-constexpr int TWIN_MAX_ACC = 9;
-
 struct PairClassDev {
     int n;
     const int* shA;
@@ -60,12 +50,6 @@ struct EriArgs {
     const int* cpre;          // [nbra+1] prefix over bras of ceil(kets / 64): waves
     const RowTask* rtask;     // K-row tasks of the bras (null: the one-wave-per-chunk kernels run)
     int nsuper;               // their number
-    const int* gklist;        // [ngroup][2 nbk + 1]: ket lists of the twin groups
-    const int* gmem;          // [ngroup][TWIN_MAX] bras of a group (-1: no member)
-    const RowTask* gtask;     // tasks of the twin groups
-    int ngroup;               // twin groups of this class (0: none)
-    int ntwtask;              // their tasks
-    int twmax;                // largest group (LDS rows per set)
     int nbk;                  // ket buckets of the class
     int lds_max;              // LDS bytes a block may use on this device
     int64_t total;            // Schwarz mode: number of diagonal pairs
