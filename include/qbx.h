@@ -276,8 +276,8 @@ int  qbx_density_purify_noalloc(qbx_ctx* ctx, int32_t n, int32_t nocc, const dou
    (solveFockMatrix, HartreeFock.jl:46-59; getD :296-302).  eigen(X' F X)
    ascending, C = X C' with each column's sign fixed so that C[0][j] >= 0,
    D = C[:, :nocc] C[:, :nocc]^T; X' F X, X C' and D are FP64 matrix-core
-   GEMMs and the symmetric eigenproblem is rocSOLVER's divide and conquer
-   (dsyevd).  Host arrays, n x n row-major (X and F symmetric); eps (n) and
+   GEMMs; the symmetric eigenproblem is reduced by an own kernel (n >= 96) and
+   solved by rocSOLVER's divide and conquer.  Host arrays, n x n row-major (X and F symmetric); eps (n) and
    D may be NULL.  QBX_ENOCONV if the eigensolver does not converge. */
 int  qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const double* F, double* C,
                     double* eps, double* D);

@@ -119,7 +119,7 @@ struct JKSink {
 };
 
 // Threads per block: classes with few accumulators (and so few registers) run
-// 8 or 16 waves per block, so that one LDS copy of the Boys rows (23 KB, six
+// 8 or 16 waves per block, so that one LDS copy of the Boys rows (19 KB, eight
 // copies fit a CU) serves more waves.
 __host__ __device__ constexpr int eri_tpb(int nacc) { return nacc <= 3 ? 1024 : nacc <= 18 ? 512 : 256; }
 
@@ -129,7 +129,7 @@ __host__ __device__ constexpr int eri_tpb(int nacc) { return nacc <= 3 ? 1024 : 
 // (relative error below 4e-17 from the first grid point past 35.5, 39.75,
 // 43.25, 46.25, 49, 51.75, 54.25, 56.75 and 59 against 40-digit values,
 // falling as e^{-T} beyond), so a kernel of total angular momentum L stages
-// only the rows below T_L: 14 KB of LDS instead of 23 KB at L = 0, more
+// only the rows below T_L: 12 KB of LDS instead of 19 KB at L = 0, more
 // resident blocks to hide the latency of the lookup.
 constexpr double kBoysTmax[QBX_BOYSL_LMAX + 1] = {36.0, 40.0, 44.0, 47.0, 50.0, 52.0, 55.0, 57.0, 60.0, 60.0};
 constexpr double boys_tmax(int L) { return kBoysTmax[L]; }
