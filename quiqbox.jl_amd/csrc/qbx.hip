@@ -1136,16 +1136,18 @@ double class_cost(const qbx_basis* b, int cls, const RangeCounts& r)
 // Sizes of K-row tasks, in operations of the cost model per lane: an item (a
 // chunk, or a part of one) is cut to about `item`, a wave's share of a task to
 // about `task`.  cost: the class's estimate, total: all classes' (over 64 lanes).
-// A chunk is split where it would take a wave longer than half of the time that
-// its class needs on a full chip, or than an eighth of what the build does: the
+// A chunk is split where it would take a wave longer than 4/3 of the time that
+// its class needs on a full chip and than an eighth of what the build does: the
 // few chunks of contracted core pairs (81 x 81 primitive quartets against a mean
 // of 82 in 24 H2O) otherwise end each class's launch on a few waves.  Below
 // kLeastItem operations and four times the digest's, an item's fixed part
 // outweighs what it shares.  A wave's share of a task is at most its share of
 // the class.  Measured per build with the chunks of one bucket and 32 chunks a
 // task before: 8 H2O UHF 5.45 -> 3.34 ms, 24 H2O 45.9 -> 35.5, the 592-function
-// cluster 33.4 -> 28.3, 64 atoms of s/p 2.19 -> 1.73; halving or doubling any of
-// the factors moves them by at most 3%.
+// cluster 33.4 -> 28.3, 64 atoms of s/p 2.19 -> 1.73.  Half of the class's time in
+// place of 4/3 splits where the chip is full: UHF builds of 30 and 36 s/p atoms 543
+// against 459 and 662 against 570 us, of 80 s/p/d atoms 3.20 against 2.96 ms; the
+// whole gave 8 H2O UHF 2.87 ms against 2.82 at half and 4/3.
 struct TaskCaps {
     double item, task;
 };
@@ -1157,7 +1159,7 @@ TaskCaps task_caps(int cls, double cost, double total)
     const double waves = 1024.0 * (cp < 300 ? 4 : cp < 1200 ? 2 : 1);   // resident on the chip, by register use
     const double least = kLeastItem + 4.0 * qbx_class_cost_quartet[cls];
     TaskCaps c;
-    c.item = std::max(least, std::max(cost / (64 * 2 * waves), total / (64 * 8 * 4096.0)));
+    c.item = std::max(least, std::max(cost / (64 * 0.75 * waves), total / (64 * 8 * 4096.0)));
     c.task = std::max(least, cost / (64 * waves));
     return c;
 }
