@@ -280,9 +280,9 @@ struct qbx_basis {
     DevBuf<double> d_D, d_JK, d_G;   // d_JK: J, K, and the ket sums in pair order
     DevBuf<double> d_pdmax;        // shell-pair max |D| for density screening
     // end of the last Fock build (recorded on its stream after the
-    // symmetrization) and that stream: a build on another stream, and every
-    // rewrite of the task lists, waits for it before it touches the shared
-    // buffers (D, J, K, task lists, workspaces)
+    // symmetrization) and that stream: a build on another stream, a dense
+    // tensor and every rewrite of the task lists wait for it before they touch
+    // the shared buffers (D, J, K, task lists, workspaces)
     hipEvent_t ev_done = nullptr;
     hipStream_t last_stream = nullptr;
     bool built = false;
@@ -1380,9 +1380,9 @@ template <class Fill> void launch_high(const qbx_basis* b, int mode, hipStream_t
     }
 }
 
-// Before a Fock build on stream st touches the basis's work buffers: a
-// previous build still running on another stream must finish first (stream
-// order covers a build on the same stream).
+// Before a Fock build or a dense tensor on stream st touches the basis's work
+// buffers: a previous build still running on another stream must finish first
+// (stream order covers a build on the same stream).
 void order_after_last_build(qbx_basis* b, hipStream_t st)
 {
     if (b->built && b->last_stream != st) QBX_HIP(hipEventSynchronize(b->ev_done));
@@ -2155,6 +2155,8 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
         QBX_HIP(hipSetDevice(ctx->device));
         hipStream_t st = ctx->stream;
         ensure_schwarz(b);
+        // the staged classes' workspaces are the Fock build's
+        order_after_last_build(b, st);
         const size_t N = b->nbf, N4 = N * N * N * N;
         DevBuf<double> d;
         d.ensure(N4);
