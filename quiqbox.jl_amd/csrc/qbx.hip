@@ -61,17 +61,27 @@ template <typename T> struct DevBuf {
         p = nullptr;
         n = 0;
     }
-    void ensure(size_t cnt)
+    hipError_t grow(size_t cnt)
     {
-        if (cnt <= n && p) return;
+        if (cnt <= n && p) return hipSuccess;
         release();
         size_t c = cnt ? cnt : 1;
         hipError_t e = hipMalloc((void**)&p, c * sizeof(T));
-        if (e != hipSuccess) {
-            p = nullptr;
-            throw QbxError(QBX_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-        }
-        n = c;
+        if (e != hipSuccess) p = nullptr;
+        else n = c;
+        return e;
+    }
+    void ensure(size_t cnt)
+    {
+        const hipError_t e = grow(cnt);
+        if (e != hipSuccess) throw QbxError(QBX_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
+    // false where there is no memory: for callers that can do without
+    bool try_ensure(size_t cnt)
+    {
+        const bool ok = grow(cnt) == hipSuccess;
+        if (!ok) (void)hipGetLastError();
+        return ok;
     }
     void upload(const std::vector<T>& v, hipStream_t s)
     {
@@ -2349,10 +2359,10 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
             QBX_HIP(hipStreamSynchronize(st));
         };
         bool own = false;
-        if (n >= kTridiagMin) {
-            ctx->la_x.ensure(tridiag_exchange(n));
+        const TridiagPlan plan = n >= kTridiagMin ? tridiag_plan(n) : TridiagPlan();
+        if (plan.blocks > 0 && ctx->la_x.try_ensure(tridiag_exchange(n))) {
             zero_async(dQ, nn, st);
-            own = tridiagonalize(n, dP, dQ, dE, dOff, dTau, ctx->la_x.p, dInfo + 1, st);
+            own = tridiagonalize(plan, dP, dQ, dE, dOff, dTau, ctx->la_x.p, dInfo + 1, st);
         }
         if (own) {
             double* back = dTau + (n - 1);   // there are n - 1 factors

@@ -58,16 +58,24 @@ void sp2_product(const double* P, double* Q, int n, int nocc, int k, double* sha
 // state and measures after k launches of sp2_product
 void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2Status* out, hipStream_t s);
 
+// Launch of the tridiagonalization of order n on the current device; no blocks where
+// the matrix does not fit the device's LDS or the device cannot run the whole grid at
+// once (above order 1850 with 256 CUs and 160 KB of LDS).
+struct TridiagPlan {
+    int n = 0, blocks = 0, threads = 0;
+    size_t shm = 0;
+};
+TridiagPlan tridiag_plan(int n);
+
 // Householder tridiagonalization of the symmetric n x n matrix A (LAPACK's lower
 // form): diagonal d (n), off-diagonal e (n - 1), reflector k (its first entry, 1,
 // left out) in V[k n + k + 2 ...], factors tau (n - 1).  exchange: tridiag_exchange(n)
-// values of work space.  false where the matrix does not fit the device's LDS or
-// the device cannot run the whole grid at once (nothing is launched then).  *status
-// (device) is 0, or 1 when a block gave up waiting for another: the outputs are
-// not valid then.
+// values of work space.  false where nothing was launched (no blocks, or the launch
+// was refused).  *status (device) is 0, or 1 when a block gave up waiting for
+// another: the outputs are not valid then.
 size_t tridiag_exchange(int n);
-bool tridiagonalize(int n, const double* A, double* V, double* d, double* e, double* tau, uint64_t* exchange,
-                    int* status, hipStream_t s);
+bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double* d, double* e, double* tau,
+                    uint64_t* exchange, int* status, hipStream_t s);
 
 // The tridiagonal matrix times a power of two, its largest entry in [1, 2) (the
 // divide and conquer solver drops what is small in absolute terms), and the

@@ -663,7 +663,7 @@ void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2St
 // ---------------------------------------------------------------------------
 constexpr uint64_t TRI_EMPTY = ~0ull;
 constexpr int TRI_SPINS = 1 << 20;
-constexpr int TRI_MAX_N = 2048;   // 1024 threads, two elements each
+constexpr int TRI_MAX_N = 2048;   // 1024 threads, two elements each; 160 KB of LDS a block end at 1850
 
 size_t tridiag_exchange(int n) { return 2 * (size_t)n * n; }
 
@@ -872,19 +872,18 @@ __global__ __launch_bounds__(1024) void tridiag_kernel(int n, const double* A, d
     }
 }
 
-bool tridiagonalize(int n, const double* A, double* V, double* d, double* e, double* tau, uint64_t* exchange,
-                    int* status, hipStream_t s)
+TridiagPlan tridiag_plan(int n)
 {
-    if (n < 2 || n > TRI_MAX_N) return false;
+    TridiagPlan plan;
+    if (n < 2 || n > TRI_MAX_N) return plan;
     int dev = 0, cus = 0, coop = 0, lds_max = 0;
     QBX_HIP(hipGetDevice(&dev));
     QBX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     QBX_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     QBX_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    if (!coop || cus <= 0) return false;
+    if (!coop || cus <= 0) return plan;
     const int threads = std::min(1024, (n + 63) / 64 * 64);
-    const bool two = n > 1024;
-    const void* f = two ? (const void*)tridiag_kernel<2> : (const void*)tridiag_kernel<1>;
+    const void* f = n > 1024 ? (const void*)tridiag_kernel<2> : (const void*)tridiag_kernel<1>;
     // the fewest blocks whose LDS holds the matrix: each value then has fewer readers
     // (n = 600: 64, 128 and 256 blocks 7.47, 7.64 and 7.95 ms a solve)
     int B = 64;
@@ -893,23 +892,34 @@ bool tridiagonalize(int n, const double* A, double* V, double* d, double* e, dou
         B = std::min(std::min(B, cus), n);
         shm = ((size_t)((n + B - 1) / B) + 3) * n * sizeof(double);
         if (shm + 1024 <= (size_t)lds_max) break;
-        if (B >= 256 || B >= cus || B >= n) return false;
-    }
-    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
+        if (B >= 256 || B >= cus || B >= n) return plan;
     }
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, threads, shm) != hipSuccess || per_cu * cus < B) {
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, threads, shm) != hipSuccess || per_cu * cus < B) {
         (void)hipGetLastError();
-        return false;
+        return plan;
     }
+    plan.n = n;
+    plan.blocks = B;
+    plan.threads = threads;
+    plan.shm = shm;
+    return plan;
+}
+
+bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double* d, double* e, double* tau,
+                    uint64_t* exchange, int* status, hipStream_t s)
+{
+    if (plan.blocks <= 0) return false;
+    int n = plan.n;
+    const void* f = n > 1024 ? (const void*)tridiag_kernel<2> : (const void*)tridiag_kernel<1>;
     const size_t nx = tridiag_exchange(n);
     hipLaunchKernelGGL(tri_empty_kernel, dim3((unsigned)std::min<size_t>((nx + 255) / 256, 2048)), dim3(256), 0, s,
                        exchange, nx, status);
     QBX_HIP(hipGetLastError());
     void* args[] = {&n, &A, &V, &d, &e, &tau, &exchange, &status};
-    if (hipLaunchCooperativeKernel(f, dim3(B), dim3(threads), args, (unsigned)shm, s) != hipSuccess) {
+    if (hipLaunchCooperativeKernel(f, dim3(plan.blocks), dim3(plan.threads), args, (unsigned)plan.shm, s) !=
+        hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
