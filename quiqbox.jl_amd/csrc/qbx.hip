@@ -222,6 +222,7 @@ struct qbx_ctx {
     DevBuf<double> la_X, la_F, la_P, la_Q, la_T, la_aux;   // density purification
     HostCopier copier;             // large host arrays
     DevBuf<uint64_t> la_x;         // exchange of the tridiagonalization
+    int tri_spins = TRI_SPINS;     // its bounded wait (QBX_TRIDIAG_SPINS: another bound)
     double* scratch = nullptr;     // this device's address of the fixed work array
     rocblas_handle blas = nullptr; // rocSOLVER's handle (qbx_fock_solve), created on first use
     std::mutex mu;
@@ -1863,6 +1864,7 @@ int qbx_init(int32_t device, qbx_ctx** out)
             c->jk_rows = !(renv && renv[0] == '0');
             const char* senv = std::getenv("QBX_STAGED_SPLIT");
             c->staged_split = !(senv && senv[0] == '0');
+            if (const char* tenv = std::getenv("QBX_TRIDIAG_SPINS")) c->tri_spins = std::max(0, std::atoi(tenv));
         }
         QBX_HIP(hipStreamSynchronize(c->stream));
         *out = c.release();
@@ -2353,16 +2355,22 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
         // eigenpairs, ascending; the column-major eigenvector matrix V read
         // row-major is V^T
         const double* dV = dP;
-        rocblas_int info[2] = {0, 0};
+        rocblas_int info = 0;
         auto read_info = [&](int k) {
-            QBX_HIP(hipMemcpyAsync(info, dInfo, k * sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
+            QBX_HIP(hipMemcpyAsync(&info, dInfo + k, sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
             QBX_HIP(hipStreamSynchronize(st));
+            return info;
         };
         bool own = false;
         const TridiagPlan plan = n >= kTridiagMin ? tridiag_plan(n) : TridiagPlan();
         if (plan.blocks > 0 && ctx->la_x.try_ensure(tridiag_exchange(n))) {
             zero_async(dQ, nn, st);
-            own = tridiagonalize(plan, dP, dQ, dE, dOff, dTau, ctx->la_x.p, dInfo + 1, st);
+            own = tridiagonalize(plan, dP, dQ, dE, dOff, dTau, ctx->la_x.p, dInfo + 1, ctx->tri_spins, st);
+        }
+        if (own) {
+            // a block that gave up waiting leaves its outputs unwritten, and the solver
+            // must not see them: the library's own reduction runs instead
+            own = read_info(1) == 0;
         }
         if (own) {
             double* back = dTau + (n - 1);   // there are n - 1 factors
@@ -2373,18 +2381,13 @@ int qbx_fock_solve(qbx_ctx* ctx, int32_t n, int32_t nocc, const double* X, const
                                  dTau, dT, n) != rocblas_status_success)
                 throw QbxError(QBX_EINTERNAL, "rocsolver_dstedc or rocsolver_dormtr failed");
             tridiag_unscale(n, dE, back, st);
-            read_info(2);
-            own = info[1] == 0;   // else a block gave up waiting: the library's own reduction
             dV = dT;
-        }
-        if (!own) {
+        } else {
             if (rocsolver_dsyevd(ctx->blas, rocblas_evect_original, rocblas_fill_upper, n, dP, n, dE, dOff, dInfo) !=
                 rocblas_status_success)
                 throw QbxError(QBX_EINTERNAL, "rocsolver_dsyevd failed");
-            read_info(1);
-            dV = dP;
         }
-        if (info[0] != 0) throw QbxError(QBX_ENOCONV, "the symmetric eigensolver did not converge");
+        if (read_info(0) != 0) throw QbxError(QBX_ENOCONV, "the symmetric eigensolver did not converge");
         // C = X V with every column's first entry made non-negative
         gemm_f64(false, true, n, n, n, 1.0, dX, n, dV, n, 0.0, nullptr, 0, dQ, n, st);
         fix_column_signs(dQ, n, dSgn, st);

@@ -72,10 +72,11 @@ TridiagPlan tridiag_plan(int n);
 // left out) in V[k n + k + 2 ...], factors tau (n - 1).  exchange: tridiag_exchange(n)
 // values of work space.  false where nothing was launched (no blocks, or the launch
 // was refused).  *status (device) is 0, or 1 when a block gave up waiting for
-// another: the outputs are not valid then.
+// another after `spins` more polls of a value: the outputs are partly unwritten then.
+constexpr int TRI_SPINS = 1 << 20;
 size_t tridiag_exchange(int n);
 bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double* d, double* e, double* tau,
-                    uint64_t* exchange, int* status, hipStream_t s);
+                    uint64_t* exchange, int* status, int spins, hipStream_t s);
 
 // The tridiagonal matrix times a power of two, its largest entry in [1, 2) (the
 // divide and conquer solver drops what is small in absolute terms), and the

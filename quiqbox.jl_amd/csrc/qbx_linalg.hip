@@ -658,11 +658,10 @@ void sp2_status(const double* shares, int n, int k, const Sp2State* state, Sp2St
 // TRI_EMPTY before the launch, and a reader polls until it holds something else.
 // Values cross the XCDs, so they are stored and loaded at agent scope.  A NaN is
 // published as the plain quiet NaN, which is not TRI_EMPTY.  The launch is
-// cooperative (all blocks resident), and a block that has polled TRI_SPINS times
-// sets *status and ends; the others then end the same way.
+// cooperative (all blocks resident), and a block that has polled one value `spins`
+// times more sets *status and ends; the others then end the same way.
 // ---------------------------------------------------------------------------
 constexpr uint64_t TRI_EMPTY = ~0ull;
-constexpr int TRI_SPINS = 1 << 20;
 constexpr int TRI_MAX_N = 2048;   // 1024 threads, two elements each; 160 KB of LDS a block end at 1850
 
 size_t tridiag_exchange(int n) { return 2 * (size_t)n * n; }
@@ -695,7 +694,7 @@ __device__ __forceinline__ double tri_wave_sum(double v)
 // threadIdx.x + e * blockDim.x.
 template <int E>
 __global__ __launch_bounds__(1024) void tridiag_kernel(int n, const double* A, double* V, double* d, double* e_out,
-                                                       double* tau_out, uint64_t* exchange, int* status)
+                                                       double* tau_out, uint64_t* exchange, int* status, int spins)
 {
     extern __shared__ double lds[];
     __shared__ double red[3][16];
@@ -744,7 +743,7 @@ __global__ __launch_bounds__(1024) void tridiag_kernel(int n, const double* A, d
 #pragma unroll
             for (int q = 0; q < E; ++q) {
                 const int r = tid + q * T;
-                for (int i = 0; i < TRI_SPINS && (up[q] == TRI_EMPTY || ux[q] == TRI_EMPTY); ++i) {
+                for (int i = 0; i < spins && (up[q] == TRI_EMPTY || ux[q] == TRI_EMPTY); ++i) {
                     up[q] = tri_get(in + r);
                     ux[q] = tri_get(in + n + r);
                 }
@@ -908,7 +907,7 @@ TridiagPlan tridiag_plan(int n)
 }
 
 bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double* d, double* e, double* tau,
-                    uint64_t* exchange, int* status, hipStream_t s)
+                    uint64_t* exchange, int* status, int spins, hipStream_t s)
 {
     if (plan.blocks <= 0) return false;
     int n = plan.n;
@@ -917,7 +916,7 @@ bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double*
     hipLaunchKernelGGL(tri_empty_kernel, dim3((unsigned)std::min<size_t>((nx + 255) / 256, 2048)), dim3(256), 0, s,
                        exchange, nx, status);
     QBX_HIP(hipGetLastError());
-    void* args[] = {&n, &A, &V, &d, &e, &tau, &exchange, &status};
+    void* args[] = {&n, &A, &V, &d, &e, &tau, &exchange, &status, &spins};
     if (hipLaunchCooperativeKernel(f, dim3(plan.blocks), dim3(plan.threads), args, (unsigned)plan.shm, s) !=
         hipSuccess) {
         (void)hipGetLastError();
