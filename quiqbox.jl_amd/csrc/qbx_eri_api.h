@@ -125,6 +125,7 @@ struct GenArgs {
     int nbra;
     int same;                 // bra and ket are one class
     int64_t total;            // quartets (blocks)
+    int64_t first;            // this launch's first one (set by the launcher)
     const int64_t* prefix;    // [nbra + 1]
     int N;
     // J/K mode (as EriArgs)

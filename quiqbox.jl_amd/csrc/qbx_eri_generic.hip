@@ -321,7 +321,7 @@ __global__ __launch_bounds__(TS * W) void eri_md_kernel(GenArgs a)
     }
 
     // shell quartet of this block
-    const int64_t task = (int64_t)blockIdx.x;
+    const int64_t task = a.first + (int64_t)blockIdx.x;
     int lo = 0, hi = a.nbra;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -553,14 +553,20 @@ __global__ __launch_bounds__(TS * W) void eri_md_kernel(GenArgs a)
     }
 }
 
-template <int NSLOT, int TS, int W> void launch_slots(const GenArgs& a, size_t shm, int mode, hipStream_t s)
+// One block a quartet; a grid holds below 2^32 threads (16.8 million blocks of 256), so
+// longer lists take several launches.
+template <int NSLOT, int TS, int W> void launch_slots(GenArgs a, size_t shm, int mode, hipStream_t s)
 {
-    if (a.total > 0x7fffffffLL) throw QbxError(QBX_EUNSUP, "too many high angular momentum quartets for one grid");
+    constexpr int64_t MAX_BLOCKS = 0xffffffffLL / (TS * W);
     auto go = [&](void (*kern)(GenArgs)) {
         // above 64 KB the limit has to be raised
         if (shm > 64 * 1024)
             QBX_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        hipLaunchKernelGGL(kern, dim3((unsigned)a.total), dim3(TS * W), shm, s, a);
+        for (a.first = 0; a.first < a.total; a.first += MAX_BLOCKS) {
+            const int64_t n = std::min(a.total - a.first, MAX_BLOCKS);
+            hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(TS * W), shm, s, a);
+            QBX_HIP(hipGetLastError());
+        }
     };
     switch (mode) {
     case MODE_JK: go(eri_md_kernel<NSLOT, MODE_JK, TS, W>); break;
@@ -568,7 +574,6 @@ template <int NSLOT, int TS, int W> void launch_slots(const GenArgs& a, size_t s
     case MODE_SCHWARZ: go(eri_md_kernel<NSLOT, MODE_SCHWARZ, TS, W>); break;
     default: throw QbxError(QBX_EINTERNAL, "unknown ERI mode");
     }
-    QBX_HIP(hipGetLastError());
 }
 
 // Primitive quartets one thread each (unit coefficients): the reference's
