@@ -204,6 +204,7 @@ struct qbx_ctx {
         hipEvent_t beg_l[QBX_N_CLASSES], end_l[QBX_N_CLASSES], beg_s[QBX_N_CLASSES], end_s[QBX_N_CLASSES];
         hipEvent_t b0, b1;
         bool pending;
+        bool forked;               // the classes' own streams were not the main one
     };
     std::vector<TimingSet> tsets;
     int tnext = 0;
@@ -1518,8 +1519,8 @@ void run_one_e(qbx_ctx* ctx, const qbx_basis* b, int kind, int nnuc, const doubl
 
 // Concurrent per-class timing: sum the per-class durations of a recorded
 // event set (each class's stretch on its auxiliary stream plus its stretch on
-// the main stream, where kernels that spill are launched) into the context's
-// accumulators.
+// the main stream, where kernels that spill are launched; the two are one stretch
+// in a build that did not fork) into the context's accumulators.
 void drain_timing_set(qbx_ctx* ctx, qbx_ctx::TimingSet& T)
 {
     if (!T.pending) return;
@@ -1528,7 +1529,7 @@ void drain_timing_set(qbx_ctx* ctx, qbx_ctx::TimingSet& T)
     for (int cls = 0; cls < QBX_N_CLASSES; ++cls) {
         float l = 0.f, m = 0.f;
         QBX_HIP(hipEventElapsedTime(&l, T.beg_l[cls], T.end_l[cls]));
-        QBX_HIP(hipEventElapsedTime(&m, T.beg_s[cls], T.end_s[cls]));
+        if (T.forked) QBX_HIP(hipEventElapsedTime(&m, T.beg_s[cls], T.end_s[cls]));
         ctx->tsum[cls] += (double)l + (double)m;
     }
     float tot = 0.f;
@@ -1647,6 +1648,7 @@ void jk_device(qbx_ctx* ctx, qbx_basis* b, int nset, const double* dD, double* d
     size_t parallel = b->has_high ? b->hl.sets.size() : 0;
     for (int cls = 0; cls < QBX_N_CLASSES; ++cls) parallel += occupied(cls);
     const bool fork = ctx->timing != 1 && parallel > 1;
+    if (T) T->forked = fork;
     if (fork) {
         QBX_HIP(hipEventRecord(ctx->ev_fork, st));
         for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
