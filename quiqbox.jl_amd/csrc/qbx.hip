@@ -2203,14 +2203,22 @@ int qbx_eri_dense(qbx_ctx* ctx, const qbx_basis* bc, double* eri)
         pool.upload(lists, st);
         ensure_hl_tasks(b, 0.0);
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-        QBX_HIP(hipEventRecord(ctx->ev_fork, st));
-        for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
-        for (size_t k = 0; k < order.size(); ++k) k_dense[order[k]](args[order[k]], ctx->aux[k % kStreams]);
-        if (b->has_high) launch_high(b, MODE_DENSE, ctx->aux, kStreams, [&](GenArgs& g) { g.eri = d.p; });
-        for (int k = 0; k < kStreams; ++k) {
-            QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
-            QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
+        // one launch stays on the main stream, as in a Fock build (two functions: 101 us
+        // with the fork, 53 without)
+        const bool fork = order.size() + b->hl.sets.size() > 1;
+        if (fork) {
+            QBX_HIP(hipEventRecord(ctx->ev_fork, st));
+            for (int k = 0; k < kStreams; ++k) QBX_HIP(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
         }
+        for (size_t k = 0; k < order.size(); ++k)
+            k_dense[order[k]](args[order[k]], fork ? ctx->aux[k % kStreams] : st);
+        if (b->has_high)
+            launch_high(b, MODE_DENSE, fork ? ctx->aux : &st, fork ? kStreams : 1, [&](GenArgs& g) { g.eri = d.p; });
+        if (fork)
+            for (int k = 0; k < kStreams; ++k) {
+                QBX_HIP(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
+                QBX_HIP(hipStreamWaitEvent(st, ctx->ev_join[k], 0));
+            }
         ctx->copier.to_host(ctx->device, eri, d.p, N4 * sizeof(double), st);
     });
 }
