@@ -163,10 +163,22 @@ __device__ __forceinline__ void mfma_16k(const dbl4* a, const dbl4* b, dbl4 (*ac
 // compiler waited for all of them at every step: 27 us at 600^3).  Against four
 // waves on one 16 x 16 tile each and K through LDS, two barriers every 16 k: 600^3
 // 27.8 -> 22 us, 301^3 10.3 -> 7.8, 1024^3 61.6 -> 53, 70 x 4900 x 4900 187 -> 124.
-// Below KSPLIT_MIN the other form is as fast or faster (20000 x 33 x 33: 7.0
-// against 9.1 us).
+// Which form takes a product (split_k) follows from times of both at 100 to 3600
+// tiles and K of 256 to 6000: below KSPLIT_MIN the other is as fast or faster (20000 x
+// 33 x 33: 7.0 against 9.1 us); many tiles fill the chip without splitting K, and a
+// short K then does not pay for the sum over the waves (20000 x 33 x 300, 1250 tiles:
+// 40 us against 34; 60000 x 32 x 256, 1875: 42 against 39; but 1200^3, 1444 tiles,
+// 8-15% faster).  Where both operands are stored along k, a load takes 16 rows of 32
+// bytes each of both, and the bounds lie lower (60000 x 32 x 256: 50 us against 39;
+// 1000 x 1000 x 2000 8% slower).
 constexpr int SPLIT = 4;
 constexpr int KSPLIT_MIN = 256;
+constexpr int KSPLIT_LONG = 512;
+bool split_k(bool along_k, size_t tiles, int K)
+{
+    if (K < KSPLIT_MIN) return false;
+    return tiles <= (along_k ? (K >= KSPLIT_LONG ? 640 : 256) : (K >= KSPLIT_LONG ? 1536 : 640));
+}
 
 template <bool TA, bool TB, bool VEC>
 __global__ __launch_bounds__(64 * SPLIT) void gemm_f64_split_kernel(GemmF64 g)
@@ -548,7 +560,7 @@ void gemm_f64(bool trans_a, bool trans_b, int M, int N, int K, double alpha, con
     if (beta != 0.0 && !Z) throw QbxError(QBX_EINVAL, "GEMM addend missing");
     GemmF64 g{A, B, Z, C, M, N, K, lda, ldb, ldz, ldc, alpha, beta};
     // 64 x 64 blocks where they give 1024 or more (four a CU), else 32 x 32 blocks,
-    // with K split over the block's waves from K = KSPLIT_MIN on
+    // with K split over the block's waves where that pays (split_k)
     const size_t big = (size_t)((N + 63) / 64) * (size_t)((M + 63) / 64);
     const int bt = big >= 1024 ? 64 : 32;
     const size_t tiles = (size_t)((N + bt - 1) / bt) * (size_t)((M + bt - 1) / bt);
@@ -571,7 +583,7 @@ void gemm_f64(bool trans_a, bool trans_b, int M, int N, int K, double alpha, con
     // 16-byte loads along k where every row of an operand with contiguous k starts on 16 bytes
     const bool vec = (trans_a || (((uintptr_t)A & 15) == 0 && (lda & 1) == 0)) &&
                      (!trans_b || (((uintptr_t)B & 15) == 0 && (ldb & 1) == 0));
-    launch(bt == 64 ? k64[op] : K >= KSPLIT_MIN ? ksplit[vec][op] : k32[op]);
+    launch(bt == 64 ? k64[op] : split_k(!trans_a && trans_b, tiles, K) ? ksplit[vec][op] : k32[op]);
     QBX_HIP(hipGetLastError());
 }
 
