@@ -261,24 +261,41 @@ __global__ __launch_bounds__(256) void mse_kernel(const float* Y, const float* T
 }
 
 // column sums of an FP32 rows x cols matrix (bias gradients): a block takes 16
-// columns, its 64 thread rows every 64th row, added in a fixed order.  One thread
-// a column took 930 us for 4096 x 256.
+// columns at a time, its 64 thread rows every 64th row, added in a fixed order.  One
+// thread a column took 930 us for 4096 x 256.  At most COLSUM_BLOCKS blocks walk the
+// columns (a grid holds below 2^32 threads, 67 million columns).
+constexpr unsigned COLSUM_BLOCKS = 1u << 16;
 __global__ __launch_bounds__(1024) void colsum_kernel(const float* X, int rows, int cols, float* out)
 {
     __shared__ float red[64][17];
     const int c = (int)threadIdx.x & 15, q = (int)threadIdx.x >> 4;
-    const int col = (int)blockIdx.x * 16 + c;
-    float s = 0.0f;
-    if (col < cols) {
+    for (int64_t c0 = (int64_t)blockIdx.x * 16; c0 < cols; c0 += (int64_t)gridDim.x * 16) {
+        const int64_t col = c0 + c;
+        float s = 0.0f;
+        if (col < cols) {
 #pragma unroll 8
-        for (int r = q; r < rows; r += 64) s += X[(size_t)r * cols + col];
+            for (int r = q; r < rows; r += 64) s += X[(size_t)r * cols + col];
+        }
+        __syncthreads();    // the last columns' sums are read
+        red[q][c] = s;
+        for (int h = 32; h > 0; h >>= 1) {
+            __syncthreads();
+            if (q < h) red[q][c] += red[q + h][c];
+        }
+        if (q == 0 && col < cols) out[col] = red[0][c];
     }
-    red[q][c] = s;
-    for (int h = 32; h > 0; h >>= 1) {
-        __syncthreads();
-        if (q < h) red[q][c] += red[q + h][c];
-    }
-    if (q == 0 && col < cols) out[col] = red[0][c];
+}
+
+// The same for few rows, one thread a column: 5 x 20000 14.7 us against 15.9, 16 x 225
+// 14.3 against 14.4, 100 x 256 21.2 against 14.5.
+constexpr int COLSUM_FEW = 16;
+__global__ __launch_bounds__(256) void colsum_few_kernel(const float* X, int rows, int cols, float* out)
+{
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (c >= cols) return;
+    float s = 0.0f;
+    for (int r = 0; r < rows; ++r) s += X[(size_t)r * cols + c];
+    out[c] = s;
 }
 
 // Adam (Kingma & Ba, 2015) on FP32 master weights; writes the BF16 copy
@@ -463,8 +480,13 @@ int qbx_mlp_colsum(int32_t rows, int32_t cols, const float* X, float* out, void*
     return qbx::guarded([&] {
         if (rows < 0 || cols < 0) throw qbx::QbxError(QBX_EINVAL, "negative size");
         if (cols == 0) return;
-        hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((cols + 15) / 16)), dim3(1024), 0, (hipStream_t)stream, X,
-                           rows, cols, out);
+        const unsigned blocks = (unsigned)(((int64_t)cols + 15) / 16);
+        if (rows <= COLSUM_FEW)
+            hipLaunchKernelGGL(colsum_few_kernel, dim3(blocks_for(cols)), dim3(256), 0, (hipStream_t)stream, X, rows,
+                               cols, out);
+        else
+            hipLaunchKernelGGL(colsum_kernel, dim3(blocks < COLSUM_BLOCKS ? blocks : COLSUM_BLOCKS), dim3(1024), 0,
+                               (hipStream_t)stream, X, rows, cols, out);
         QBX_HIP(hipGetLastError());
     });
 }
