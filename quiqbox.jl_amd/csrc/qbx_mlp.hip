@@ -324,10 +324,13 @@ struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;
 };
 
-__global__ __launch_bounds__(256) void adam_multi_kernel(AdamArgs a)
+// ONE: a single tensor, whose pointers need no search (25.6 million parameters: 132 us
+// with it, 127 without)
+template <bool ONE> __global__ __launch_bounds__(256) void adam_multi_kernel(AdamArgs a)
 {
     int t = 0;
-    while (t + 1 < a.count && blockIdx.x >= a.first[t + 1]) ++t;
+    if (!ONE)
+        while (t + 1 < a.count && blockIdx.x >= a.first[t + 1]) ++t;
     const int64_t i = (int64_t)(blockIdx.x - a.first[t]) * 256 + threadIdx.x;
     if (i < a.n[t])
         adam_one(a.w[t], a.mo[t], a.ve[t], a.gr[t], a.wb[t], i, a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
@@ -533,7 +536,7 @@ int qbx_mlp_adam_multi(int32_t count, const int64_t* n, float* const* w, float* 
         a.eps = eps;
         a.c1 = 1.0f - powf(b1, (float)step);
         a.c2 = 1.0f - powf(b2, (float)step);
-        hipLaunchKernelGGL(adam_multi_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+        hipLaunchKernelGGL(count == 1 ? adam_multi_kernel<true> : adam_multi_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
         QBX_HIP(hipGetLastError());
     });
 }
