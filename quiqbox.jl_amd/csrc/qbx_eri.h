@@ -1320,7 +1320,8 @@ void eri_staged_split_rows_kernel(EriArgs a)
     }
 }
 
-// Lanes that share a diagonal shell pair in the Schwarz kernel.
+// Lanes that share a diagonal shell pair in the Schwarz kernel, and its largest grid.
+constexpr int64_t SCHWARZ_BLOCKS = 1 << 16;
 __host__ __device__ constexpr int schwarz_lanes(int nacc) { return nacc <= 9 ? 64 : nacc <= 100 ? 16 : 1; }
 
 // Schwarz bounds: schwarz_lanes lanes per diagonal shell pair (ab|ab), each with
@@ -1339,42 +1340,46 @@ __global__ __launch_bounds__(256) void eri_schwarz_kernel(EriArgs a)
     __shared__ double2 sboys[BOYS_HEAD2 + boys_rows(LT) * QBX_BOYSL_STRIDE / 2];
     stage_boys<256, boys_rows(LT)>(sboys, a.boysl);
     __syncthreads();
-    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G;
     const int part = (int)threadIdx.x % G;
-    const bool on = t < a.total;
-    const int bi = on ? (int)t : 0;
-    R acc[Cls::NACC];
+    // SCHWARZ_BLOCKS blocks at most walk the pairs: a thread grid ends at 2^32, 67 million
+    // pairs of 64 lanes
+    for (int64_t t0 = (int64_t)blockIdx.x * (256 / G); t0 < a.total; t0 += (int64_t)gridDim.x * (256 / G)) {
+        const int64_t t = t0 + (int)threadIdx.x / G;
+        const bool on = t < a.total;
+        const int bi = on ? (int)t : 0;
+        R acc[Cls::NACC];
 #pragma unroll
-    for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
-    const PrimPair* P = a.pp + a.bra.ppo[bi];
-    const int n = on ? a.bra.ppn[bi] : 0;
-    const int per = (n + G - 1) / G, u0 = min(part * per, n);
-    prim_loop<Cls, LT, R, false, -1>(acc, P + u0, min(per, n - u0), P, n, (const double*)sboys + BOYS_HEAD);
-    if constexpr (G > 1) {
+        for (int n = 0; n < Cls::NACC; ++n) acc[n] = (R)0;
+        const PrimPair* P = a.pp + a.bra.ppo[bi];
+        const int n = on ? a.bra.ppn[bi] : 0;
+        const int per = (n + G - 1) / G, u0 = min(part * per, n);
+        prim_loop<Cls, LT, R, false, -1>(acc, P + u0, min(per, n - u0), P, n, (const double*)sboys + BOYS_HEAD);
+        if constexpr (G > 1) {
 #pragma unroll
-        for (int k = 0; k < Cls::NACC; ++k)
+            for (int k = 0; k < Cls::NACC; ++k)
 #pragma unroll
-            for (int o = G / 2; o >= 1; o >>= 1) acc[k] += __shfl_xor(acc[k], o, 64);
-    }
-    if (!on || part != 0) return;
-    const double* AB = a.bra.AB + 3 * bi;
-    R kacc[Cls::NE * NCD];
-    Cls::hrr_ket(acc, kacc, (R)AB[0], (R)AB[1], (R)AB[2]);
-    const DevShell& SA = a.sh[a.bra.shA[bi]];
-    const DevShell& SB = a.sh[a.bra.shB[bi]];
-    double mx = 0.0;
-#pragma unroll
-    for (int ia = 0; ia < NA; ++ia) {
-        R out[NB * NCD];
-        Cls::hrr_bra(ia, kacc, out, (R)AB[0], (R)AB[1], (R)AB[2]);
-#pragma unroll
-        for (int ib = 0; ib < NB; ++ib) {
-            const double w = SA.sc[ia] * SB.sc[ib];
-            const double v = fabs((double)out[ib * NCD + ia * NB + ib] * w * w);
-            mx = v > mx ? v : mx;
+                for (int o = G / 2; o >= 1; o >>= 1) acc[k] += __shfl_xor(acc[k], o, 64);
         }
+        if (!on || part != 0) continue;
+        const double* AB = a.bra.AB + 3 * bi;
+        R kacc[Cls::NE * NCD];
+        Cls::hrr_ket(acc, kacc, (R)AB[0], (R)AB[1], (R)AB[2]);
+        const DevShell& SA = a.sh[a.bra.shA[bi]];
+        const DevShell& SB = a.sh[a.bra.shB[bi]];
+        double mx = 0.0;
+#pragma unroll
+        for (int ia = 0; ia < NA; ++ia) {
+            R out[NB * NCD];
+            Cls::hrr_bra(ia, kacc, out, (R)AB[0], (R)AB[1], (R)AB[2]);
+#pragma unroll
+            for (int ib = 0; ib < NB; ++ib) {
+                const double w = SA.sc[ia] * SB.sc[ib];
+                const double v = fabs((double)out[ib * NCD + ia * NB + ib] * w * w);
+                mx = v > mx ? v : mx;
+            }
+        }
+        a.qout[bi] = sqrt(mx);
     }
-    a.qout[bi] = sqrt(mx);
 }
 
 
@@ -1385,7 +1390,8 @@ void launch_eri(const EriArgs& a, hipStream_t s)
         static_assert(LA == LC && LB == LD, "Schwarz bounds need a diagonal class");
         if (a.total <= 0) return;
         constexpr int PAIRS = 256 / schwarz_lanes(EriClass<LA, LB, LC, LD, R>::NACC);
-        const int64_t blocks = (a.total + PAIRS - 1) / PAIRS;
+        const int64_t need = (a.total + PAIRS - 1) / PAIRS;
+        const int64_t blocks = need < SCHWARZ_BLOCKS ? need : SCHWARZ_BLOCKS;
         hipLaunchKernelGGL((eri_schwarz_kernel<LA, LB, R>), dim3((unsigned)blocks), dim3(256), 0, s, a);
         QBX_HIP(hipGetLastError());
     } else if constexpr (EriClass<LA, LB, LC, LD, R>::STAGED) {
