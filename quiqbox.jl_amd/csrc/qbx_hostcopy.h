@@ -3,6 +3,8 @@
 #include "qbx_common.h"
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -19,8 +21,17 @@ namespace qbx {
 // of a fresh one.  192 MB: to the device 7.2 -> 4.8 ms, to a touched array 10.9 ->
 // 5.0 ms, to a fresh one 55.7 -> 9.0 ms (17 ms with 4 threads, 10.7 with 8; chunks
 // of 1 MB 6.2 and 6.3 ms, of 4 MB 4.3 and 4.4, at twice the pinned memory).
-// One per context, one copy at a time: kThreads * 2 chunks (48 MB) of pinned
-// memory, allocated at the first large copy and freed with the context.
+// One per context, one copy at a time: two chunks of pinned memory for each of up to
+// kThreads threads (48 MB), allocated at the first large copy and freed with the context.
+
+// Threads of a staged copy: the CPUs that the calling thread may use, up to `most`.
+inline int copy_threads(int most)
+{
+    cpu_set_t set;
+    if (sched_getaffinity(0, sizeof(set), &set) != 0) return most;   // more CPUs than the set holds
+    return std::max(1, std::min(most, CPU_COUNT(&set)));
+}
+
 class HostCopier {
 public:
     HostCopier() = default;
@@ -60,7 +71,8 @@ public:
         });
     }
 
-    // device dst = src[0, bytes) in the order of st; src may be reused on return
+    // device dst = src[0, bytes) in the order of st; a pageable src may be reused on
+    // return, pinned memory once st has come this far
     void to_device(int device, void* dst, const void* src, size_t bytes, hipStream_t st)
     {
         std::lock_guard<std::mutex> lk(mu_);
@@ -117,20 +129,23 @@ private:
     bool staged(const void* host, size_t bytes)
     {
         if (bytes < kMinBytes) return false;
+        threads_ = copy_threads(kThreads);
+        if (threads_ < 2) return false;   // one CPU: the threads would take turns
         hipPointerAttribute_t at;
         if (hipPointerGetAttributes(&at, host) == hipSuccess) {
             if (at.type != hipMemoryTypeUnregistered) return false;   // pinned or managed already
         } else {
             (void)hipGetLastError();
         }
-        if (mem_) return true;
-        if (hipHostMalloc((void**)&mem_, kChunk * 2 * kThreads, hipHostMallocDefault) != hipSuccess) {
+        if (threads_ <= (int)workers_.size()) return true;
+        release();
+        if (hipHostMalloc((void**)&mem_, kChunk * 2 * threads_, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             mem_ = nullptr;
             return false;
         }
-        workers_.assign(kThreads, Worker());
-        for (int t = 0; t < kThreads; ++t)
+        workers_.assign(threads_, Worker());
+        for (int t = 0; t < threads_; ++t)
             for (int s = 0; s < 2; ++s) {
                 workers_[t].p[s] = mem_ + kChunk * (size_t)(2 * t + s);
                 if (hipEventCreateWithFlags(&workers_[t].ev[s], hipEventDisableTiming) != hipSuccess) {
@@ -143,15 +158,15 @@ private:
         return true;
     }
 
-    // body on up to kThreads threads, which take the copy's chunks from next_
+    // body on up to threads_ threads, which take the copy's chunks from next_
     template <class Body> void run(int device, size_t bytes, Body body)
     {
         const size_t n = (bytes + kChunk - 1) / kChunk;
         next_ = 0;
         for (Worker& w : workers_) w.err = hipSuccess;
         std::vector<std::thread> pool;
-        pool.reserve(kThreads);
-        for (int t = 1; t < kThreads && (size_t)t < n; ++t) {
+        pool.reserve(threads_);
+        for (int t = 1; t < threads_ && (size_t)t < n; ++t) {
             try {
                 pool.emplace_back([&, t] {
                     if (!workers_[t].check(hipSetDevice(device))) body(workers_[t], n);
@@ -168,6 +183,7 @@ private:
     std::mutex mu_;
     char* mem_ = nullptr;
     std::vector<Worker> workers_;
+    int threads_ = 0;   // of the current copy
     std::atomic<size_t> next_{0};
 };
 
