@@ -43,7 +43,7 @@ public:
     void to_host(int device, void* dst, const void* src, size_t bytes, hipStream_t st)
     {
         std::lock_guard<std::mutex> lk(mu_);
-        if (!staged(dst, bytes)) {
+        if (!staged(dst, bytes, kMinToHost)) {
             QBX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
             QBX_HIP(hipStreamSynchronize(st));
             return;
@@ -76,7 +76,7 @@ public:
     void to_device(int device, void* dst, const void* src, size_t bytes, hipStream_t st)
     {
         std::lock_guard<std::mutex> lk(mu_);
-        if (!staged(src, bytes)) {
+        if (!staged(src, bytes, kMinToDevice)) {
             QBX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
             return;
         }
@@ -108,10 +108,12 @@ public:
 
     static constexpr size_t kChunk = 2u << 20;
     static constexpr int kThreads = 12;
-    // Smallest staged copy.  Staged against plain, to the host and to the device: 8
-    // MB 0.31 against 0.49 and 0.32 against 0.33 ms, 16 MB 0.59 against 1.05 and 0.53
-    // against 0.64; the pinned memory costs a context about 0.7 ms once.
-    static constexpr size_t kMinBytes = 16u << 20;
+    // Smallest staged copies.  Staged against plain, 18, 31, 44 and 52 MB: to the host (a
+    // touched array) 0.79 against 1.14, 1.19/2.01, 2.1/3.0 and 2.0/3.5 ms, to the device
+    // 0.72/0.60, 1.11/1.08, 2.06/2.03 and 2.00/2.37; the pinned memory costs a context
+    // about 0.7 ms once.
+    static constexpr size_t kMinToHost = 16u << 20;
+    static constexpr size_t kMinToDevice = 48u << 20;
 
 private:
     struct Worker {
@@ -126,9 +128,9 @@ private:
     };
 
     // staging pays, and its memory is there (no pinned memory left: the plain copy runs)
-    bool staged(const void* host, size_t bytes)
+    bool staged(const void* host, size_t bytes, size_t least)
     {
-        if (bytes < kMinBytes) return false;
+        if (bytes < least) return false;
         threads_ = copy_threads(kThreads);
         if (threads_ < 2) return false;   // one CPU: the threads would take turns
         hipPointerAttribute_t at;
