@@ -104,6 +104,14 @@ struct JKSink {
         pset = a.jp_set;
         npair = a.ket.n;
     }
+    // the generic kernel's: all sums straight to J and K
+    __device__ __forceinline__ JKSink(const GenArgs& a)
+        : P(nullptr), pset(0), npair(0), local(a.xcd_local != 0)
+    {
+        const size_t copy = local ? (size_t)qbx_xcc_id() : 0;
+        J = a.J + copy * a.jk_stride;
+        K = a.K + copy * a.jk_stride;
+    }
     // J_cd of component cd of ket ki: in pair order the 64 lanes' kets are
     // neighbours, so a wave's atomics go to a few cache lines; in J every lane's
     // element lies on its own line (24 H2O in cc-pVDZ: (ps|ps) 5.6 -> 4.2 ms).

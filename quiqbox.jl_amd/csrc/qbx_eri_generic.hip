@@ -354,12 +354,7 @@ __global__ __launch_bounds__(TS * W) void eri_md_kernel(GenArgs a)
     if (sC == sD) f *= 0.5;
     if (a.same && bi == ki) f *= 0.5;
     const size_t N = (size_t)a.N;
-    EriArgs ea;
-    ea.J = a.J;
-    ea.K = a.K;
-    ea.xcd_local = a.xcd_local;
-    ea.jk_stride = a.jk_stride;
-    const JKSink sink(ea);
+    const JKSink sink(a);
     double qmax = 0.0;
 
     for (int c0 = 0; c0 < z.ncd; c0 += cdc) {
