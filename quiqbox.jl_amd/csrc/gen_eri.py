@@ -526,9 +526,10 @@ def adjoint_statements(sub, tidx):
 
 def gen_adjoint(la, lb, lc, ld, groups=None):
     """EriAdj<la, lb, lc, ld> (see the module docstring) and its flop counts.
-    groups=None: vrr_adj over all targets; an integer: vrr_adj_grp<0 ..
-    groups - 1>, each over its share of the bra components e, which also adds
-    the forward values to acc."""
+    groups=None: vrr_adj over all targets (evaluated by the CPU pins only); an
+    integer, the form the kernels are built with: vrr_adj_grp<0 .. groups - 1>,
+    each over its share of the bra components e, which also adds the forward
+    values to acc."""
     es = [e for L in range(la, la + lb + 1) for e in cart(L)]
     fs = [f for L in range(lc, lc + ld + 1) for f in cart(L)]
     eidx = {e: n for n, e in enumerate(es)}

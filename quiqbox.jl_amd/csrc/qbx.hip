@@ -4,16 +4,19 @@
 // Layout in HBM (one basis):
 //   DevShell[n_shell]            centre, L, component -> basis function map
 //   PrimPair[n_primpair]         primitive-pair records of every shell pair
-//   per pair class (la >= lb):   oriented shell pairs sorted by Schwarz bound
-//                                (descending): shell ids, primitive-pair
-//                                range, Q, A-B
-//   per ERI class and precision: int64 prefix over bra pairs of the number of
-//                                surviving kets, and the first ket of each bra
-//   D (2*n_set*N^2), J, K, G (n_set*N^2) FP64 work buffers
+//   per pair class (la >= lb):   oriented shell pairs by bucket of primitive-pair
+//                                count, Schwarz bound descending within a bucket:
+//                                shell ids, primitive-pair range, Q, A-B
+//   per ERI class and precision: one allocation a basis: every bra's ket list (KetList),
+//                                the prefix sums of its 64-ket waves, the K-row tasks
+//                                (RowTask)
+//   D (2*n_set*N^2), G (n_set*N^2); J and K (n_set*N^2 each, one copy per XCD) and the
+//   ket sums of J in pair order: FP64 work buffers
 //
-// One thread evaluates one contracted shell quartet: primitive loop with the
-// generated vertical recurrence, contraction, generated horizontal recurrence,
-// then the J/K digest with per-thread pre-reduction and FP64 atomics.
+// One wave evaluates one bra with 64 of its kets, a contracted shell quartet a lane:
+// primitive loop with the generated vertical recurrence, contraction, generated
+// horizontal recurrence, then the J/K digest (qbx_eri.h); quartets with an f or g shell
+// take a block each (qbx_eri_generic.hip).
 #include "qbx.h"
 #include "qbx_device.h"
 

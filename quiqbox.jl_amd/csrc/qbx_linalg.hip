@@ -1,5 +1,5 @@
-// FP64 GEMM on the CDNA4 matrix cores (v_mfma_f64_16x16x4f64) and the
-// small kernels of trace-correcting purification.
+// FP64 GEMM on the CDNA4 matrix cores (v_mfma_f64_16x16x4f64), trace-correcting
+// purification on the device, and the Householder tridiagonalization of the Fock solve.
 //
 // MFMA f64 16x16x4 operand layout (one wave): lane l holds A[l % 16][l / 16]
 // and B[l / 16][l % 16]; the four result registers r hold

@@ -293,16 +293,18 @@ class PurifiedDensity:
 
 
 # Basis size from which the default SCF step runs on the GPU.  One step
-# (X' F X, eigen, C = X C', D) measured on the box, device against numpy on
-# the host: n = 128 2.44 / 1.18 ms, 256 6.18 / 4.38 ms, 384 8.86 / 8.79 ms,
-# 512 12.0 / 23.0 ms, 600 13.6 / 18.0 ms (rocSOLVER's fixed costs dominate
-# small problems).
+# (X' F X, eigen, C = X C', D), device against numpy on the host: n = 128 1.95 /
+# 0.96 ms, 200 2.75 / 2.16 ms, 256 3.33 / 4.19 ms, 320 4.00 / 5.97 ms, 384 4.64 /
+# 8.73 ms, 512 6.0 / 22.4 ms, 600 7.3 / 17.6 ms.  The two meet between 200 and 256;
+# the bound is that of the library's tridiagonalization (8.86 / 8.79 ms at 384) and
+# has not been moved.
 DEVICE_EIGEN_MIN_N = 384
 
 
 class DeviceEigen:
     """getC + getD of the SCF steps on the GPU (Context.fock_solve): X' F X
-    and X C' on the FP64 matrix cores, the symmetric eigenproblem by rocSOLVER;
+    and X C' on the FP64 matrix cores, the symmetric eigenproblem by an own
+    tridiagonalization (from order 96 on) and rocSOLVER's divide and conquer;
     the same matrices as solveFockMatrix/getD up to rounding."""
 
     def __init__(self, ctx):
@@ -1054,7 +1056,7 @@ def runHartreeFock(nucInfo, basis, config=None, *, printInfo=True, infoLevel=def
     Fock-build mode; `densitySolver` selects each step's orbitals and density:
     "eigen" (default) diagonalizes X' F X as the reference does, on the GPU
     when the Fock build is and the basis has at least DEVICE_EIGEN_MIN_N
-    functions (matrix-core GEMMs, rocSOLVER eigensolver), on the host (numpy)
+    functions (matrix-core GEMMs, Context.fock_solve), on the host (numpy)
     below that; "eigen-device" and "eigen-host" force either; "purify" forms
     the density by purification on the GPU instead (the same matrix; the
     coefficients of the result still come from one diagonalization).  The
