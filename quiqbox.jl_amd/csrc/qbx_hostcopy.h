@@ -108,12 +108,12 @@ public:
 
     static constexpr size_t kChunk = 2u << 20;
     static constexpr int kThreads = 12;
-    // Smallest staged copies.  Staged against plain, 18, 31, 44 and 52 MB: to the host (a
-    // touched array) 0.79 against 1.14, 1.19/2.01, 2.1/3.0 and 2.0/3.5 ms, to the device
-    // 0.72/0.60, 1.11/1.08, 2.06/2.03 and 2.00/2.37; the pinned memory costs a context
-    // about 0.7 ms once.
-    static constexpr size_t kMinToHost = 16u << 20;
-    static constexpr size_t kMinToDevice = 48u << 20;
+    // Smallest staged copies.  Staged against plain, to the host: 17 MiB 1.3 against 1.05
+    // ms (with few chunks most calls wait for a thread to wake), 18.1 MiB 0.82/1.10, 24
+    // 0.95/1.43, 37 2.0/4.0, 49 2.0/3.5; to the device: 17 MiB 0.72/0.60, 30 1.11/1.08, 42
+    // 2.06/2.03, 48 1.85/2.10.  The pinned memory costs a context about 0.7 ms once.
+    static constexpr size_t kMinToHost = 19u << 20;
+    static constexpr size_t kMinToDevice = 46u << 20;
 
 private:
     struct Worker {
