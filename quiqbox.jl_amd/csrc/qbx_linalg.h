@@ -80,8 +80,9 @@ bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double*
 
 // The tridiagonal matrix times a power of two, its largest entry in [1, 2) (the
 // divide and conquer solver drops what is small in absolute terms), and the
-// eigenvalues d brought back; back: one double of device memory.
-void tridiag_scale(int n, double* d, double* e, double* back, hipStream_t s);
+// eigenvalues d brought back; back: one double of device memory.  Where *status is not 0
+// the matrix and the factors tau become zero.
+void tridiag_scale(int n, double* d, double* e, double* tau, const int* status, double* back, hipStream_t s);
 void tridiag_unscale(int n, double* d, const double* back, hipStream_t s);
 
 }  // namespace qbx

@@ -938,10 +938,20 @@ bool tridiagonalize(const TridiagPlan& plan, const double* A, double* V, double*
 }
 
 // One block: d (n) and e (n - 1) times the power of two that brings their largest
-// entry into [1, 2); *back undoes it.
-__global__ void tri_scale_kernel(int n, double* d, double* e, double* back)
+// entry into [1, 2); *back undoes it.  Where the tridiagonalization gave up, its outputs
+// are partly unwritten: the zero matrix and no reflectors instead, so that the solver
+// queued behind never sees them.
+__global__ void tri_scale_kernel(int n, double* d, double* e, double* tau, const int* status, double* back)
 {
     __shared__ double red[16];
+    if (*status != 0) {
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            d[i] = 0.0;
+            if (i < n - 1) e[i] = tau[i] = 0.0;
+        }
+        if (threadIdx.x == 0) *back = 0.0;
+        return;
+    }
     double big = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) big = fmax(big, fmax(fabs(d[i]), i < n - 1 ? fabs(e[i]) : 0.0));
     for (int o = 32; o >= 1; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
@@ -960,9 +970,9 @@ __global__ void tri_unscale_kernel(int n, double* d, const double* back)
     for (int i = threadIdx.x; i < n; i += blockDim.x) d[i] = ldexp(d[i], (int)*back);
 }
 
-void tridiag_scale(int n, double* d, double* e, double* back, hipStream_t s)
+void tridiag_scale(int n, double* d, double* e, double* tau, const int* status, double* back, hipStream_t s)
 {
-    hipLaunchKernelGGL(tri_scale_kernel, dim3(1), dim3(1024), 0, s, n, d, e, back);
+    hipLaunchKernelGGL(tri_scale_kernel, dim3(1), dim3(1024), 0, s, n, d, e, tau, status, back);
     QBX_HIP(hipGetLastError());
 }
 void tridiag_unscale(int n, double* d, const double* back, hipStream_t s)
